@@ -298,7 +298,7 @@ static_assert(kCbCount <= kCtxBuffers, "context buffers");
 struct Batch {
   tcx_ctx* ctx = nullptr;
   hipStream_t st = nullptr;
-  // second stream: the block-form Gram Lanczos runs beside the one-wave
+  // second stream: the block-form Gram Lanczos runs beside the resident
   // form (default priority; joined back into st by an event)
   hipStream_t st2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -634,7 +634,7 @@ int refine_power(Batch& b, const std::vector<GJob*>& act, double* ms_power) {
   std::vector<GramItem> gitems;
   std::vector<GramVecJob> gmap;
   std::vector<GramLzJob> glz;
-  std::vector<LzWaveJob> wlz;
+  std::vector<LzResJob> wlz;
   size_t lds_map = 0, lds_lz = 0;
   Launch<FillSeg> fills;
   for (size_t q = 0; q < act.size(); ++q) {
@@ -655,12 +655,12 @@ int refine_power(Batch& b, const std::vector<GJob*>& act, double* ms_power) {
       const long nd = off[c + 1] - off[c];
       j->thin[c] = gram_form(j->m, nd, cnt[c]);
       j->fat[c] = cnt[c] > 0 && !j->thin[c];
-      // fat clusters of short series: one wave each; the others by block
-      const bool fat_wave = j->fat[c] && j->m <= kLzWaveMaxD;
+      // fat clusters of short series: one block each, the others all together
+      const bool fat_wave = j->fat[c] && j->m <= kLzResMaxD;
       j->nfat += j->fat[c] && !fat_wave;
       fills.add(FillSeg{j->scount + c, 1, j->fat[c] && !fat_wave ? cnt[c] : 0}, 1);
       if (fat_wave)
-        wlz.push_back(LzWaveJob{j->S + c * mm, j->m, 0, steps, j->o.seed, j->it, c, nullptr,
+        wlz.push_back(LzResJob{j->S + c * mm, j->m, 0, steps, j->o.seed, j->it, c, nullptr,
                                 j->Q + (long)c * (kLanczosMax + 1) * j->m, j->v + (long)c * j->m,
                                 j->r + (long)c * j->m, j->sv + (long)c * j->m, j->steps + c,
                                 j->conv + c});
@@ -677,8 +677,8 @@ int refine_power(Batch& b, const std::vector<GJob*>& act, double* ms_power) {
                                     tj, ti == tj ? rc : nullptr, j->o.seed, j->it, c});
       double* svc = j->sv + (long)c * j->m;
       double* Qc = j->Q + (long)c * (kLanczosMax + 1) * j->m;
-      if (gn <= kLzWaveMaxD) {
-        wlz.push_back(LzWaveJob{j->S + c * mm, gn, 1, steps - 1, 0, 0, 0, rc, Qc, wc, nullptr,
+      if (gn <= kLzResMaxD) {
+        wlz.push_back(LzResJob{j->S + c * mm, gn, 1, steps - 1, 0, 0, 0, rc, Qc, wc, nullptr,
                                 svc, j->steps + c, j->conv + c});
       } else {
         glz.push_back(GramLzJob{j->S + c * mm, gn, steps - 1, rc, Qc, wc, svc, j->steps + c,
@@ -698,7 +698,7 @@ int refine_power(Batch& b, const std::vector<GJob*>& act, double* ms_power) {
   std::vector<GJob*> split_set;
   for (GJob* j : act) {
     const int steps = j->m > 1000 ? 1000 : j->m;
-    // fat clusters of m > kLzWaveMaxD take the two-launch form: each Lanczos
+    // fat clusters of m > kLzResMaxD take the two-launch form: each Lanczos
     // step of all of them is one grid-wide matvec and one step kernel,
     // instead of one latency-bound block per cluster
     if (j->nfat > 0) split_set.push_back(j);
@@ -726,10 +726,7 @@ int refine_power(Batch& b, const std::vector<GJob*>& act, double* ms_power) {
   // so those start in the first wave of blocks (each cluster's result is
   // independent of its position)
   std::stable_sort(wlz.begin(), wlz.end(),
-                   [](const LzWaveJob& a, const LzWaveJob& c) { return a.d > c.d; });
-  // orders above kLzWaveSplitD (at the front) take four waves per cluster
-  size_t nw4 = 0;
-  while (nw4 < wlz.size() && wlz[nw4].d > kLzWaveSplitD) ++nw4;
+                   [](const LzResJob& a, const LzResJob& c) { return a.d > c.d; });
   std::stable_sort(glz.begin(), glz.end(),
                    [](const GramLzJob& a, const GramLzJob& c) { return a.nd > c.nd; });
   b.up.reset();
@@ -744,9 +741,14 @@ int refine_power(Batch& b, const std::vector<GJob*>& act, double* ms_power) {
                                (int)glz.size(), lds_lz, kLzPowerTol, b.st2));
     GX_HIP(hipEventRecord(b.ev_join, b.st2));
   }
-  const LzWaveJob* dwl = reinterpret_cast<const LzWaveJob*>(b.up.dev(wl_off));
-  GX_HIP(launch_lanczos_wave(dwl, (int)nw4, 4, kLzPowerTol, b.st));
-  GX_HIP(launch_lanczos_wave(dwl + nw4, (int)(wlz.size() - nw4), 1, kLzPowerTol, b.st));
+  const LzResJob* dwl = reinterpret_cast<const LzResJob*>(b.up.dev(wl_off));
+  for (size_t i = 0; i < wlz.size();) {  // one launch per register split
+    const int form = lz_res_form(wlz[i].d);
+    size_t e = i;
+    while (e < wlz.size() && lz_res_form(wlz[e].d) == form) ++e;
+    GX_HIP(launch_lz_res_group(dwl + i, (int)(e - i), form, kLzPowerTol, b.st));
+    i = e;
+  }
   if (!glz.empty()) GX_HIP(hipStreamWaitEvent(b.st, b.ev_join, 0));
   GX_HIP(launch_gram_map(reinterpret_cast<const GramVecJob*>(b.up.dev(gm_off)), (int)gmap.size(),
                          lds_map, b.st));

@@ -3186,346 +3186,542 @@ __global__ __launch_bounds__(256) void k_gram_map(const GramVecJob* __restrict__
 }
 
 
-// ------------------------------------------- one wave per small cluster
-// The Lanczos evaluation of power_lanczos_cluster for dimension d <=
-// kLzWaveMaxD by one wave, with no block barriers: vectors are held in
-// registers (element e = lane + 64 u), the matvec reads column c of the
-// symmetric matrix as one coalesced row segment with x[c] broadcast from
-// the wave's LDS, sums are DPP wave sums, and T^I e1 is the one-wave recurrence
-// (tridiag_power_wave).  Four clusters per block of 256 threads.  Same
-// steps and acceptance rule as the block form (which takes the recurrence
-// by binary powering for short T: the two agree to rounding).
-constexpr int kLzWaveU = kLzWaveMaxD / 64;
-constexpr int kLzWaveLds = 3 * (kLzMax + 1) + 2 * kLzMax + kLzWaveMaxD;  // alpha, beta, cf, y, yp, x
+// ------------------------------------------- resident Lanczos, order <= 256
+// The Lanczos evaluation of power_lanczos_cluster for order d <= 64 U by one
+// block of NW waves that reads the matrix once and keeps it in registers:
+// wave p holds the columns [p CS, (p+1) CS), lane l of it the rows l + 64 u
+// (T = double while they fit, else FP32 widened as they are used), so a
+// matvec is U CS multiply-adds per lane with x[c] broadcast from LDS and one
+// exchange of the NW partial products.  Every wave then holds the whole
+// vector and computes all sums alike; the dots with the basis (rows in LDS,
+// the rows past QL in the cluster's Q buffer) are split by rows over the
+// waves, the projection by elements: four barriers per step.  T^I e1 up to
+// length kLzResSq is squared on the FP64 matrix cores (tridiag_power_mfma).
+// A step is bound by the latency of its exchanges and of its FP64 sums (at
+// order 256 also by the 128 widenings and multiply-adds per lane), not by
+// the matrix.  Measured, k = 4, m = 128, n = 512: 175 us per refinement when
+// the block read S from L2 every step behind a dozen barriers, 62 us now; a
+// launch of 16 steps takes 39 us at order 64, 50 us at 128, 76 us at 256.
+// In a batch of 64 uneven jobs the clusters of order <= 256 took 1.9 ms per
+// iteration with a wave (order <= 128) or four waves reading the matrix from
+// L2, 0.3 ms now.
+constexpr int kLzResSq = 32;
+constexpr int kLzResSqLd = kLzResSq + 1;
+constexpr int kLzResSqDoubles = 2 * kLzResSq * kLzResSqLd + 2 * kLzResSq;
 
-// y = S x for symmetric S (FP32, d x d) through the wave's LDS slot xb (d
-// doubles); entries e >= d of y come back zero.  Loads past the last row
-// are clamped to it.
-// kW > 1: the kW waves of the block share one cluster, wave `part` takes
-// the columns [part * d/kW, (part+1) * d/kW) and the partial products are
-// summed through `red` (kW x kLzWaveMaxD doubles) in wave order, so every
-// wave ends with the same y.
-template <int kW>
-__device__ __forceinline__ void wave_sym_matvec(const float* __restrict__ S, int d, int U,
-                                                const double (&x)[kLzWaveU],
-                                                double (&y)[kLzWaveU], double* xb, int part,
-                                                double* red) {
-  constexpr int kCols = 8;  // columns whose loads are in flight together
-  const int lane = threadIdx.x & 63;
-  int ec[kLzWaveU];
-#pragma unroll
-  for (int u = 0; u < kLzWaveU; ++u) {
-    y[u] = 0.0;
-    const int e = lane + 64 * u;
-    ec[u] = e < d ? e : d - 1;
-    if (e < d) xb[e] = x[u];
+// Per lane without bit O: a plus the partner's a (lane ^ O); with it: b plus
+// the partner's b (v_permlane16_swap / v_permlane32_swap of the halves).
+template <int O>
+__device__ __forceinline__ double swap_sum_f64(double a, double b) {
+  static_assert(O == 16 || O == 32, "row or half swap");
+  const uint32_t al = (uint32_t)__double2loint(a), ah = (uint32_t)__double2hiint(a);
+  const uint32_t bl = (uint32_t)__double2loint(b), bh = (uint32_t)__double2hiint(b);
+  if constexpr (O == 16) {
+    const auto l = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+    return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+  } else {
+    const auto l = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
+    return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
   }
-  wave_lds_sync();
-  const int share = (d + kW - 1) / kW;
-  const int cb = kW > 1 ? part * share : 0, ce = kW > 1 ? (cb + share < d ? cb + share : d) : d;
-  for (int c0 = cb; c0 < ce; c0 += kCols) {
-    float sv[kCols][kLzWaveU];
+}
+
+// Wave sums of four values at once: every lane of row q (16 lanes) gets the
+// sum of t_q.  Seven additions deep, a quarter of four wave_sum_f64.
+__device__ __forceinline__ double wave_sum4_f64(double t0, double t1, double t2, double t3) {
+  double v = swap_sum_f64<16>(swap_sum_f64<32>(t0, t2), swap_sum_f64<32>(t1, t3));
+  v += dpp_f64<0xB1>(v);   // lane ^ 1
+  v += dpp_f64<0x4E>(v);   // lane ^ 2
+  v += dpp_f64<0x124>(v);  // row_ror:4
+  v += dpp_f64<0x128>(v);  // row_ror:8
+  return v;
+}
+
+// B = (A / tr A)^2 (first: A^2) for symmetric A of order n (np = 16 TT, zero
+// past n, LDS row stride kLzResSqLd) in 16 x 16 tiles over the waves, FP64
+// MFMA: operand lane l holds element (l % 16, k = l / 16), result register r
+// of lane l element (4 r + l / 16, l % 16).
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+template <int NW, int TT>
+__device__ __forceinline__ void sym_square_mfma(const double* A, double* B, int n, bool first) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int i = lane & 15, kq = lane >> 4;
+  for (int tile = wv; tile < TT * TT; tile += NW) {
+    const int ti = tile / TT, tj = tile % TT;
+    const double* pa = A + (ti * 16 + i) * kLzResSqLd + kq;
+    const double* pb = A + (tj * 16 + i) * kLzResSqLd + kq;
+    double a[4 * TT], b[4 * TT];
 #pragma unroll
-    for (int t = 0; t < kCols; ++t) {
-      const int c = c0 + t < ce ? c0 + t : ce - 1;
-      const float* col = S + (long)c * d;
-#pragma unroll
-      for (int u = 0; u < kLzWaveU; ++u) sv[t][u] = u < U ? col[ec[u]] : 0.f;
+    for (int s = 0; s < 4 * TT; ++s) {
+      a[s] = pa[4 * s];
+      b[s] = pb[4 * s];
     }
+    const double dg = lane < n ? A[lane * kLzResSqLd + lane] : 0.0;
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int t = 0; t < kCols; ++t) {
-      const double xc = c0 + t < ce ? xb[c0 + t] : 0.0;
+    for (int s = 0; s < 4 * TT; ++s)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], acc, 0, 0, 0);
+    const double tr = wave_sum_f64(dg);
+    const double f = first ? 1.0 : (tr > 0.0 ? 1.0 / tr : 0.0);
 #pragma unroll
-      for (int u = 0; u < kLzWaveU; ++u) y[u] += (double)sv[t][u] * xc;
-    }
+    for (int r = 0; r < 4; ++r)
+      B[(ti * 16 + 4 * r + kq) * kLzResSqLd + tj * 16 + i] = acc[r] * (f * f);
   }
-  if constexpr (kW > 1) {
+}
+
+// tridiag_power_block for len <= kLzResSq by NW waves: the same scaling and
+// the same powers, the squarings by sym_square_mfma (wk: kLzResSqDoubles of
+// LDS).  Ends with a barrier.
+template <int NW>
+__device__ void tridiag_power_mfma(const double* alpha, const double* beta, int len, int I,
+                                   double* wk, double* y) {
+  constexpr int NT = 64 * NW;
+  const int tid = threadIdx.x, lane = tid & 63, n = len;
+  const int np = n <= 16 ? 16 : 32;
+  double* A = wk;
+  double* B = wk + kLzResSq * kLzResSqLd;
+  double* yv = wk + 2 * kLzResSq * kLzResSqLd;
+  double* yt = yv + kLzResSq;
+  double g = 0.0;
+  if (lane < n)
+    g = fabs(alpha[lane]) + (lane > 0 ? fabs(beta[lane]) : 0.0) +
+        (lane + 1 < n ? fabs(beta[lane + 1]) : 0.0);
+  g = wave_max_f64(g);
+  const double sc = g > 0.0 ? 1.0 / g : 0.0;
+  const int sh = n <= 16 ? 4 : 5;
+  for (int idx = tid; idx < np * np; idx += NT) {
+    const int i = idx >> sh, jj = idx & (np - 1);
+    double v = 0.0;
+    if (i < n && jj < n)
+      v = i == jj ? alpha[i] : (jj == i + 1 ? beta[jj] : (i == jj + 1 ? beta[i] : 0.0));
+    A[i * kLzResSqLd + jj] = v * sc;
+  }
+  if (tid < kLzResSq) {
+    yv[tid] = tid == 0 ? 1.0 : 0.0;
+    yt[tid] = 0.0;
+  }
+  __syncthreads();
+  bool first = true;  // the current power is A, after the first squaring A / tr A
+  for (int e = I;;) {
+    if (e & 1) {  // yt = A yv / tr A, four lanes per row, then swap
+      const double dg = lane < n ? A[lane * kLzResSqLd + lane] : 0.0;
+      const double tr = wave_sum_f64(dg);
+      const double f = first ? 1.0 : (tr > 0.0 ? 1.0 / tr : 0.0);
+      if (tid < 4 * np) {
+        const int i = tid >> 2;
+        const double* ai = A + i * kLzResSqLd;
+        double s0 = 0.0;
+#pragma unroll 4
+        for (int c = tid & 3; c < np; c += 4) s0 += ai[c] * yv[c];
+        s0 += dpp_f64<0xB1>(s0);
+        s0 += dpp_f64<0x4E>(s0);
+        if ((tid & 3) == 0) yt[i] = s0 * f;
+      }
+      __syncthreads();
+      double* t = yv;
+      yv = yt;
+      yt = t;
+    }
+    e >>= 1;
+    if (e == 0) break;
+    if (np == 16)
+      sym_square_mfma<NW, 1>(A, B, n, first);
+    else
+      sym_square_mfma<NW, 2>(A, B, n, first);
+    first = false;
+    __syncthreads();
+    double* t = A;
+    A = B;
+    B = t;
+  }
+  const double yl = lane < n ? yv[lane] : 0.0;
+  const double nn = wave_sum_f64(yl * yl);
+  const double inv = nn > 0.0 ? 1.0 / sqrt(nn) : 0.0;
+  if (tid < n) y[tid] = yl * inv;
+  __syncthreads();
+}
+
+// Basis rows kept in LDS: what leaves two blocks per CU (order <= 128), one
+// block above.
+template <int U>
+constexpr int lz_res_rows() { return U == 1 ? 48 : 40; }
+template <int NW, int U>
+constexpr size_t lz_res_lds() {
+  return sizeof(double) * (64 * U * (size_t)(2 + NW + lz_res_rows<U>()) + 3 * (kLzMax + 1) + 1 +
+                           kLzMax + kLzResSqDoubles);
+}
+
+template <int NW, int U, typename T>
+__device__ __forceinline__ void lz_res_body(const LzResJob& a, double lz_tol) {
+  constexpr int D = 64 * U, CS = D / NW, QL = lz_res_rows<U>();
+  constexpr int EPW = D / NW, NG = 64 / EPW;  // projection: elements per wave, row groups
+  static_assert(CS % 2 == 0 && EPW <= 64 && 64 % EPW == 0, "split of the vector over the waves");
+  extern __shared__ __align__(16) double rsh[];
+  double* xb = rsh;                     // D: the matvec's x
+  double* wb = xb + D;                  // D: the projected w
+  double* part = wb + D;                // NW x D partial products
+  double* Qs = part + NW * D;           // QL x D basis rows
+  double* alpha = Qs + QL * D;          // kLzMax + 1
+  double* beta = alpha + kLzMax + 1;    // kLzMax + 1
+  double* cf = beta + kLzMax + 1;       // kLzMax + 1 (+ 1 to keep pairs aligned)
+  double* y = cf + kLzMax + 2;          // kLzMax
+  double* wk = y + kLzMax;              // kLzResSqDoubles
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int d = a.d, c0 = wv * CS;
+  // the wave's columns of the symmetric matrix, zero outside d x d
+  T av[U][CS];
 #pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) {
+  for (int c = 0; c < CS; ++c)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
       const int e = lane + 64 * u;
-      if (e < d) red[part * kLzWaveMaxD + e] = y[u];
+      av[u][c] = c0 + c < d && e < d ? (T)a.S[(long)(c0 + c) * d + e] : (T)0;
+    }
+  const int own_e = wv * EPW + (lane & (EPW - 1)), gr = lane / EPW;  // project: element, rows
+  // w = S x for x in xb (visible to the block); every wave gets all of w,
+  // and own the element its lane projects.  The empty asm keeps the FP32
+  // columns from being widened once for all steps, into twice the registers.
+  auto matvec = [&](double (&w)[U], double& own) {
+    double acc[U];
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int c = 0; c < CS; ++c)
+#pragma unroll
+        for (int u = 0; u < U; ++u) asm volatile("" : "+v"(av[u][c]));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc[u] = 0.0;
+#pragma unroll
+    for (int c = 0; c < CS; c += 2) {
+      const double2 x2 = *reinterpret_cast<const double2*>(xb + c0 + c);
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc[u] += (double)av[u][c] * x2.x;
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc[u] += (double)av[u][c + 1] * x2.y;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) part[wv * D + lane + 64 * u] = acc[u];
+    __syncthreads();
+    double t = 0.0;
+#pragma unroll
+    for (int p = 0; p < NW; ++p) t += part[p * D + own_e];
+    own = t;
+    if constexpr (U <= 2) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        t = 0.0;
+#pragma unroll
+        for (int p = 0; p < NW; ++p) t += part[p * D + lane + 64 * u];
+        w[u] = t;
+      }
+    } else {  // one more exchange reads less LDS than all partials in every wave
+      wb[own_e] = own;
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = wb[lane + 64 * u];
+    }
+  };
+  auto dot = [&](const double (&p)[U], const double (&q)[U]) {
+    double t = 0.0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) t += p[u] * q[u];
+    return wave_sum_f64(t);
+  };
+  auto dot2 = [&](const double (&p)[U], const double (&q)[U], const double (&p2)[U],
+                  const double (&q2)[U], double& d1, double& d2) {
+    double t1 = 0.0, t2 = 0.0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      t1 += p[u] * q[u];
+      t2 += p2[u] * q2[u];
+    }
+    const double v = wave_sum4_f64(t1, t2, 0.0, 0.0);
+    d1 = readlane_f64(v, 0);
+    d2 = readlane_f64(v, 16);
+  };
+  // the waves share the writes of a vector every wave holds
+  auto put = [&](double* dst, const double (&v)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (u % NW == wv) dst[lane + 64 * u] = v[u];
+  };
+  auto put_row = [&](int l, const double (&v)[U]) {
+    if (l < QL) {
+      put(Qs + l * D, v);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (u % NW == wv && lane + 64 * u < d) a.Q[(long)l * d + lane + 64 * u] = v[u];
+    }
+  };
+  // basis rows past QL come from the cluster's Q buffer (rare: QL is past
+  // the usual acceptance lengths)
+  auto far_row = [&](int l, int e) { return e < d ? a.Q[(long)l * d + e] : 0.0; };
+  // cf[l] = q_l . w for l <= it, rows split over the waves; ends with a barrier
+  auto dots = [&](const double (&w)[U], int it) {
+    constexpr int kB = 4;  // rows whose loads and sums are in flight together
+    const int near = it < QL ? it : QL - 1;
+    for (int l0 = wv; l0 <= near; l0 += kB * NW) {
+      double t[kB];
+#pragma unroll
+      for (int q = 0; q < kB; ++q) {
+        const double* row = Qs + (l0 + q * NW <= near ? l0 + q * NW : l0) * D + lane;
+        t[q] = 0.0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) t[q] += row[64 * u] * w[u];
+      }
+      const double v = wave_sum4_f64(t[0], t[1], t[2], t[3]);
+      const int l = l0 + (lane >> 4) * NW;
+      if ((lane & 15) == 0 && l <= near) cf[l] = v;
+    }
+    for (int l = QL + wv; l <= it; l += NW) {
+      double t = 0.0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) t += far_row(l, lane + 64 * u) * w[u];
+      t = wave_sum_f64(t);
+      if (lane == 0) cf[l] = t;
     }
     __syncthreads();
-#pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) {
-      const int e = lane + 64 * u;
-      double t = 0.0;
-      if (e < d)
-#pragma unroll
-        for (int p = 0; p < kW; ++p) t += red[p * kLzWaveMaxD + e];
-      y[u] = t;
+  };
+  // w -= sum_{l <= it} cf[l] q_l: each lane forms its own element over its
+  // group's rows; every wave reads the whole result back
+  auto project = [&](double (&w)[U], double& own, int it) {
+    const int near = it < QL ? it : QL - 1;
+    const double* row = Qs + gr * D + own_e;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    int l = gr;
+    for (; l + 3 * NG <= near; l += 4 * NG, row += 4 * NG * D) {
+      s0 += cf[l] * row[0];
+      s1 += cf[l + NG] * row[NG * D];
+      s2 += cf[l + 2 * NG] * row[2 * NG * D];
+      s3 += cf[l + 3 * NG] * row[3 * NG * D];
     }
-    __syncthreads();  // red is rewritten by the next product
-  }
+    if (l <= near) s0 += cf[l] * row[0];
+    if (l + NG <= near) s1 += cf[l + NG] * row[NG * D];
+    if (l + 2 * NG <= near) s2 += cf[l + 2 * NG] * row[2 * NG * D];
+    for (l = QL + gr; l <= it; l += NG) s0 += cf[l] * far_row(l, own_e);
+    double t = (s0 + s1) + (s2 + s3);
+    if constexpr (EPW <= 16) t = swap_sum_f64<16>(t, t);
+    if constexpr (EPW <= 32) t = swap_sum_f64<32>(t, t);
+    own -= t;
+    wb[own_e] = own;  // the groups of a wave write the same value
+    __syncthreads();
 #pragma unroll
-  for (int u = 0; u < kLzWaveU; ++u)
-    if (lane + 64 * u >= d) y[u] = 0.0;
-  wave_lds_sync();  // xb is rewritten by the next product
-}
-
-// Rows l0 .. l0 + kLzWaveRows - 1 of the basis (rows past `last`, and
-// entries e >= d, read as zero), loaded together.
-constexpr int kLzWaveRows = 8;
-__device__ __forceinline__ void wave_basis_rows(const double* __restrict__ Q, int d, int U, int l0,
-                                                int last,
-                                                double (&qv)[kLzWaveRows][kLzWaveU]) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int t = 0; t < kLzWaveRows; ++t) {
-    const double* ql = Q + (long)(l0 + t) * d;
-#pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) {
-      const int e = lane + 64 * u;
-      qv[t][u] = (u < U && l0 + t <= last && e < d) ? ql[e] : 0.0;
-    }
-  }
-}
-
-// kW = 1: four clusters per block, one wave each.  kW = 4: one cluster per
-// block, the four waves sharing each matvec by columns (the product's
-// latency chain is a quarter as long) and computing everything else alike;
-// wave 0 writes the results, every wave the (identical) basis rows it reads
-// back itself.
-template <int kW>
-__global__ __launch_bounds__(256, 3) void k_lanczos_wave(const LzWaveJob* __restrict__ jobs,
-                                                      int njobs, double lz_tol) {
-  __shared__ double lds[4][kLzWaveLds];
-  __shared__ double red[kW > 1 ? kW * kLzWaveMaxD : 1];
-  // the wave index is uniform in the wave: readfirstlane lets the job's
-  // fields live in scalar registers
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int jid = kW > 1 ? (int)blockIdx.x : (int)blockIdx.x * 4 + wv;
-  if (jid >= njobs) return;  // whole wave (kW = 1) or whole block
-  const int part = kW > 1 ? wv : 0;
-  const bool writer = part == 0;
-  const LzWaveJob a = jobs[jid];
-  double* alpha = lds[wv];
-  double* beta = alpha + kLzMax + 1;
-  double* cf = beta + kLzMax + 1;
-  double* y = cf + kLzMax + 1;
-  double* yp = y + kLzMax;
-  double* xb = yp + kLzMax;
-  const int d = a.d, U = (d + 63) / 64;
-  const float* S = a.S;
-  double q[kLzWaveU], w[kLzWaveU], qp[kLzWaveU], r[kLzWaveU];
+    for (int u = 0; u < U; ++u) w[u] = wb[lane + 64 * u];
+  };
+  double q[U], w[U], r[U];
+  double own, own_r = 0.0;
   double sigma = 0.0, n0 = 0.0;
   const double inv_d = 1.0 / (double)d;
   if (a.gram) {
 #pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int e = lane + 64 * u;
       q[u] = e < d ? a.vstart[e] : 0.0;
-      r[u] = qp[u] = 0.0;
-      n0 += q[u] * q[u];
+      r[u] = 0.0;
     }
-    n0 = sqrt(wave_sum_f64(n0));
-    if (!(n0 > 0.0)) {  // wave-uniform
-#pragma unroll
-      for (int u = 0; u < kLzWaveU; ++u) {
-        const int e = lane + 64 * u;
-        if (e < d && writer) {
-          a.v[e] = 0.0;
-          a.h[e] = 0.0;
-        }
+    n0 = sqrt(dot(q, q));
+    if (!(n0 > 0.0)) {  // the same in every wave
+      for (int e = threadIdx.x; e < d; e += 64 * NW) {
+        a.v[e] = 0.0;
+        a.h[e] = 0.0;
       }
-      if (lane == 0 && writer) {
+      if (threadIdx.x == 0) {
         *a.steps = 0;
         *a.conv = 1;
       }
       return;
     }
   } else {
-    double one[kLzWaveU];
+    double one[U];
 #pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) one[u] = lane + 64 * u < d ? 1.0 : 0.0;
-    wave_sym_matvec<kW>(S, d, U, one, r, xb, part, red);  // r = S 1
+    for (int u = 0; u < U; ++u) one[u] = lane + 64 * u < d ? 1.0 : 0.0;
+    put(xb, one);
+    __syncthreads();
+    matvec(r, own_r);  // r = S 1
+    sigma = dot(r, one);
 #pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int e = lane + 64 * u;
-      sigma += r[u];
       q[u] = e < d ? power_v0(a.seed, a.iter, a.cluster, e) : 0.0;
-      qp[u] = 0.0;
-      n0 += q[u] * q[u];
-      if (e < d && writer) a.r[e] = r[u];
+      if (u % NW == wv && e < d) a.r[e] = r[u];
     }
-    sigma = wave_sum_f64(sigma);
-    n0 = sqrt(wave_sum_f64(n0));
+    n0 = sqrt(dot(q, q));
+    __syncthreads();  // xb and part are rewritten below
   }
 #pragma unroll
-  for (int u = 0; u < kLzWaveU; ++u) {
-    const int e = lane + 64 * u;
-    q[u] /= n0;
-    if (e < d) a.Q[e] = q[u];
-  }
+  for (int u = 0; u < U; ++u) q[u] /= n0;
+  put(xb, q);
+  put_row(0, q);
+  __syncthreads();
   const int jmax = d < kLzMax ? d : kLzMax;
   int len = 0, conv = 0, prev_len = 0;
-  double bprev = 0.0;
+  double yp0 = 0.0, yp1 = 0.0;  // the last check's y, entries lane and lane + 64
+  // sums of a vector every wave holds: |w|^2, and for the centring 1.w, r.w
+  auto sums = [&](const double (&w)[U], double& ww, double& sw, double& rw) {
+    double t0 = 0.0, t1 = 0.0, t2 = 0.0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      t0 += w[u] * w[u];
+      t1 += w[u];
+      t2 += r[u] * w[u];
+    }
+    const double v = wave_sum4_f64(t0, t1, t2, 0.0);
+    ww = readlane_f64(v, 0);
+    sw = readlane_f64(v, 16);
+    rw = readlane_f64(v, 32);
+  };
+  double qq, sv, rv;  // 1.q and r.q of the current basis vector
+  sums(q, qq, sv, rv);
+  double qp[U], own_q = xb[own_e], own_qp = 0.0, bprev = 0.0;  // the last vector, beta
+#pragma unroll
+  for (int u = 0; u < U; ++u) qp[u] = 0.0;
   for (int it = 0; it < jmax; ++it) {
-    wave_sym_matvec<kW>(S, d, U, q, w, xb, part, red);  // w = S q
-    if (!a.gram) {                   // w = M q = P S P q
-      double sv = 0.0, rv = 0.0;
+    matvec(w, own);  // w = S q
+    if (!a.gram) {   // w = M q = P S P q
+      const double shift = sigma * sv * inv_d * inv_d;
 #pragma unroll
-      for (int u = 0; u < kLzWaveU; ++u) {
-        sv += q[u];
-        rv += r[u] * q[u];
-      }
-      sv = wave_sum_f64(sv);
-      rv = wave_sum_f64(rv);
-#pragma unroll
-      for (int u = 0; u < kLzWaveU; ++u)
-        if (lane + 64 * u < d)
-          w[u] = w[u] - (r[u] * sv + rv) * inv_d + sigma * sv * inv_d * inv_d;
+      for (int u = 0; u < U; ++u)
+        if (lane + 64 * u < d) w[u] = w[u] - (r[u] * sv + rv) * inv_d + shift;
+      if (own_e < d) own = own - (own_r * sv + rv) * inv_d + shift;
     }
-    double nw2 = 0.0, qw = 0.0;
+    // three-term recurrence, then Gram-Schmidt against the whole basis,
+    // again when it removed more than half of |w|^2
+    double nw2, al;
+    dot2(w, w, q, w, nw2, al);
 #pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) {
-      nw2 += w[u] * w[u];
-      qw += q[u] * w[u];
+    for (int u = 0; u < U; ++u) {
+      w[u] = w[u] - al * q[u] - bprev * qp[u];
+      qp[u] = q[u];
     }
-    nw2 = wave_sum_f64(nw2);
-    qw = wave_sum_f64(qw);
-    double w1 = 0.0;
-#pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) {
-      w[u] = w[u] - qw * q[u] - bprev * qp[u];
-      w1 += w[u] * w[u];
-    }
-    w1 = wave_sum_f64(w1);
-    double b = sqrt(w1);
+    own = own - al * own_q - bprev * own_qp;
+    double w1 = dot(w, w), bb, sw, rw;
     for (int pass = 0; pass < 2; ++pass) {
-      // classical Gram-Schmidt against q_0..q_it, repeated when it removed
-      // more than 1 - 1/sqrt(2) of the norm; basis rows in groups of
-      // kLzWaveRows so that their loads are in flight together
-      for (int l0 = 0; l0 <= it; l0 += kLzWaveRows) {
-        double qv[kLzWaveRows][kLzWaveU];
-        wave_basis_rows(a.Q, d, U, l0, it, qv);
-#pragma unroll
-        for (int t = 0; t < kLzWaveRows; ++t) {
-          double dt = 0.0;
-#pragma unroll
-          for (int u = 0; u < kLzWaveU; ++u) dt += qv[t][u] * w[u];
-          dt = wave_sum_f64(dt);
-          if (lane == 0 && l0 + t <= it) cf[l0 + t] = dt;
-        }
-      }
-      wave_lds_sync();
-      for (int l0 = 0; l0 <= it; l0 += kLzWaveRows) {
-        double qv[kLzWaveRows][kLzWaveU];
-        wave_basis_rows(a.Q, d, U, l0, it, qv);
-#pragma unroll
-        for (int t = 0; t < kLzWaveRows; ++t) {
-          const double c = l0 + t <= it ? cf[l0 + t] : 0.0;
-#pragma unroll
-          for (int u = 0; u < kLzWaveU; ++u) w[u] -= c * qv[t][u];
-        }
-      }
-      double w2 = 0.0;
-#pragma unroll
-      for (int u = 0; u < kLzWaveU; ++u) w2 += w[u] * w[u];
-      w2 = wave_sum_f64(w2);
-      const bool again = w2 < 0.5 * w1;
-      b = sqrt(w2);
-      w1 = w2;
-      wave_lds_sync();  // cf is rewritten by the next pass
-      if (!again) break;
+      dots(w, it);
+      project(w, own, it);
+      sums(w, bb, sw, rw);
+      if (!(bb < 0.5 * w1)) break;
+      w1 = bb;
     }
-    if (lane == 0) alpha[it] = qw;
+    const double b = sqrt(bb);
+    if (threadIdx.x == 0) alpha[it] = al;
     len = it + 1;
     const bool breakdown = !(b > 1e-12 * sqrt(nw2));
     if (breakdown || len == jmax || lz_power_check(len)) {
-      wave_lds_sync();
-      tridiag_power_wave(alpha, beta, len, a.I, y);
-      wave_lds_sync();
-      double dd = 0.0;
-      for (int e = lane; e < len; e += 64) {
-        const double pv = e < prev_len ? yp[e] : 0.0;
-        dd += (y[e] - pv) * (y[e] - pv);
+      __syncthreads();  // alpha, beta visible
+      if (len <= kLzResSq) {
+        tridiag_power_mfma<NW>(alpha, beta, len, a.I, wk, y);
+      } else {
+        if (wv == 0) tridiag_power_wave(alpha, beta, len, a.I, y);
+        __syncthreads();
       }
-      dd = wave_sum_f64(dd);
+      const double y0 = lane < len ? y[lane] : 0.0, y1 = lane + 64 < len ? y[lane + 64] : 0.0;
+      const double dd = wave_sum_f64((y0 - yp0) * (y0 - yp0) + (y1 - yp1) * (y1 - yp1));
       conv = breakdown || (prev_len > 0 && sqrt(dd) <= lz_tol);
-      for (int e = lane; e < len; e += 64) yp[e] = y[e];
-      wave_lds_sync();
+      yp0 = y0;
+      yp1 = y1;
       prev_len = len;
       if (conv || breakdown) break;
     }
     if (len == jmax) break;
-    if (lane == 0) beta[it + 1] = b;
+    if (threadIdx.x == 0) beta[it + 1] = b;
     const double inv_b = 1.0 / b;
-    double* qn = a.Q + (long)(it + 1) * d;
 #pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) {
-      const int e = lane + 64 * u;
-      qp[u] = q[u];
-      q[u] = w[u] * inv_b;
-      if (e < d) qn[e] = q[u];
-    }
+    for (int u = 0; u < U; ++u) q[u] = w[u] * inv_b;
+    own_qp = own_q;
+    own_q = own * inv_b;
     bprev = b;
+    sv = sw * inv_b;
+    rv = rw * inv_b;
+    put(xb, q);
+    put_row(it + 1, q);
+    __syncthreads();
   }
   // v = Q y (zero when the check never passed, in the S form)
-  double v[kLzWaveU];
+  double v[U];
   int steps = len;
+#pragma unroll
+  for (int u = 0; u < U; ++u) v[u] = 0.0;
   if (conv) {
+    const int near = len < QL ? len : QL;
+#pragma unroll 4
+    for (int l = 0; l < near; ++l) {
+      const double c = y[l];
 #pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) v[u] = 0.0;
-    for (int l0 = 0; l0 < len; l0 += kLzWaveRows) {
-      double qv[kLzWaveRows][kLzWaveU];
-      wave_basis_rows(a.Q, d, U, l0, len - 1, qv);
-#pragma unroll
-      for (int t = 0; t < kLzWaveRows; ++t) {
-        const double c = l0 + t < len ? y[l0 + t] : 0.0;
-#pragma unroll
-        for (int u = 0; u < kLzWaveU; ++u) v[u] += c * qv[t][u];
-      }
+      for (int u = 0; u < U; ++u) v[u] += c * Qs[l * D + lane + 64 * u];
     }
-  } else if (!a.gram) {
+    for (int l = QL; l < len; ++l)
 #pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) v[u] = 0.0;
-  } else {
+      for (int u = 0; u < U; ++u) v[u] += y[l] * far_row(l, lane + 64 * u);
+  } else if (a.gram) {
     // Gram form: plain power steps from vstart (at most I, until the
     // Rayleigh quotient moves by <= 1e-12 relative); S v = 0 gives v = 0
 #pragma unroll
-    for (int u = 0; u < kLzWaveU; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int e = lane + 64 * u;
       v[u] = e < d ? a.vstart[e] / n0 : 0.0;
     }
     double lam_prev = 0.0;
     for (int t = 0; t < a.I; ++t) {
-      wave_sym_matvec<kW>(S, d, U, v, w, xb, part, red);
-      double nw2 = 0.0, vw = 0.0;
-#pragma unroll
-      for (int u = 0; u < kLzWaveU; ++u) {
-        nw2 += w[u] * w[u];
-        vw += v[u] * w[u];
-      }
-      nw2 = wave_sum_f64(nw2);
-      vw = wave_sum_f64(vw);
+      __syncthreads();  // the last product's reads of xb and part are done
+      put(xb, v);
+      __syncthreads();
+      matvec(w, own);
+      const double nw2 = dot(w, w), vw = dot(v, w);
       if (!(nw2 > 0.0)) {
 #pragma unroll
-        for (int u = 0; u < kLzWaveU; ++u) v[u] = 0.0;
+        for (int u = 0; u < U; ++u) v[u] = 0.0;
         break;
       }
       const double inv = 1.0 / sqrt(nw2);
 #pragma unroll
-      for (int u = 0; u < kLzWaveU; ++u) v[u] = w[u] * inv;
+      for (int u = 0; u < U; ++u) v[u] = w[u] * inv;
       ++steps;
       if (t > 0 && fabs(vw - lam_prev) <= 1e-12 * fabs(vw)) break;
       lam_prev = vw;
     }
     conv = 1;
   }
-  wave_sym_matvec<kW>(S, d, U, v, w, xb, part, red);  // h = S v
+  __syncthreads();
+  put(xb, v);
+  __syncthreads();
+  matvec(w, own);  // h = S v
 #pragma unroll
-  for (int u = 0; u < kLzWaveU; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int e = lane + 64 * u;
-    if (e < d && writer) {
+    if (u % NW == wv && e < d) {
       a.v[e] = v[u];
       a.h[e] = w[u];
     }
   }
-  if (lane == 0 && writer) {
+  if (threadIdx.x == 0) {
     *a.steps = steps;
     *a.conv = conv;
   }
+}
+
+// Clusters of a batch, one block each.
+template <int NW, int U, typename T>
+__global__ __launch_bounds__(64 * NW) void k_lz_res_group(const LzResJob* __restrict__ jobs,
+                                                          double lz_tol) {
+  const LzResJob a = jobs[blockIdx.x];
+  lz_res_body<NW, U, T>(a, lz_tol);
+}
+
+// The k clusters of one fit (S form), one block each.
+template <int NW, int U, typename T>
+__global__ __launch_bounds__(64 * NW) void k_lz_res(
+    const float* __restrict__ S, int m, const int* __restrict__ counts, uint64_t seed, int iter,
+    int I, double lz_tol, double* __restrict__ Q, double* __restrict__ vout,
+    double* __restrict__ svout, double* __restrict__ rout, int* __restrict__ steps_out,
+    int* __restrict__ conv_out) {
+  const long j = blockIdx.x;
+  if (counts[j] == 0) return;
+  const LzResJob a{S + j * m * m, m,        0,          I,           seed,          iter,
+                   (int)j,        nullptr,  Q + j * (kLzMax + 1) * m, vout + j * m, rout + j * m,
+                   svout + j * m, steps_out + j, conv_out + j};
+  lz_res_body<NW, U, T>(a, lz_tol);
 }
 
 #define TCX_GROUP_ARGS(T) static_cast<const T*>(g.jobs), g.first, g.njobs
@@ -3648,17 +3844,50 @@ hipError_t launch_gram_map(const GramVecJob* jobs, int njobs, size_t lds, hipStr
   return hipGetLastError();
 }
 
-hipError_t launch_lanczos_wave(const LzWaveJob* jobs, int njobs, int waves_per_cluster,
-                               double lz_tol, hipStream_t st) {
+int lz_res_form(int d) { return d <= 64 ? 0 : (d <= 128 ? 1 : 2); }
+
+hipError_t launch_lz_res_group(const LzResJob* jobs, int njobs, int form, double lz_tol,
+                               hipStream_t st) {
   if (njobs <= 0) return hipSuccess;
-  if (waves_per_cluster == 4)
-    hipLaunchKernelGGL(k_lanczos_wave<4>, dim3((unsigned)njobs), dim3(256), 0, st, jobs, njobs,
-                       lz_tol);
-  else if (waves_per_cluster == 1)
-    hipLaunchKernelGGL(k_lanczos_wave<1>, dim3((unsigned)((njobs + 3) / 4)), dim3(256), 0, st,
-                       jobs, njobs, lz_tol);
-  else
-    return hipErrorInvalidValue;
+  const dim3 grid((unsigned)njobs);
+  switch (form) {
+    case 0:
+      hipLaunchKernelGGL((k_lz_res_group<4, 1, double>), grid, dim3(256), (lz_res_lds<4, 1>()), st,
+                         jobs, lz_tol);
+      break;
+    case 1:
+      hipLaunchKernelGGL((k_lz_res_group<4, 2, double>), grid, dim3(256), (lz_res_lds<4, 2>()), st,
+                         jobs, lz_tol);
+      break;
+    case 2:
+      hipLaunchKernelGGL((k_lz_res_group<8, 4, float>), grid, dim3(512), (lz_res_lds<8, 4>()), st,
+                         jobs, lz_tol);
+      break;
+    default:
+      return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_lz_res(const float* S, int m, int k, const int* counts, uint64_t seed, int iter,
+                         int I, double lz_tol, double* Q, double* vout, double* svout,
+                         double* rout, int* steps_out, int* conv_out, hipStream_t st) {
+  if (k <= 0) return hipSuccess;
+  if (m > kLzResMaxD) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)k);
+  switch (lz_res_form(m)) {
+    case 0:
+      hipLaunchKernelGGL((k_lz_res<4, 1, double>), grid, dim3(256), (lz_res_lds<4, 1>()), st, S, m,
+                         counts, seed, iter, I, lz_tol, Q, vout, svout, rout, steps_out, conv_out);
+      break;
+    case 1:
+      hipLaunchKernelGGL((k_lz_res<4, 2, double>), grid, dim3(256), (lz_res_lds<4, 2>()), st, S, m,
+                         counts, seed, iter, I, lz_tol, Q, vout, svout, rout, steps_out, conv_out);
+      break;
+    default:
+      hipLaunchKernelGGL((k_lz_res<8, 4, float>), grid, dim3(512), (lz_res_lds<8, 4>()), st, S, m,
+                         counts, seed, iter, I, lz_tol, Q, vout, svout, rout, steps_out, conv_out);
+  }
   return hipGetLastError();
 }
 
@@ -3742,6 +3971,19 @@ hipError_t configure_extract_kernels() {
   if (e == hipSuccess)
     e = hipFuncSetAttribute((const void*)k_align_pack_lds<16>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, kPackLdsMaxBytes);
+#define TCX_LZ_RES(NW, U, T)                                                                 \
+  if (e == hipSuccess)                                                                       \
+    e = hipFuncSetAttribute((const void*)k_lz_res<NW, U, T>,                                 \
+                            hipFuncAttributeMaxDynamicSharedMemorySize,                      \
+                            (int)lz_res_lds<NW, U>());                                       \
+  if (e == hipSuccess)                                                                       \
+    e = hipFuncSetAttribute((const void*)k_lz_res_group<NW, U, T>,                           \
+                            hipFuncAttributeMaxDynamicSharedMemorySize,                      \
+                            (int)lz_res_lds<NW, U>());
+  TCX_LZ_RES(4, 1, double)
+  TCX_LZ_RES(4, 2, double)
+  TCX_LZ_RES(8, 4, float)
+#undef TCX_LZ_RES
   // grouped forms
   if (e == hipSuccess)
     e = hipFuncSetAttribute((const void*)k_power_group, hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -412,6 +412,17 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
   TCX_TRY(ws(c, kSlotSteps, (size_t)k, &st_out));
   TCX_TRY(ws(c, kSlotConv, (size_t)k, &cv_out));
   TCX_TRY(ws(c, kSlotLzState, (size_t)k, &state));
+  if (mode == 0 && !mask && m <= tcx::kLzResMaxD) {
+    // S_j fits the registers of one block: every step in one launch, S v too
+    TCX_HIP(tcx::launch_lz_res(S, m, k, counts, seed, iter, steps, tcx::kLzPowerTol, Q, v, sv, r,
+                               st_out, cv_out, st));
+    *vout = v;
+    *svout = sv;
+    *rout = r;
+    *steps_out = st_out;
+    *conv_out = cv_out;
+    return TCX_OK;
+  }
   tcx::LzCoopPlan cp;
   if (mode == 0 && !mask && tcx::plan_lz_coop(m, k, c->cus, &cp)) {
     // exchange words and per-cluster failure words; their contents only

@@ -511,30 +511,31 @@ hipError_t launch_gram_lanczos(const GramLzJob* jobs, int njobs, size_t lds, dou
                                hipStream_t st);
 hipError_t launch_gram_map(const GramVecJob* jobs, int njobs, size_t lds, hipStream_t st);
 
-// One wave per cluster of dimension d <= kLzWaveMaxD: the Lanczos
-// evaluation of the power iterate on the cluster's S (S form: centring,
-// start power_v0(seed, iter, cluster, .), r = S 1 written) or on its Gram
-// matrix (start vstart, no centring, power steps when the check never
-// passes); v = the iterate's direction, h = S v (the matrix given).
-constexpr int kLzWaveMaxD = 256;
-struct LzWaveJob {
+// Resident Lanczos for orders d <= kLzResMaxD: one block per cluster, the
+// matrix in registers (k_lz_res).  S form: M = P S P from power_v0, v =
+// M^I v0, h = S v, r = S 1.  Gram form: no centring, start vstart, v =
+// S^I vstart / |.|, h = S v.
+constexpr int kLzResMaxD = 256;
+struct LzResJob {
   const float* S;  // d x d, row stride d
   int d, gram, I;
   uint64_t seed;
   int iter, cluster;
   const double* vstart;  // Gram form
-  double* Q;             // (kLanczosMax + 1) x d
+  double* Q;             // (kLanczosMax + 1) x d: basis rows past those in LDS
   double* v;
   double* r;             // S form
   double* h;
   int* steps;
   int* conv;
 };
-// waves_per_cluster 1: four clusters per block; 4: one cluster per block,
-// each matvec shared by its four waves (for the larger orders)
-hipError_t launch_lanczos_wave(const LzWaveJob* jobs, int njobs, int waves_per_cluster,
-                               double lz_tol, hipStream_t st);
-constexpr int kLzWaveSplitD = 128;  // orders above this take four waves
+// Register split by order: 0 up to 64, 1 up to 128, 2 up to 256.
+int lz_res_form(int d);
+hipError_t launch_lz_res_group(const LzResJob* jobs, int njobs, int form, double lz_tol,
+                               hipStream_t st);
+hipError_t launch_lz_res(const float* S, int m, int k, const int* counts, uint64_t seed, int iter,
+                         int I, double lz_tol, double* Q, double* vout, double* svout,
+                         double* rout, int* steps_out, int* conv_out, hipStream_t st);
 
 struct ClusterMatvecJob {
   const float* S;
