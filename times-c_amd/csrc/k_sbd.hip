@@ -123,11 +123,11 @@ __device__ __forceinline__ void spectra_body(const int bid, const int nblk,
   constexpr int L = G::L, P = G::P;
   extern __shared__ float2 smem[];
   float2* tw = smem;
-  float* red = reinterpret_cast<float*>(smem + F + G::kGroups * fft_buf_len<F>());
-  for (int i = threadIdx.x; i < F; i += blockDim.x) tw[i] = twg[i];
+  float* red = reinterpret_cast<float*>(smem + fft_tw_lds<F>() + G::kGroups * fft_buf_len<F>());
+  for (int i = threadIdx.x; i < fft_tw_lds<F>(); i += blockDim.x) tw[i] = twg[i];
   __syncthreads();
   const int g = threadIdx.x / L, lane = threadIdx.x % L;
-  float2* buf = smem + F + g * fft_buf_len<F>();
+  float2* buf = smem + fft_tw_lds<F>() + g * fft_buf_len<F>();
   for (int row = bid * G::kGroups + g; row < rows; row += nblk * G::kGroups) {
     const float* yr = y + (long)row * m;
     float2 v[P];
@@ -143,7 +143,7 @@ __device__ __forceinline__ void spectra_body(const int bid, const int nblk,
     }
     ss = group_sum<L>(ss, red);
     float fnz = group_sum<L>((float)nz, red);
-    fft<F, L, false>(v, buf, tw, lane);
+    fft<F, L, false>(v, buf, tw, twg, lane);
     float2* o = spec + (long)row * F;
 #pragma unroll
     for (int s = 0; s < P; ++s) o[s * L + lane] = v[s];
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock) void k_spectra(
 // NCC: write cc / F / (|x| |y|) for all 2m-1 lags (ncc.cuh:467-517 layout
 // out[x][y][lag]).
 template <int F, int MODE>
-__global__ __launch_bounds__(FftGeom<F>::kBlock) void k_sbd(
+__global__ __launch_bounds__(FftGeom<F>::kBlock, MODE == kModeAssign ? FftGeom<F>::kMinWaves : 1) void k_sbd(
     const float* __restrict__ x, long n, int m, int k,
     const float2* __restrict__ cspec, const float* __restrict__ cnorm,
     const float2* __restrict__ twg, int rev, int* __restrict__ label,
@@ -199,15 +199,13 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock) void k_sbd(
   constexpr int L = G::L, P = G::P;
   extern __shared__ float2 smem[];
   float2* tw = smem;
-  float* red = reinterpret_cast<float*>(smem + F + G::kGroups * fft_buf_len<F>());
-  for (int i = threadIdx.x; i < F; i += blockDim.x) tw[i] = twg[i];
+  float* red = reinterpret_cast<float*>(smem + fft_tw_lds<F>() + G::kGroups * fft_buf_len<F>());
+  for (int i = threadIdx.x; i < fft_tw_lds<F>(); i += blockDim.x) tw[i] = twg[i];
   __syncthreads();
   const int g = threadIdx.x / L, lane = threadIdx.x % L;
-  float2* buf = smem + F + g * fft_buf_len<F>();
+  float2* buf = smem + fft_tw_lds<F>() + g * fft_buf_len<F>();
   const long npairs = (n + 1) / 2;
   const int nlag = 2 * m - 1;
-  int s_lo, s_hi;
-  lag_rows(lane, L, m, F, s_lo, s_hi);
   for (long pr = (long)blockIdx.x * G::kGroups + g; pr < npairs;
        pr += (long)gridDim.x * G::kGroups) {
     const long ia = 2 * pr, ib = 2 * pr + 1;
@@ -216,11 +214,12 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock) void k_sbd(
     const float* xb = x + (hasb ? ib : ia) * (long)m;
     float2 zx[P];
     float sa = 0.f, sb = 0.f;
+    const int ml = opaque(m);
 #pragma unroll
     for (int s = 0; s < P; ++s) {
       int t = lane + L * s;
-      float a = t < m ? xa[t] : 0.f;
-      float b = (hasb && t < m) ? xb[t] : 0.f;
+      float a = t < ml ? xa[t] : 0.f;
+      float b = (hasb && t < ml) ? xb[t] : 0.f;
       zx[s] = make_float2(a, b);
       sa += a * a;
       sb += b * b;
@@ -228,7 +227,7 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock) void k_sbd(
     sa = group_sum<L>(sa, red);
     sb = group_sum<L>(sb, red);
     const float na = sqrtf(sa), nb = sqrtf(sb);
-    fft<F, L, false>(zx, buf, tw, lane);
+    fft<F, L, false>(zx, buf, tw, twg, lane);
 
     float bestA = INFINITY, bestB = INFINITY;
     int labA = 0, labB = 0, keyA = 0, keyB = 0;
@@ -240,15 +239,13 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock) void k_sbd(
       float2 z[P];
 #pragma unroll
       for (int s = 0; s < P; ++s) z[s] = cmulc(zx[s], cj[s * L + lane]);
-      fft<F, L, true>(z, buf, tw, lane);
+      fft<F, L, true>(z, buf, tw, twg, lane);
       const float cn = cnorm[j];
       const float dena = na * cn, denb = nb * cn;
       if constexpr (MODE == kModeAssign) {
         float va, vb;
         int ka, kb;
-        lag_argmax2<L, P>(z, s_lo, s_hi, rev, lane, m, F, va, ka, vb, kb);
-        group_argmax<L>(va, ka, red);
-        group_argmax<L>(vb, kb, red);
+        lag_max<F, L, P>(z, rev, lane, m, red, va, ka, vb, kb);
         // den == 0: NumPy divides by inf, every lag is 0, argmax is index 0
         float da = 1.f, db = 1.f;
         if (dena != 0.f) da = 1.f - (va / (float)F) / dena; else ka = 0;
@@ -437,11 +434,11 @@ __device__ __forceinline__ void series_spec_body(const int bid, const int nblk,
   constexpr long HS = F / 2 + 1;
   extern __shared__ float2 smem[];
   float2* tw = smem;
-  float* red = reinterpret_cast<float*>(smem + F + G::kGroups * fft_buf_len<F>());
-  for (int i = threadIdx.x; i < F; i += blockDim.x) tw[i] = twg[i];
+  float* red = reinterpret_cast<float*>(smem + fft_tw_lds<F>() + G::kGroups * fft_buf_len<F>());
+  for (int i = threadIdx.x; i < fft_tw_lds<F>(); i += blockDim.x) tw[i] = twg[i];
   __syncthreads();
   const int g = threadIdx.x / L, lane = threadIdx.x % L;
-  float2* buf = smem + F + g * fft_buf_len<F>();
+  float2* buf = smem + fft_tw_lds<F>() + g * fft_buf_len<F>();
   const long npairs = (n + 1) / 2;
   for (long pr = (long)bid * G::kGroups + g; pr < npairs;
        pr += (long)nblk * G::kGroups) {
@@ -451,11 +448,12 @@ __device__ __forceinline__ void series_spec_body(const int bid, const int nblk,
     const float* xb = x + (hasb ? ib : ia) * (long)m;
     float2 zx[P];
     float sa = 0.f, sb = 0.f;
+    const int ml = opaque(m);
 #pragma unroll
     for (int s = 0; s < P; ++s) {
       const int t = lane + L * s;
-      const float a = t < m ? xa[t] : 0.f;
-      const float b = (hasb && t < m) ? xb[t] : 0.f;
+      const float a = t < ml ? xa[t] : 0.f;
+      const float b = (hasb && t < ml) ? xb[t] : 0.f;
       zx[s] = make_float2(a, b);
       sa += a * a;
       sb += b * b;
@@ -466,7 +464,7 @@ __device__ __forceinline__ void series_spec_body(const int bid, const int nblk,
       xn[ia] = sqrtf(sa);
       if (hasb) xn[ib] = sqrtf(sb);
     }
-    fft<F, L, false>(zx, buf, tw, lane);
+    fft<F, L, false>(zx, buf, tw, twg, lane);
     float px[H + 1], py[H + 1];
     partner_half<F, L, P>(zx, buf, lane, px, py);
     float2* oa = xs + ia * HS;
@@ -501,7 +499,7 @@ __device__ __forceinline__ void series_spec_body(const int bid, const int nblk,
 }
 
 template <int F>
-__global__ __launch_bounds__(FftGeom<F>::kBlock) void k_series_spec(
+__global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWaves) void k_series_spec(
     const float* __restrict__ x, long n, int m, const float2* __restrict__ twg,
     float2* __restrict__ xs, float* __restrict__ xn, uint16_t* __restrict__ xm) {
   series_spec_body<F>(blockIdx.x, gridDim.x, x, n, m, twg, xs, xn, xm);
@@ -665,9 +663,7 @@ struct PruneGeom {
   static constexpr int L = FftGeom<F>::L;
   static constexpr int kBlock = FftGeom<F>::kBlock;
   static constexpr int kGroups = kBlock / L;
-  // waves per SIMD the register allocation must allow: three 256-thread
-  // blocks fit a CU's LDS up to F = 1024 (168 VGPRs per lane)
-  static constexpr int kMinWaves = F <= 1024 ? 3 : 1;
+  static constexpr int kMinWaves = FftGeom<F>::kMinWaves;
 };
 
 template <int F, bool kPre>
@@ -682,16 +678,14 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
   constexpr int L = G::L, P = FftGeom<F>::P;
   extern __shared__ float2 smem[];
   float2* tw = smem;
-  float* red = reinterpret_cast<float*>(smem + F + G::kGroups * fft_buf_len<F>());
+  float* red = reinterpret_cast<float*>(smem + fft_tw_lds<F>() + G::kGroups * fft_buf_len<F>());
   float* ubs_all = red + 64;
-  for (int i = threadIdx.x; i < F; i += blockDim.x) tw[i] = twg[i];
+  for (int i = threadIdx.x; i < fft_tw_lds<F>(); i += blockDim.x) tw[i] = twg[i];
   __syncthreads();
   const int g = threadIdx.x / L, lane = threadIdx.x % L;
-  float2* buf = smem + F + g * fft_buf_len<F>();
+  float2* buf = smem + fft_tw_lds<F>() + g * fft_buf_len<F>();
   float* ubs = ubs_all + (long)g * 2 * k;  // [0,k): series a, [k,2k): series b
   unsigned long long my_evals = 0;
-  int s_lo, s_hi;
-  lag_rows(lane, L, m, F, s_lo, s_hi);
   for (long pr = (long)bid * G::kGroups + g; pr < npairs;
        pr += (long)nblk * G::kGroups) {
     long ia = order ? order[2 * pr] : 2 * pr;
@@ -747,11 +741,12 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
       const float* xa = x + ia * (long)m;
       const float* xb = x + (hasb ? ib : ia) * (long)m;
       float sa = 0.f, sb = 0.f;
+    const int ml = opaque(m);
 #pragma unroll
       for (int s = 0; s < P; ++s) {
         const int t = lane + L * s;
-        const float a = t < m ? xa[t] : 0.f;
-        const float b = (hasb && t < m) ? xb[t] : 0.f;
+        const float a = t < ml ? xa[t] : 0.f;
+        const float b = (hasb && t < ml) ? xb[t] : 0.f;
         zx[s] = make_float2(a, b);
         sa += a * a;
         sb += b * b;
@@ -760,7 +755,7 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
       sb = group_sum<L>(sb, red);
       na = sqrtf(sa);
       nb = sqrtf(sb);
-      fft<F, L, false>(zx, buf, tw, lane);
+      fft<F, L, false>(zx, buf, tw, twg, lane);
       // |X_a[f]| = |Z[f] + conj(Z[F-f])| / 2, |X_b[f]| = |Z[f] - conj(Z[F-f])| / 2
       float px[H + 1], py[H + 1];
       float ma[H + 1], mb[H + 1];
@@ -778,13 +773,15 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
     group_sync<L>();
     float bestA = INFINITY, bestB = hasb ? INFINITY : -INFINITY;
     int labA = 0, labB = 0, keyA = 0, keyB = 0;
-    // one-wave group with k <= 64: centroid j's two bounds stay in lane j's
-    // registers (-1: evaluated), the next candidate is a wave max and a ballot
-    const bool inreg = L == kWave && k <= kWave;  // uniform
+    // groups of whole waves with k <= 64: centroid j's two bounds stay in the
+    // registers of lane j of every wave (-1: evaluated), the next candidate
+    // is a wave max and a ballot, the same in every wave
+    const bool inreg = L >= kWave && k <= kWave;  // uniform
+    const int wl = lane & (kWave - 1);
     float myA = -1.f, myB = -1.f;
-    if (inreg && lane < k) {
-      myA = ubs[lane];
-      myB = ubs[k + lane];
+    if (inreg && wl < k) {
+      myA = ubs[wl];
+      myB = ubs[k + wl];
     }
     for (int round = 0; round < k; ++round) {
       // candidate with the largest bound among centroids that can still win
@@ -812,15 +809,17 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
       }
       if (!(sc > -INFINITY)) break;
       const int j = cj;
-      group_sync<L>();
       if (inreg) {
-        if (lane == j) {
+        if (wl == j) {
           myA = -1.f;  // evaluated
           myB = -1.f;
         }
-      } else if (lane == 0) {
-        ubs[j] = -1.f;  // evaluated
-        ubs[k + j] = -1.f;
+      } else {
+        group_sync<L>();
+        if (lane == 0) {
+          ubs[j] = -1.f;  // evaluated
+          ubs[k + j] = -1.f;
+        }
       }
       const float cn = cnorm[j];
       const float dena = na * cn, denb = nb * cn;
@@ -832,31 +831,17 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
         float2 z[P];
 #pragma unroll
         for (int s = 0; s < P; ++s) z[s] = cmulc(zx[s], cjs[s * L + lane]);
-        fft<F, L, true>(z, buf, tw, lane);
+        fft<F, L, true>(z, buf, tw, twg, lane);
         float va, vb;
-        if constexpr (L == kWave) {
-          // m through an empty asm: the row tests are then a few scalar
-          // operations here instead of loop invariants held (and spilled)
-          // across the whole loop
-          int mo = m;
-          asm volatile("" : "+s"(mo));
-          lag_max_wave<P>(z, rev, lane, mo, F, va, ka, vb, kb);
-        } else if constexpr (L > kWave) {
-          int mo = m;
-          asm volatile("" : "+s"(mo));
-          lag_max_group<L, P>(z, rev, lane, mo, F, red, va, ka, vb, kb);
-        } else {
-          lag_argmax2<L, P>(z, s_lo, s_hi, rev, lane, m, F, va, ka, vb, kb);
-          group_argmax<L>(va, ka, red);
-          group_argmax<L>(vb, kb, red);
-        }
+        lag_max<F, L, P>(z, rev, lane, m, red, va, ka, vb, kb);
         if (dena != 0.f) da = 1.f - (va / (float)F) / dena; else ka = 0;
         if (denb != 0.f) db = 1.f - (vb / (float)F) / denb; else kb = 0;
       }
       if (da < bestA || (da == bestA && j < labA)) { bestA = da; labA = j; keyA = ka; }
       if (hasb && (db < bestB || (db == bestB && j < labB))) { bestB = db; labB = j; keyB = kb; }
-      group_sync<L>();
+      if (!inreg) group_sync<L>();  // ubs of the evaluated centroid is written
     }
+    group_sync<L>();  // ubs is rewritten by the next pair
     if (lane == 0) {
       if (changed && label[ia] != labA) *changed = 1;
       label[ia] = labA;
@@ -936,7 +921,7 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock) void k_spectra_group(
 }
 
 template <int F>
-__global__ __launch_bounds__(FftGeom<F>::kBlock) void k_series_spec_group(
+__global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWaves) void k_series_spec_group(
     const SeriesSpecJob* __restrict__ jobs, const int* __restrict__ first, int njobs,
     const float2* __restrict__ twg) {
   TCX_GROUP_JOB(SeriesSpecJob)
@@ -966,7 +951,7 @@ __global__ __launch_bounds__(PruneGeom<F>::kBlock, PruneGeom<F>::kMinWaves) void
 template <int F>
 static size_t sbd_smem() {
   using G = FftGeom<F>;
-  return sizeof(float2) * (F + G::kGroups * fft_buf_len<F>()) + sizeof(float) * 64;
+  return sizeof(float2) * (fft_tw_lds<F>() + G::kGroups * fft_buf_len<F>()) + sizeof(float) * 64;
 }
 
 template <int F>
@@ -998,7 +983,7 @@ static hipError_t launch_sbd_F(const SbdArgs& a, hipStream_t st) {
 template <int F>
 static size_t prune_smem(int k) {
   using G = PruneGeom<F>;
-  return sizeof(float2) * (F + G::kGroups * fft_buf_len<F>()) + sizeof(float) * 64 +
+  return sizeof(float2) * (fft_tw_lds<F>() + G::kGroups * fft_buf_len<F>()) + sizeof(float) * 64 +
          sizeof(float) * 2 * (size_t)k * G::kGroups;
 }
 

@@ -39,6 +39,14 @@ __device__ __forceinline__ int group_job(const int* __restrict__ first, int njob
   return lo;
 }
 
+// v (uniform) through an empty asm: what is computed from it stays where it is
+// used, e.g. the row masks lane + L*s < m of a load phase, which as loop
+// invariants would hold (and spill) two scalar registers each.
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
+
 // ------------------------------------------------------- synchronisation
 // LDS exchange inside one wavefront: a wave's LDS operations complete in
 // issue order, so only the compiler must be kept from reordering.
@@ -335,7 +343,9 @@ __device__ __forceinline__ void dft(float2* v) {
 //     v[s] of lane l  <->  element l + L*s.
 // Passes are radix P (the first reads registers directly, the last leaves
 // its output in registers); between passes the data goes through the
-// group's LDS buffer `buf`.  `tw` holds exp(-2 pi i q / F), q < F, in LDS.
+// group's LDS buffer `buf`.  `tw` holds the twiddles in LDS (the first
+// fft_tw_lds entries of the table `twg` in global memory, which the passes
+// past them read).
 // The forward transform's output order equals the inverse transform's input
 // order, so spectra are multiplied in place without any reordering.
 __device__ __forceinline__ int lds_pad(int i) { return i + (i >> 5); }
@@ -365,9 +375,23 @@ __host__ __device__ constexpr int tw_offset(int F, int P, int Ns) {
   return off;
 }
 
+// Entries of the twiddle table a block keeps in LDS.  Up to F = 1024 all of
+// them.  Above, only the pass with stride 16 (240 entries); the later passes
+// read the global table (consecutive entries per wave, 14 to 30 KB per pass,
+// shared by every block through L1 and L2), so that the LDS of a block is
+// little more than its exchange buffer: 19 instead of 33 KB at F = 2048, 36
+// instead of 67 KB at 4096, 70 instead of 132 KB at 8192, i.e. twice the
+// blocks per CU.
+constexpr int kTwLdsMaxNs = 16;
+template <int F>
+constexpr int fft_tw_lds() {
+  return F <= 1024 ? F : tw_offset(F, F / fft_lanes(F), kTwLdsMaxNs * 16);
+}
+
 template <int F, int L, bool INV, int Ns>
 __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
-                                              const float2* tw, int lane) {
+                                              const float2* tw,
+                                              const float2* __restrict__ twg, int lane) {
   constexpr int P = F / L;
   constexpr int R = (F / Ns < P) ? F / Ns : P;
   constexpr int NB = P / R;
@@ -406,9 +430,12 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
     float2* b = u + t * R;
     if constexpr (!kFirst) {
       constexpr int kOff = tw_offset(F, P, Ns);
+      constexpr bool kLds = kOff + (R - 1) * Ns <= fft_tw_lds<F>();
+      int z = 0;  // opaque: table entries are read per pass, not held in registers
+      if constexpr (!kLds) asm volatile("" : "+s"(z));
 #pragma unroll
       for (int r = 1; r < R; ++r) {
-        const float2 w = tw[kOff + (r - 1) * Ns + kk];
+        const float2 w = kLds ? tw[kOff + (r - 1) * Ns + kk] : twg[z + kOff + (r - 1) * Ns + kk];
         b[r] = INV ? cmulc(b[r], w) : cmul(b[r], w);
       }
     }
@@ -429,16 +456,16 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
   }
   if constexpr (!kLast) {
     group_sync<L>();
-    stockham_pass<F, L, INV, Ns * R>(v, buf, tw, lane);
+    stockham_pass<F, L, INV, Ns * R>(v, buf, tw, twg, lane);
   }
 }
 
 // Unnormalized transform: forward uses exp(-2 pi i f t / F), inverse
 // exp(+2 pi i f t / F) (no 1/F).
 template <int F, int L, bool INV>
-__device__ __forceinline__ void fft(float2 (&v)[F / L], float2* buf,
-                                    const float2* tw, int lane) {
-  stockham_pass<F, L, INV, 1>(v, buf, tw, lane);
+__device__ __forceinline__ void fft(float2 (&v)[F / L], float2* buf, const float2* tw,
+                                    const float2* __restrict__ twg, int lane) {
+  stockham_pass<F, L, INV, 1>(v, buf, tw, twg, lane);
 }
 
 // Lane-group geometry per FFT length: L lanes, P = F/L values per lane.
@@ -448,6 +475,10 @@ struct FftGeom {
   static constexpr int P = F / L;
   static constexpr int kBlock = L <= kWave ? 256 : L;  // threads per block
   static constexpr int kGroups = kBlock / L;           // lane groups per block
+  // waves per SIMD the register allocation must allow, as many as the LDS of
+  // a CU's blocks does: three at 168 VGPRs, at F = 8192 (blocks of 8 waves)
+  // two blocks or four waves at 128
+  static constexpr int kMinWaves = F <= 4096 ? 3 : 4;
 };
 
 // Lag key of circular correlation position tau (0 <= tau < F): the index in
@@ -522,197 +553,166 @@ __device__ __forceinline__ int dpp_i32(int v) {
   return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, false);
 }
 
+// Maximum (minimum) of an integer over a group of W <= 64 lanes; every lane
+// of the group gets it.
+template <int W, bool MAX>
+__device__ __forceinline__ int group_ext_i32(int k) {
+  auto ext = [](int a, int b) { return MAX ? max(a, b) : min(a, b); };
+  if constexpr (W >= 2) k = ext(k, dpp_i32<0xB1>(k));   // lane ^ 1
+  if constexpr (W >= 4) k = ext(k, dpp_i32<0x4E>(k));   // lane ^ 2
+  if constexpr (W >= 8) k = ext(k, dpp_i32<0x141>(k));  // mirror in 8 lanes
+  if constexpr (W >= 16) k = ext(k, dpp_i32<0x140>(k)); // mirror in 16 lanes
+  if constexpr (W == 32) {
+    const int a = ext(__builtin_amdgcn_readlane(k, 0), __builtin_amdgcn_readlane(k, 16));
+    const int b = ext(__builtin_amdgcn_readlane(k, 32), __builtin_amdgcn_readlane(k, 48));
+    k = (threadIdx.x & 32) ? b : a;
+  } else if constexpr (W == 64) {
+    k = ext(ext(__builtin_amdgcn_readlane(k, 0), __builtin_amdgcn_readlane(k, 16)),
+            ext(__builtin_amdgcn_readlane(k, 32), __builtin_amdgcn_readlane(k, 48)));
+  }
+  return k;
+}
+
 // Wave maximum of v, which must not be NaN (every lane gets it), on the
 // integer images: no NaN canonicalization between the DPP steps.
 __device__ __forceinline__ float wave_max(float v) {
-  int k = f32_ord(v);
-  k = max(k, dpp_i32<0xB1>(k));   // lane ^ 1
-  k = max(k, dpp_i32<0x4E>(k));   // lane ^ 2
-  k = max(k, dpp_i32<0x141>(k));  // mirror in 8 lanes
-  k = max(k, dpp_i32<0x140>(k));  // mirror in 16 lanes
-  const int a = max(__builtin_amdgcn_readlane(k, 0), __builtin_amdgcn_readlane(k, 16));
-  const int b = max(__builtin_amdgcn_readlane(k, 32), __builtin_amdgcn_readlane(k, 48));
-  return ord_f32(max(a, b));
+  return ord_f32(group_ext_i32<kWave, true>(f32_ord(v)));
 }
 
-// lag_argmax2 followed by group_argmax of both results, for a one-wave
-// group (L = 64): the same values and keys, fewer instructions.  Each
-// series' maximum g is a per-lane max (NaN never wins, as the scan's '>'
-// never takes it) then a wave max; its key is the first lag holding g in
-// key order, found by one ballot per row visited in key order (rows
-// P/2..P-1 then 0..P/2-1, ascending lanes; mirrored when rev, whose keys
-// run the other way), so ties keep the smallest key; a row holding g is
-// then masked to its lags (tau in [m, F-m] is no lag).  g is first taken
-// over all F positions; only if no lag holds it (every lag below some
-// non-lag: the non-lags hold the circular wrap, about 0) is it taken again
-// over the lags alone.
+// First lag key, in a one-wave group, whose value in z (isx: the first
+// series') is g, INT_MAX if none.  Rows are visited in key order (P/2..P-1
+// then 0..P/2-1, ascending lanes; mirrored when rev, whose keys run the other
+// way), one compare and one scalar test each until the first hit: that
+// leaves the vector ALU, which bounds the one-wave kernels, less work than a
+// select per row.
 template <int P>
-__device__ __forceinline__ void lag_max_wave(const float2 (&z)[P], int rev, int lane, int m,
-                                             int F, float& va, int& ka, float& vb, int& kb) {
-  constexpr int L = kWave;
-  auto is_lag = [&](int s) {
-    const int tau = lane + L * s;
-    return tau <= m - 1 || tau >= F - m + 1;
+__device__ __forceinline__ int wave_first_key(const float2 (&z)[P], bool isx, float g, int rev,
+                                              int m, int F) {
+  if (!(g > -INFINITY)) return 0x7fffffff;  // no lag taken (uniform)
+  const int lane = threadIdx.x & (kWave - 1);
+  int key = 0x7fffffff;
+  auto row = [&](int s) -> bool {
+    uint64_t b = __ballot((isx ? z[s].x : z[s].y) == g);
+    if (!b) return false;
+    const int tau = lane + kWave * s;
+    b &= __ballot(tau <= m - 1 || tau >= F - m + 1);  // only on a row holding g
+    if (!b) return false;
+    const int ln = rev ? 63 - __builtin_clzll(b) : __builtin_ctzll(b);
+    key = lag_key(ln + kWave * s, m, F, rev);
+    return true;
   };
-  auto find = [&](float g, bool isx, int& key) -> bool {
-    key = 0x7fffffff;
-    if (!(g > -INFINITY)) return true;  // no lag taken (uniform)
-    auto row = [&](int s) -> bool {
-      uint64_t b = __ballot((isx ? z[s].x : z[s].y) == g);
-      if (!b) return false;
-      b &= __ballot(is_lag(s));  // only on a row holding g
-      if (!b) return false;
-      const int ln = rev ? 63 - __builtin_clzll(b) : __builtin_ctzll(b);
-      key = lag_key(ln + L * s, m, F, rev);
-      return true;
-    };
-    if (!rev) {
+  if (!rev) {
 #pragma unroll
-      for (int s = P / 2; s < P; ++s)
-        if (row(s)) return true;
+    for (int s = P / 2; s < P; ++s)
+      if (row(s)) return key;
 #pragma unroll
-      for (int s = 0; s < P / 2; ++s)
-        if (row(s)) return true;
-    } else {
+    for (int s = 0; s < P / 2; ++s)
+      if (row(s)) return key;
+  } else {
 #pragma unroll
-      for (int s = P / 2 - 1; s >= 0; --s)
-        if (row(s)) return true;
+    for (int s = P / 2 - 1; s >= 0; --s)
+      if (row(s)) return key;
 #pragma unroll
-      for (int s = P - 1; s >= P / 2; --s)
-        if (row(s)) return true;
-    }
-    return false;
-  };
-  float mx = -INFINITY, my = -INFINITY;
-#pragma unroll
-  for (int s = 0; s < P; ++s) {
-    mx = fmaxf(mx, z[s].x);
-    my = fmaxf(my, z[s].y);
+    for (int s = P - 1; s >= P / 2; --s)
+      if (row(s)) return key;
   }
-  va = wave_max(mx);
-  vb = wave_max(my);
-  if (find(va, true, ka) && find(vb, false, kb)) return;
-  // rare: the maximum over the lags alone
-  mx = -INFINITY;
-  my = -INFINITY;
-#pragma unroll
-  for (int s = 0; s < P; ++s) {
-    const bool ok = is_lag(s);
-    mx = ok ? fmaxf(mx, z[s].x) : mx;
-    my = ok ? fmaxf(my, z[s].y) : my;
-  }
-  va = wave_max(mx);
-  vb = wave_max(my);
-  find(va, true, ka);
-  find(vb, false, kb);
+  return key;
 }
 
-// lag_max_wave for a group of L = 64 * NW lanes (NW waves, the whole
-// block, P values per lane): each wave takes the maximum of its lanes; the
-// group maximum g goes through LDS (`red`, 2 * NW words); each wave then
-// finds its first lag holding g in key order over its own lanes (rows in
-// key order; within a row the keys run with the group lane, so the first
-// key of the group is the smallest of the waves' first keys), and the
-// smallest key goes through LDS again.  If no lag holds g, the same over
-// the lags alone.  Equal to lag_argmax2 followed by group_argmax.
-template <int L, int P>
-__device__ __forceinline__ void lag_max_group(const float2 (&z)[P], int rev, int glane, int m,
-                                              int F, float* red, float& va, int& ka, float& vb,
-                                              int& kb) {
-  static_assert(L > kWave && L % kWave == 0, "multi-wave group");
-  constexpr int NW = L / kWave;
-  const int w = glane / kWave, lane = glane % kWave;
+// lag_argmax2 followed by group_argmax of both results: the same values and
+// keys with fewer instructions.  The group's maximum g of a series is taken
+// over all F positions (NaN never wins, as the scan's '>' never takes it),
+// without masking the ones that are no lag (the circular wrap, about 0, below
+// any real maximum); then the first key holding g is found: in one-wave
+// groups by wave_first_key, else by one compare and select per row (each
+// lane keeps its first row in key order that holds g) and a group minimum,
+// where a search would run to the slowest of the groups in a wave or of the
+// waves in a group.  If no lag holds g (rare: every lag below some wrap
+// position), the group takes the masked scan.  Groups wider than a wave
+// exchange maxima and keys through `red` (32 words; its two halves and the
+// transform's own barriers keep the accesses of consecutive calls apart).
+// Measured with the other form at each width: inside a fit at F = 1024 the
+// select took k_assign_prune from 424 to 504 us (n=100000 m=512 k=16); at
+// F = 256 it took the standalone kernel from 1.10 to 0.91 ms (n=200000 m=96
+// k=32), at F = 2048 all distances of n=8000 m=1000 k=20 take 282 us against
+// 290 with the search and 364 with the scan.
+template <int F, int L, int P>
+__device__ __forceinline__ void lag_max(const float2 (&z)[P], int rev, int lane, int m, float* red,
+                                        float& va, int& ka, float& vb, int& kb) {
+  constexpr int W = L < kWave ? L : kWave, NW = L / W;
+  static_assert(2 * NW <= 16, "exchange words");
   int* ir = reinterpret_cast<int*>(red);
-  auto is_lag = [&](int s) {
-    const int tau = glane + L * s;
-    return tau <= m - 1 || tau >= F - m + 1;
-  };
-  // the group maxima of the two series from per-lane maxima
-  auto group_max = [&](float mx, float my, float& gx, float& gy) {
-    const float wx = wave_max(mx), wy = wave_max(my);
-    __syncthreads();  // earlier users of red are done
-    if (lane == 0) {
-      ir[w] = f32_ord(wx);
-      ir[NW + w] = f32_ord(wy);
-    }
-    __syncthreads();
-    int ax = ir[0], ay = ir[NW];
-#pragma unroll
-    for (int u = 1; u < NW; ++u) {
-      ax = max(ax, ir[u]);
-      ay = max(ay, ir[NW + u]);
-    }
-    gx = ord_f32(ax);
-    gy = ord_f32(ay);
-  };
-  // this wave's first lag key holding g (INT_MAX if none)
-  auto find = [&](float g, bool isx) -> int {
-    if (!(g > -INFINITY)) return 0x7fffffff;
-    auto row = [&](int s, int& key) -> bool {
-      uint64_t b = __ballot((isx ? z[s].x : z[s].y) == g);
-      if (!b) return false;
-      b &= __ballot(is_lag(s));
-      if (!b) return false;
-      const int ln = rev ? 63 - __builtin_clzll(b) : __builtin_ctzll(b);
-      key = lag_key(ln + kWave * w + L * s, m, F, rev);
-      return true;
-    };
-    int key = 0x7fffffff;
-    if (!rev) {
-#pragma unroll
-      for (int s = P / 2; s < P; ++s)
-        if (row(s, key)) return key;
-#pragma unroll
-      for (int s = 0; s < P / 2; ++s)
-        if (row(s, key)) return key;
-    } else {
-#pragma unroll
-      for (int s = P / 2 - 1; s >= 0; --s)
-        if (row(s, key)) return key;
-#pragma unroll
-      for (int s = P - 1; s >= P / 2; --s)
-        if (row(s, key)) return key;
-    }
-    return key;
-  };
-  // the smallest of the waves' keys
-  auto group_min_keys = [&](int kx, int ky, int& ox, int& oy) {
-    __syncthreads();
-    if (lane == 0) {
-      ir[w] = kx;
-      ir[NW + w] = ky;
-    }
-    __syncthreads();
-    int ax = ir[0], ay = ir[NW];
-#pragma unroll
-    for (int u = 1; u < NW; ++u) {
-      ax = min(ax, ir[u]);
-      ay = min(ay, ir[NW + u]);
-    }
-    ox = ax;
-    oy = ay;
-  };
+  const int w = lane / W;
   float mx = -INFINITY, my = -INFINITY;
 #pragma unroll
   for (int s = 0; s < P; ++s) {
     mx = fmaxf(mx, z[s].x);
     my = fmaxf(my, z[s].y);
   }
-  group_max(mx, my, va, vb);
-  group_min_keys(find(va, true), find(vb, false), ka, kb);
-  const bool miss_a = va > -INFINITY && ka == 0x7fffffff;
-  const bool miss_b = vb > -INFINITY && kb == 0x7fffffff;
-  if (miss_a || miss_b) {  // uniform: the maximum over the lags alone
-    mx = -INFINITY;
-    my = -INFINITY;
-#pragma unroll
-    for (int s = 0; s < P; ++s) {
-      const bool ok = is_lag(s);
-      mx = ok ? fmaxf(mx, z[s].x) : mx;
-      my = ok ? fmaxf(my, z[s].y) : my;
+  int gx = group_ext_i32<W, true>(f32_ord(mx)), gy = group_ext_i32<W, true>(f32_ord(my));
+  if constexpr (NW > 1) {
+    if (lane % W == 0) {
+      ir[w] = gx;
+      ir[NW + w] = gy;
     }
-    group_max(mx, my, va, vb);
-    group_min_keys(find(va, true), find(vb, false), ka, kb);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < NW; ++u) {
+      gx = max(gx, ir[u]);
+      gy = max(gy, ir[NW + u]);
+    }
+  }
+  va = ord_f32(gx);
+  vb = ord_f32(gy);
+  const int mo = opaque(m);
+  if constexpr (L == kWave) {
+    ka = wave_first_key<P>(z, true, va, rev, mo, F);
+    kb = wave_first_key<P>(z, false, vb, rev, mo, F);
+    if (ka == 0x7fffffff && va > -INFINITY) ka = -1;
+    if (kb == 0x7fffffff && vb > -INFINITY) kb = -1;
+  } else {
+    // rows in falling key order, so the last match is the first in key order
+    int sx = -1, sy = -1;
+    auto visit = [&](int s) {
+      sx = z[s].x == va ? s : sx;
+      sy = z[s].y == vb ? s : sy;
+    };
+    if (!rev) {
+#pragma unroll
+      for (int s = P / 2 - 1; s >= 0; --s) visit(s);
+#pragma unroll
+      for (int s = P - 1; s >= P / 2; --s) visit(s);
+    } else {
+#pragma unroll
+      for (int s = P / 2; s < P; ++s) visit(s);
+#pragma unroll
+      for (int s = 0; s < P / 2; ++s) visit(s);
+    }
+    // a row that is no lag gives key -1
+    auto key = [&](int s, float g) {
+      return s >= 0 && g > -INFINITY ? lag_key(lane + L * s, m, F, rev) : 0x7fffffff;
+    };
+    ka = group_ext_i32<W, false>(key(sx, va));
+    kb = group_ext_i32<W, false>(key(sy, vb));
+    if constexpr (NW > 1) {
+      if (lane % W == 0) {
+        ir[16 + w] = ka;
+        ir[16 + NW + w] = kb;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < NW; ++u) {
+        ka = min(ka, ir[16 + u]);
+        kb = min(kb, ir[16 + NW + u]);
+      }
+    }
+  }
+  if (__any(ka < 0 || kb < 0)) {  // the same in every wave of a wide group
+    int s_lo, s_hi;
+    lag_rows(lane, L, mo, F, s_lo, s_hi);
+    lag_argmax2<L, P>(z, s_lo, s_hi, rev, lane, mo, F, va, ka, vb, kb);
+    group_argmax<L>(va, ka, red);
+    group_argmax<L>(vb, kb, red);
   }
 }
 
