@@ -381,17 +381,48 @@ __host__ __device__ constexpr int tw_offset(int F, int P, int Ns) {
 // shared by every block through L1 and L2), so that the LDS of a block is
 // little more than its exchange buffer: 19 instead of 33 KB at F = 2048, 36
 // instead of 67 KB at 4096, 70 instead of 132 KB at 8192, i.e. twice the
-// blocks per CU.
+// blocks per CU.  The entries are loaded ahead of the exchange before their
+// pass; read in the pass, their latency cost as much as the occupancy gave
+// (assign n=1024 m=1000 k=24: 138 us from LDS, 184 read in the pass, 128
+// loaded ahead; n=8192 m=3000 k=64: 5.69 ms from LDS, 3.2 ms now).
 constexpr int kTwLdsMaxNs = 16;
 template <int F>
 constexpr int fft_tw_lds() {
   return F <= 1024 ? F : tw_offset(F, F / fft_lanes(F), kTwLdsMaxNs * 16);
 }
 
+// Whether the pass with stride Ns reads its twiddles from LDS.
+template <int F, int L, int Ns>
+constexpr bool tw_in_lds() {
+  constexpr int P = F / L, R = (F / Ns < P) ? F / Ns : P;
+  return tw_offset(F, P, Ns) + (R - 1) * Ns <= fft_tw_lds<F>();
+}
+
+// This lane's twiddles of the pass with stride Ns from the global table: its
+// P / R butterflies' R - 1 factors, butterfly by butterfly.  The offset goes
+// through an empty asm, so that they are read for each transform and not held
+// in registers across transforms.
+template <int F, int L, int Ns>
+__device__ __forceinline__ void load_twiddles(const float2* __restrict__ twg, int lane,
+                                              float2 (&w)[F / L]) {
+  constexpr int P = F / L, R = (F / Ns < P) ? F / Ns : P, NB = P / R;
+  const float2* t = twg + opaque(tw_offset(F, P, Ns));
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int kk = (lane + L * b) & (Ns - 1);
+#pragma unroll
+    for (int r = 1; r < R; ++r) w[b * (R - 1) + r - 1] = t[(r - 1) * Ns + kk];
+  }
+}
+
+// wg: the pass's twiddles where they come from the global table, loaded by
+// the pass before ahead of its exchange, so that their latency runs beside
+// the exchange's.
 template <int F, int L, bool INV, int Ns>
 __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
                                               const float2* tw,
-                                              const float2* __restrict__ twg, int lane) {
+                                              const float2* __restrict__ twg, int lane,
+                                              float2 (&wg)[F / L]) {
   constexpr int P = F / L;
   constexpr int R = (F / Ns < P) ? F / Ns : P;
   constexpr int NB = P / R;
@@ -423,6 +454,7 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
     }
     if constexpr (L > kWave) __syncthreads();  // reads done before writes
   }
+  float2 wn[P];  // the next pass's
 #pragma unroll
   for (int t = 0; t < NB; ++t) {
     const int j = lane + L * t;
@@ -430,17 +462,27 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
     float2* b = u + t * R;
     if constexpr (!kFirst) {
       constexpr int kOff = tw_offset(F, P, Ns);
-      constexpr bool kLds = kOff + (R - 1) * Ns <= fft_tw_lds<F>();
-      int z = 0;  // opaque: table entries are read per pass, not held in registers
-      if constexpr (!kLds) asm volatile("" : "+s"(z));
 #pragma unroll
       for (int r = 1; r < R; ++r) {
-        const float2 w = kLds ? tw[kOff + (r - 1) * Ns + kk] : twg[z + kOff + (r - 1) * Ns + kk];
+        float2 w;
+        if constexpr (tw_in_lds<F, L, Ns>()) {
+          w = tw[kOff + (r - 1) * Ns + kk];
+        } else {
+          // the empty asms stand where a load would: the compiler orders the
+          // two products of a sum (and so which of them it fuses) by where
+          // their factors are made, and results are to be those of twiddles
+          // read here
+          w = wg[t * (R - 1) + r - 1];
+          asm("" : "+v"(w.x));
+          asm("" : "+v"(w.y));
+        }
         b[r] = INV ? cmulc(b[r], w) : cmul(b[r], w);
       }
     }
     dft<R, INV>(b);
     if constexpr (!kLast) {
+      if constexpr (!tw_in_lds<F, L, Ns * R>())
+        if (t == NB - 1) load_twiddles<F, L, Ns * R>(twg, lane, wn);
       // base + r*Ns: (j-kk)*R is a multiple of Ns*R and kk < Ns, so
       // (base & 31) + ((r*Ns) & 31) < 32 for every r < R (Ns, R powers of
       // two): one padded base plus immediate offsets
@@ -456,7 +498,7 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
   }
   if constexpr (!kLast) {
     group_sync<L>();
-    stockham_pass<F, L, INV, Ns * R>(v, buf, tw, twg, lane);
+    stockham_pass<F, L, INV, Ns * R>(v, buf, tw, twg, lane, wn);
   }
 }
 
@@ -465,7 +507,8 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
 template <int F, int L, bool INV>
 __device__ __forceinline__ void fft(float2 (&v)[F / L], float2* buf, const float2* tw,
                                     const float2* __restrict__ twg, int lane) {
-  stockham_pass<F, L, INV, 1>(v, buf, tw, twg, lane);
+  float2 none[F / L];
+  stockham_pass<F, L, INV, 1>(v, buf, tw, twg, lane, none);
 }
 
 // Lane-group geometry per FFT length: L lanes, P = F/L values per lane.
