@@ -185,11 +185,23 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock) void k_spectra(
 // ASSIGN: per series keep the centroid with the smallest
 //   dist = 1 - (max_lag cc / F) / (|x| |c_j|)       (first argmin)
 // and the lag key of its maximum (first argmax), test_timesC.py:258-260.
+// OWN: the same of one given centroid per series (fixed_label): at most two
+// inverse transforms per pair.
 // NCC: write cc / F / (|x| |y|) for all 2m-1 lags (ncc.cuh:467-517 layout
 // out[x][y][lag]).
+// blockIdx.y is a chunk of kc centroids; with several chunks ASSIGN writes
+// each chunk's result at y * n (k_split_min then takes the first smallest).
+
+// z / d where r = 1 / d: the residual step makes the quotient the division's
+// (Markstein) as long as nothing over- or underflows on the way.
+__device__ __forceinline__ float div_by(float z, float d, float r) {
+  const float q = z * r;
+  return __builtin_fmaf(__builtin_fmaf(-q, d, z), r, q);
+}
+
 template <int F, int MODE>
-__global__ __launch_bounds__(FftGeom<F>::kBlock, MODE == kModeAssign ? FftGeom<F>::kMinWaves : 1) void k_sbd(
-    const float* __restrict__ x, long n, int m, int k,
+__global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWaves) void k_sbd(
+    const float* __restrict__ x, long n, int m, int k, int kc,
     const float2* __restrict__ cspec, const float* __restrict__ cnorm,
     const float2* __restrict__ twg, int rev, int* __restrict__ label,
     float* __restrict__ dist, int* __restrict__ shift, float* __restrict__ dmat,
@@ -206,6 +218,7 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, MODE == kModeAssign ? FftGeom<F
   float2* buf = smem + fft_tw_lds<F>() + g * fft_buf_len<F>();
   const long npairs = (n + 1) / 2;
   const int nlag = 2 * m - 1;
+  const int j0 = blockIdx.y * kc, j1 = j0 + kc < k ? j0 + kc : k;
   for (long pr = (long)blockIdx.x * G::kGroups + g; pr < npairs;
        pr += (long)gridDim.x * G::kGroups) {
     const long ia = 2 * pr, ib = 2 * pr + 1;
@@ -231,10 +244,17 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, MODE == kModeAssign ? FftGeom<F
 
     float bestA = INFINITY, bestB = INFINITY;
     int labA = 0, labB = 0, keyA = 0, keyB = 0;
-    // fixed_label: report the lag for the given centroid instead of the argmin
-    const int fixA = fixed_label ? fixed_label[ia] : -1;
-    const int fixB = (fixed_label && hasb) ? fixed_label[ib] : -1;
-    for (int j = 0; j < k; ++j) {
+    int fixA = -1, fixB = -1, e0 = j0, e1 = j1;
+    if constexpr (MODE == kModeOwn) {  // a label outside [0, k) is left to the caller
+      fixA = fixed_label[ia];
+      fixB = hasb ? fixed_label[ib] : fixA;
+      if (fixA < 0 || fixA >= k) fixA = -1;
+      if (fixB < 0 || fixB >= k) fixB = -1;
+      e0 = fixA >= 0 ? 0 : 1;
+      e1 = fixB >= 0 && fixB != fixA ? 2 : 1;
+    }
+    for (int e = e0; e < e1; ++e) {
+      const int j = MODE == kModeOwn ? (e == 0 ? fixA : fixB) : e;
       const float2* cj = cspec + (long)j * F;
       float2 z[P];
 #pragma unroll
@@ -242,7 +262,7 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, MODE == kModeAssign ? FftGeom<F
       fft<F, L, true>(z, buf, tw, twg, lane);
       const float cn = cnorm[j];
       const float dena = na * cn, denb = nb * cn;
-      if constexpr (MODE == kModeAssign) {
+      if constexpr (MODE != kModeNcc) {
         float va, vb;
         int ka, kb;
         lag_max<F, L, P>(z, rev, lane, m, red, va, ka, vb, kb);
@@ -250,9 +270,9 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, MODE == kModeAssign ? FftGeom<F
         float da = 1.f, db = 1.f;
         if (dena != 0.f) da = 1.f - (va / (float)F) / dena; else ka = 0;
         if (denb != 0.f) db = 1.f - (vb / (float)F) / denb; else kb = 0;
-        if (fixed_label ? (j == fixA) : (da < bestA)) { bestA = da; labA = j; keyA = ka; }
-        if (fixed_label ? (j == fixB) : (db < bestB)) { bestB = db; labB = j; keyB = kb; }
-        if (dmat && lane == 0) {
+        if (MODE == kModeOwn ? (j == fixA) : (da < bestA)) { bestA = da; labA = j; keyA = ka; }
+        if (MODE == kModeOwn ? (j == fixB) : (db < bestB)) { bestB = db; labB = j; keyB = kb; }
+        if (MODE == kModeAssign && dmat && lane == 0) {
           dmat[ia * k + j] = da;
           if (hasb) dmat[ib * k + j] = db;
         }
@@ -261,31 +281,67 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, MODE == kModeAssign ? FftGeom<F
         const float dA = dena != 0.f ? dena : 1.f, dB = denb != 0.f ? denb : 1.f;
         float* oa = ncc_out + (ia * (long)k + j) * nlag;
         float* ob = ncc_out + (ib * (long)k + j) * nlag;
+        const int mo = opaque(m);
+        auto write = [&](auto quot) {
 #pragma unroll
-        for (int s = 0; s < P; ++s) {
-          int key = lag_key(lane + L * s, m, F, 0);
-          if (key >= 0) {
-            oa[key] = sca * ((z[s].x / (float)F) / dA);
-            if (hasb) ob[key] = scb * ((z[s].y / (float)F) / dB);
+          for (int s = 0; s < P; ++s) {
+            const int key = lag_key(lane + L * s, mo, F, 0);
+            if (key >= 0) {
+              oa[key] = sca * quot(z[s].x / (float)F, 0);
+              if (hasb) ob[key] = scb * quot(z[s].y / (float)F, 1);
+            }
           }
+        };
+        // z / F is at most about the denominator, so in this range of it
+        // nothing over- or underflows but quotients below 2^-76
+        if (fminf(dA, dB) > 0x1p-50f && fmaxf(dA, dB) < 0x1p50f) {
+          const float rA = 1.f / dA, rB = 1.f / dB;
+          write([&](float v, int b) { return b ? div_by(v, dB, rB) : div_by(v, dA, rA); });
+        } else {
+          write([&](float v, int b) { return v / (b ? dB : dA); });
         }
       }
     }
-    if constexpr (MODE == kModeAssign) {
+    if constexpr (MODE != kModeNcc) {
       if (lane == 0) {
+        const long o = (long)blockIdx.y * n;
         if (changed && label[ia] != labA) *changed = 1;
-        label[ia] = labA;
-        if (dist) dist[ia] = bestA;
-        if (shift) shift[ia] = keyA + 1 - m;
+        if (label) label[o + ia] = labA;
+        if (dist) dist[o + ia] = bestA;
+        if (shift) shift[o + ia] = keyA + 1 - m;
         if (hasb) {
           if (changed && label[ib] != labB) *changed = 1;
-          label[ib] = labB;
-          if (dist) dist[ib] = bestB;
-          if (shift) shift[ib] = keyB + 1 - m;
+          if (label) label[o + ib] = labB;
+          if (dist) dist[o + ib] = bestB;
+          if (shift) shift[o + ib] = keyB + 1 - m;
         }
       }
     }
   }
+}
+
+// The chunk results [chunks][n] of k_sbd to one: the first smallest distance
+// in chunk order, as one pass over all centroids keeps it.
+__global__ __launch_bounds__(256) void k_split_min(
+    const float* __restrict__ pdist, const int* __restrict__ plabel,
+    const int* __restrict__ pshift, long n, int m, int chunks, int* __restrict__ label,
+    float* __restrict__ dist, int* __restrict__ shift) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  float best = INFINITY;
+  int lab = 0, sh = 1 - m;
+  for (int c = 0; c < chunks; ++c) {
+    const float d = pdist[c * n + i];
+    const int l = plabel[c * n + i], s = pshift[c * n + i];
+    if (d < best) {
+      best = d;
+      lab = l;
+      sh = s;
+    }
+  }
+  label[i] = lab;
+  if (dist) dist[i] = best;
+  if (shift) shift[i] = sh;
 }
 
 // The first N (<= P) magnitudes of a lane from its lane-major row segment
@@ -967,6 +1023,20 @@ static hipError_t launch_spectra_F(const float* y, int rows, int m, const float2
   return hipGetLastError();
 }
 
+// Chunks of centroids (blockIdx.y) that fill the device when the pairs alone
+// do not: as many as keep at most three waves per SIMD busy.
+template <int F>
+static int sbd_chunks_F(long npairs, int k, int cus) {
+  using G = FftGeom<F>;
+  const long blocks = (npairs + G::kGroups - 1) / G::kGroups;
+  const long waves = blocks * (G::kBlock / kWave);
+  long c = 12L * cus / (waves > 0 ? waves : 1);
+  if (c > k) c = k;
+  if (c < 2) return 1;
+  const long kc = (k + c - 1) / c;
+  return (int)((k + kc - 1) / kc);
+}
+
 template <int F, int MODE>
 static hipError_t launch_sbd_F(const SbdArgs& a, hipStream_t st) {
   using G = FftGeom<F>;
@@ -974,9 +1044,21 @@ static hipError_t launch_sbd_F(const SbdArgs& a, hipStream_t st) {
   long blocks = (npairs + G::kGroups - 1) / G::kGroups;
   if (blocks < 1) blocks = 1;
   if (blocks > 8192) blocks = 8192;
-  hipLaunchKernelGGL((k_sbd<F, MODE>), dim3((unsigned)blocks), dim3(G::kBlock),
-                     sbd_smem<F>(), st, a.x, a.n, a.m, a.k, a.cspec, a.cnorm, a.tw, a.rev,
-                     a.label, a.dist, a.shift, a.dmat, a.changed, a.ncc_out, a.fixed_label);
+  const bool split = MODE == kModeAssign && a.chunks > 1;
+  if (split && a.changed) return hipErrorInvalidValue;
+  const int chunks = MODE == kModeOwn || a.chunks < 1 ? 1 : a.chunks;
+  if (split && (!a.part_dist || !a.part_label || !a.part_shift)) return hipErrorInvalidValue;
+  const int kc = (a.k + chunks - 1) / chunks;
+  hipLaunchKernelGGL((k_sbd<F, MODE>), dim3((unsigned)blocks, (unsigned)chunks), dim3(G::kBlock),
+                     sbd_smem<F>(), st, a.x, a.n, a.m, a.k, kc, a.cspec, a.cnorm, a.tw, a.rev,
+                     split ? a.part_label : a.label, split ? a.part_dist : a.dist,
+                     split ? a.part_shift : a.shift, a.dmat, split ? nullptr : a.changed,
+                     a.ncc_out, a.fixed_label);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !split) return e;
+  hipLaunchKernelGGL(k_split_min, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, st,
+                     a.part_dist, a.part_label, a.part_shift, a.n, a.m, chunks, a.label, a.dist,
+                     a.shift);
   return hipGetLastError();
 }
 
@@ -1135,14 +1217,27 @@ hipError_t launch_assign_prune(int F, const PruneArgs& a, hipStream_t st) {
 
 hipError_t launch_sbd(int F, int mode, const SbdArgs& a, hipStream_t st) {
   switch (F) {
-#define X(FF)                                                     \
-  case FF:                                                        \
-    return mode == kModeAssign ? launch_sbd_F<FF, kModeAssign>(a, st) \
+#define X(FF)                                                          \
+  case FF:                                                             \
+    return mode == kModeAssign ? launch_sbd_F<FF, kModeAssign>(a, st)   \
+           : mode == kModeOwn  ? launch_sbd_F<FF, kModeOwn>(a, st)      \
                                : launch_sbd_F<FF, kModeNcc>(a, st);
     TCX_FOR_EACH_F(X)
 #undef X
     default:
       return hipErrorInvalidValue;
+  }
+}
+
+int sbd_chunks(int F, long n, int k, int cus) {
+  switch (F) {
+#define X(FF) \
+  case FF:    \
+    return sbd_chunks_F<FF>((n + 1) / 2, k, cus);
+    TCX_FOR_EACH_F(X)
+#undef X
+    default:
+      return 1;
   }
 }
 
@@ -1155,6 +1250,9 @@ hipError_t configure_sbd_kernels() {
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
   if (e == hipSuccess)                                                                        \
     e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeNcc>,                                 \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
+  if (e == hipSuccess)                                                                        \
+    e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeOwn>,                                 \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
   if (e == hipSuccess)                                                                        \
     e = hipFuncSetAttribute((const void*)k_spectra<FF>,                                       \

@@ -54,7 +54,7 @@ enum Slot {
   kSlotS, kSlotInfo, kSlotDummy, kSlotWbuf, kSlotRbuf, kSlotBar, kSlotVout, kSlotSteps,
   kSlotConv, kSlotErr, kSlotCmag, kSlotEvals, kSlotSvout, kSlotLzW, kSlotLzState, kSlotMask,
   kSlotRowStats, kSlotFitRowStats, kSlotKeyCounts, kSlotKeyOff, kSlotMinRow, kSlotXs, kSlotXn,
-  kSlotLzXch, kSlotXm, kSlotUb, kSlotCm, kSlotCheck, kSlotCheckInfo, kNumSlots
+  kSlotLzXch, kSlotXm, kSlotUb, kSlotCm, kSlotCheck, kSlotCheckInfo, kSlotSplit, kNumSlots
 };
 
 struct FitState {
@@ -228,6 +228,10 @@ int spectra(tcx_ctx* c, const float* d_rows, int rows, int m, float2** spec, flo
   return TCX_OK;
 }
 
+// Chunks from which tcx_assign without distances splits the centroids of few
+// series over the grid instead of pruning.
+constexpr int kSplitMinChunks = 4;
+
 // Assignment with the twiddle table tw of F = fft_size(m) and the
 // centroid magnitudes cmag given.  Without a distance matrix the exact
 // pruned kernel runs, pairing the rows of `order` (npairs pairs, -1 = hole)
@@ -237,9 +241,30 @@ int assign_core_tw(tcx_ctx* c, const float2* tw, const float* d_x, long n, int m
                    float* dist, int* shift, float* dmat, int* changed,
                    const int* order = nullptr, long npairs = 0,
                    unsigned long long* evals = nullptr, const float2* xs = nullptr,
-                   const float* xn = nullptr, const float* ub = nullptr, int ub_ld = 0) {
+                   const float* xn = nullptr, const float* ub = nullptr, int ub_ld = 0,
+                   bool may_split = false) {
   const int F = fft_size(m);
-  if (!dmat && k <= tcx::prune_max_k(F)) {
+  int chunks = 1;
+  float* part = nullptr;
+  if (may_split && !changed && !order && !xs) {
+    // few series: their centroids in chunks over the grid, each chunk
+    // searched in full.  With all distances asked for, as soon as it fills
+    // the device better; else from kSplitMinChunks on, since the pruned
+    // search of a pair skips half of its transforms or more, one after
+    // another (n=256 m=256 k=24: 35 us split, 127 pruned; n=4096 m=500 k=24,
+    // where two chunks would fit: 154 pruned).  With well separated classes
+    // (noise 0.05, most of the search pruned) the smallest gain measured at
+    // the line is 49 against 262 us (n=2048 m=128 k=64).  Not when the budget
+    // has no room for the chunk results.
+    chunks = tcx::sbd_chunks(F, n, k, c->cus);
+    if (!dmat && chunks < kSplitMinChunks) chunks = 1;
+    const size_t bytes = ((size_t)chunks * n * 3 * sizeof(float) + 255) & ~(size_t)255;
+    if (chunks > 1 && c->slot_bytes[kSlotSplit] < bytes && c->budget &&
+        c->ws_bytes + c->user_bytes + bytes > c->budget)
+      chunks = 1;
+    if (chunks > 1) TCX_TRY(ws(c, kSlotSplit, (size_t)chunks * n * 3, &part));
+  }
+  if (!dmat && chunks == 1 && k <= tcx::prune_max_k(F)) {
     tcx::PruneArgs p;
     p.x = d_x; p.n = n; p.m = m; p.k = k; p.cspec = cspec; p.cnorm = cnorm; p.tw = tw;
     p.cmag = cmag;
@@ -258,6 +283,12 @@ int assign_core_tw(tcx_ctx* c, const float2* tw, const float* d_x, long n, int m
   a.x = d_x; a.n = n; a.m = m; a.k = k; a.cspec = cspec; a.cnorm = cnorm; a.tw = tw;
   a.rev = rev; a.label = label; a.dist = dist; a.shift = shift; a.dmat = dmat;
   a.changed = changed;
+  a.chunks = chunks;
+  if (part) {
+    a.part_dist = part;
+    a.part_label = reinterpret_cast<int*>(part + (size_t)chunks * n);
+    a.part_shift = a.part_label + (size_t)chunks * n;
+  }
   TCX_HIP(tcx::launch_sbd(F, tcx::kModeAssign, a, c->stream));
   return TCX_OK;
 }
@@ -269,12 +300,12 @@ int assign_core(tcx_ctx* c, const float* d_x, long n, int m, int k, const float2
                 int* changed, const int* order = nullptr, long npairs = 0,
                 unsigned long long* evals = nullptr, const float* cmag = nullptr,
                 const float2* xs = nullptr, const float* xn = nullptr,
-                const float* ub = nullptr, int ub_ld = 0) {
+                const float* ub = nullptr, int ub_ld = 0, bool may_split = false) {
   const float2* tw;
   TCX_TRY(twiddles(c, fft_size(m), &tw));
   if (!cmag) cmag = reinterpret_cast<const float*>(c->slot_ptr[kSlotCmag]);
   return assign_core_tw(c, tw, d_x, n, m, k, cspec, cnorm, cmag, rev, label, dist, shift, dmat,
-                        changed, order, npairs, evals, xs, xn, ub, ub_ld);
+                        changed, order, npairs, evals, xs, xn, ub, ub_ld, may_split);
 }
 
 // ------------------------------------------------ allocation-free assignment
@@ -1030,6 +1061,7 @@ int tcx_ncc(tcx_ctx* c, const float* d_x, const float* d_y, float* d_out, int x_
   tcx::SbdArgs a;
   a.x = d_x; a.n = x_rows; a.m = cols; a.k = y_rows; a.cspec = spec; a.cnorm = norm;
   a.tw = tw; a.ncc_out = d_out;
+  a.chunks = tcx::sbd_chunks(F, x_rows, y_rows, c->cus);
   TCX_HIP(tcx::launch_sbd(F, tcx::kModeNcc, a, c->stream));
   TCX_HIP(hipStreamSynchronize(c->stream));
   return TCX_OK;
@@ -1064,7 +1096,8 @@ int tcx_assign(tcx_ctx* c, const float* d_x, const float* d_centroids, int n, in
   float* norm;
   int* zero;
   TCX_TRY(spectra(c, d_centroids, k, m, &spec, &norm, &zero));
-  TCX_TRY(assign_core(c, d_x, n, m, k, spec, norm, 0, d_label, d_dist, d_shift, d_dmat, nullptr));
+  TCX_TRY(assign_core(c, d_x, n, m, k, spec, norm, 0, d_label, d_dist, d_shift, d_dmat, nullptr,
+                      nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr, 0, true));
   TCX_HIP(hipStreamSynchronize(c->stream));
   return TCX_OK;
 }
@@ -1111,16 +1144,15 @@ int tcx_extract_shape(tcx_ctx* c, const int* d_label, const float* d_x, const in
   TCX_TRY(spectra(c, d_centroids, k, m, &spec, &norm, &zero));  // old-centroid zero flags
   if (!d_shift) {
     // shift of each series against its own cluster's old centroid
-    int *lab, *sh;
-    TCX_TRY(ws(c, kSlotDummy, (size_t)n, &lab));
+    int* sh;
     TCX_TRY(ws(c, kSlotShift, (size_t)n, &sh));
     int F = fft_size(m);
     const float2* tw;
     TCX_TRY(twiddles(c, F, &tw));
     tcx::SbdArgs a;
     a.x = d_x; a.n = n; a.m = m; a.k = k; a.cspec = spec; a.cnorm = norm; a.tw = tw;
-    a.label = lab; a.shift = sh; a.fixed_label = d_label;
-    TCX_HIP(tcx::launch_sbd(F, tcx::kModeAssign, a, c->stream));
+    a.shift = sh; a.fixed_label = d_label;
+    TCX_HIP(tcx::launch_sbd(F, tcx::kModeOwn, a, c->stream));
     d_shift = sh;
   }
   float* cnew;

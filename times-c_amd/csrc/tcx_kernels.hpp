@@ -7,6 +7,7 @@ namespace tcx {
 
 constexpr int kModeAssign = 0;
 constexpr int kModeNcc = 1;
+constexpr int kModeOwn = 2;
 
 struct SbdArgs {
   const float* x = nullptr;      // [n][m] series
@@ -17,13 +18,19 @@ struct SbdArgs {
   const float* cnorm = nullptr;  // [k]
   const float2* tw = nullptr;    // [F] exp(-2 pi i q / F)
   int rev = 0;                   // 1: k-Shape lag order
-  int* label = nullptr;
+  int* label = nullptr;          // required (assign), may be NULL (own)
   float* dist = nullptr;
   int* shift = nullptr;
   float* dmat = nullptr;
   int* changed = nullptr;
   float* ncc_out = nullptr;
-  const int* fixed_label = nullptr;  // shift against this centroid, no argmin
+  const int* fixed_label = nullptr;  // own: the centroid of each series
+  // centroids split into this many chunks over the grid (sbd_chunks); assign
+  // with more than one also needs the chunk results, [chunks][n] each
+  int chunks = 1;
+  float* part_dist = nullptr;
+  int* part_label = nullptr;
+  int* part_shift = nullptr;
 };
 
 // largest supported FFT length (m <= 4096)
@@ -93,6 +100,8 @@ hipError_t launch_series_spec(int F, const float* x, long n, int m, const float2
 hipError_t launch_bounds(int F, const uint16_t* xm, long n, const uint16_t* cm, int k, float* ub,
                          int ld, hipStream_t st);
 hipError_t launch_sbd(int F, int mode, const SbdArgs& a, hipStream_t st);
+// Chunks the centroids of n series are worth splitting into (1: none).
+int sbd_chunks(int F, long n, int k, int cus);
 hipError_t launch_apply_shift(float* x, long rows, int m, const int* shift, const int* skip,
                               hipStream_t st);
 hipError_t configure_sbd_kernels();
