@@ -358,13 +358,14 @@ int setup_jobs(Batch& b, const std::vector<GJob*>& fresh) {
   long fill_max = 0;
   for (GJob* j : fresh) {
     if (j->job->znorm_ddof >= 0) {
-      const int nv = znorm_vectors(j->job->d_x, j->m);
-      zn.at(nv).add(ZnormJob{j->job->d_x, j->n, j->m, j->job->znorm_ddof}, znorm_blocks(j->n));
+      const int form = znorm_form(j->job->d_x, j->m);
+      zn.at(form).add(ZnormJob{j->job->d_x, j->n, j->m, j->job->znorm_ddof},
+                      znorm_blocks(form, j->n));
     }
     ss.at(j->F).add(SeriesSpecJob{j->job->d_x, j->n, j->m, j->xs, j->xn, j->xm},
                     series_spec_blocks(j->F, j->n));
     if (j->row_stats)
-      rs.add(RowStatsJob{j->job->d_x, j->n, j->m, j->row_stats}, znorm_blocks(j->n));
+      rs.add(RowStatsJob{j->job->d_x, j->n, j->m, j->row_stats}, row_stats_blocks(j->n));
     fills.add(FillSeg{reinterpret_cast<int*>(j->cent), (long)j->k * j->m, 0}, 1);
     fills.add(FillSeg{j->shift, j->n, 0}, 1);
     fills.add(FillSeg{j->zero, j->k, 1}, 1);  // the initial centroids are zero

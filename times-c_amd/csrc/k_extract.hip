@@ -2768,9 +2768,11 @@ hipError_t launch_group_place(const int* label, long n, int k, const float* dist
   return hipGetLastError();
 }
 
+long row_stats_blocks(long rows) { return (rows + 3) / 4; }
+
 hipError_t launch_row_stats(const float* x, long rows, int m, double2* stats, hipStream_t st) {
   if (rows <= 0) return hipSuccess;
-  const long blocks = (rows + 3) / 4;
+  const long blocks = row_stats_blocks(rows);
   hipLaunchKernelGGL(k_row_stats, dim3((unsigned)blocks), dim3(256), 0, st, x, rows, m, stats);
   return hipGetLastError();
 }

@@ -1,6 +1,6 @@
 // SBD kernels: z-normalization, centroid spectra, the fused
 // FFT -> conj-multiply -> inverse FFT -> max-over-lags -> argmin assignment,
-// the materialized NCC and the zero-fill shift.
+// the materialized NCC and the alignment.
 //
 // Layout: series are rows of a row-major FP32 [n][m] matrix.  A spectrum is
 // F complex values stored lane-strided ([s][lane], s < P, lane < L) so that
@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "tcx_device.hpp"
 #include "tcx_internal.hpp"
@@ -56,57 +57,90 @@ __global__ __launch_bounds__(256) void k_znorm(float* __restrict__ x, long rows,
   znorm_body(blockIdx.x, gridDim.x, x, rows, m, ddof);
 }
 
-// The same for m % 4 == 0, m <= 256 * NV: the row is read once, as float4
-// vectors held in registers (lane l holds vectors l, l + 64, ...), and
-// written once; the sums are the same two-pass FP64 sums (in another
-// order).
-template <int NV>
+// (v - mean) / sd of a row as a float: the residual step makes q the
+// division's quotient (Markstein) where the row's sd is in a range in which
+// nothing over- or underflows and nothing is NaN (kFast); else the division
+// with nan_to_num.
+template <bool kFast>
+__device__ __forceinline__ float znorm_value(float v, double mean, double sd, double rsd) {
+  const double d = (double)v - mean;
+  if constexpr (kFast) {
+    const double q = d * rsd;
+    return (float)__builtin_fma(__builtin_fma(-q, sd, d), rsd, q);
+  }
+  const double w = d / sd;
+  return isnan(w) ? 0.f : (isinf(w) ? (w > 0 ? 3.402823466e38f : -3.402823466e38f) : (float)w);
+}
+
+// The same with the row read once into registers, for m <= 4 G NV: lane l of
+// the row's G lanes holds the 16-byte vectors l, l + G, ... and one of the m %
+// 4 values after the last (kTail: rows that start at any float; without it
+// the rows are whole aligned vectors); the sums are the same two-pass FP64
+// sums in another order.  HBM bound; 16 lanes per row up to m = 128, where a
+// wave per row leaves most of its lanes idle.  Times of a call (14 us of it
+// the launch and the wait), before: rows that are no whole aligned vectors in
+// three passes, a wave per row, the division: n=60000 m=365 65 -> 40 us, n=
+// 30000 m=1001 91 -> 48 us (5.0 TB/s), n=100000 m=128 55 -> 28 us, m=37 43 ->
+// 24 us.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef f32x4 f32x4_u __attribute__((aligned(4)));
+template <int G, bool kTail, int NV>
 __device__ __forceinline__ void znorm_v_body(const int bid, const int nblk,
-    float* __restrict__ x, long rows, int m,
-                                                 int ddof) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const long row = (long)bid * 4 + (threadIdx.x >> 6);
+    float* __restrict__ x, long rows, int m, int ddof) {
+  using vec = std::conditional_t<kTail, f32x4_u, f32x4>;
+  const int lane = threadIdx.x & (G - 1);
+  const long row = (long)bid * (256 / G) + threadIdx.x / G;
   if (row >= rows) return;
-  float4* r = reinterpret_cast<float4*>(x + row * (long)m);
-  const int nv = m >> 2;
-  float4 v[NV];
+  float* r = x + row * (long)m;
+  vec* rv = reinterpret_cast<vec*>(r);
+  const int nv = m >> 2, tail = kTail ? m & 3 : 0;
+  f32x4 v[NV];
 #pragma unroll
   for (int u = 0; u < NV; ++u) {
-    const int i = lane + kWave * u;
-    v[u] = i < nv ? r[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const int i = lane + G * u;
+    v[u] = i < nv ? rv[i] : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  double s = 0.0;
+  float vt = 0.f;
+  if (kTail && lane < tail) vt = r[4 * nv + lane];
+  auto sum = [](double t) { return G == kWave ? wave_sum_f64(t) : row16_sum_f64(t); };
+  double s = (double)vt;
 #pragma unroll
   for (int u = 0; u < NV; ++u)
     s += ((double)v[u].x + (double)v[u].y) + ((double)v[u].z + (double)v[u].w);
-  s = wave_sum_f64(s);
+  s = sum(s);
   const double mean = s / (double)m;
   double ss = 0.0;
+  if (kTail && lane < tail) ss = ((double)vt - mean) * ((double)vt - mean);
 #pragma unroll
   for (int u = 0; u < NV; ++u) {
-    if (lane + kWave * u < nv) {
+    if (lane + G * u < nv) {
       const double a = (double)v[u].x - mean, b = (double)v[u].y - mean;
       const double c = (double)v[u].z - mean, d = (double)v[u].w - mean;
       ss += (a * a + b * b) + (c * c + d * d);
     }
   }
-  ss = wave_sum_f64(ss);
+  ss = sum(ss);
   const double sd = sqrt(ss / (double)(m - ddof));
-  auto z = [&](float e) {
-    const double w = ((double)e - mean) / sd;
-    return isnan(w) ? 0.f : (isinf(w) ? (w > 0 ? 3.402823466e38f : -3.402823466e38f) : (float)w);
-  };
+  const double rsd = 1.0 / sd;
+  auto write = [&](auto fast) {
+    auto z = [&](float e) { return znorm_value<decltype(fast)::value>(e, mean, sd, rsd); };
 #pragma unroll
-  for (int u = 0; u < NV; ++u) {
-    const int i = lane + kWave * u;
-    if (i < nv) r[i] = make_float4(z(v[u].x), z(v[u].y), z(v[u].z), z(v[u].w));
-  }
+    for (int u = 0; u < NV; ++u) {
+      const int i = lane + G * u;
+      if (i < nv) rv[i] = f32x4{z(v[u].x), z(v[u].y), z(v[u].z), z(v[u].w)};
+    }
+    if (kTail && lane < tail) r[4 * nv + lane] = z(vt);
+  };
+  if (__all(sd > 1e-100 && sd < 1e100))  // over the wave's rows; false for NaN
+    write(std::true_type{});
+  else
+    write(std::false_type{});
 }
 
-template <int NV>
+template <int G, bool kTail, int NV>
 __global__ __launch_bounds__(256) void k_znorm_v(float* __restrict__ x, long rows, int m,
                                                  int ddof) {
-  znorm_v_body<NV>(blockIdx.x, gridDim.x, x, rows, m, ddof);
+  znorm_v_body<G, kTail, NV>(blockIdx.x, gridDim.x, x, rows, m, ddof);
 }
 
 // ------------------------------------------------------------- spectra
@@ -925,25 +959,77 @@ __global__ __launch_bounds__(PruneGeom<F>::kBlock, PruneGeom<F>::kMinWaves) void
   assign_prune_body<F, kPre>(blockIdx.x, gridDim.x, x, xs, xn, ubg, ub_ld, n, npairs, m, k, cspec, cmag, cnorm, twg, rev, order, label, dist, shift, changed, evals);
 }
 
-// ---------------------------------------------------------- zero-fill shift
-// out[t] = in[t - s] (0 outside), s = shift[row]; skipped when *skip != 0.
-// roll_zeropad, test_timesC.py:55-77.  In place: one block per row, the row
-// is staged in LDS.
-__global__ __launch_bounds__(256) void k_apply_shift(float* __restrict__ x, long rows, int m,
-                                                    const int* __restrict__ shift,
-                                                    const int* __restrict__ skip) {
-  extern __shared__ float row_s[];
-  if (skip && *skip) return;
-  for (long row = blockIdx.x; row < rows; row += gridDim.x) {
-    float* r = x + row * (long)m;
-    for (int t = threadIdx.x; t < m; t += blockDim.x) row_s[t] = r[t];
-    __syncthreads();
-    const int s = shift[row];
-    for (int t = threadIdx.x; t < m; t += blockDim.x) {
-      long src = (long)t - s;
-      r[t] = (src >= 0 && src < m) ? row_s[src] : 0.f;
+// ------------------------------------------------------------- alignment
+// Each series against one centroid, shifted in place by the lag of its
+// largest NCC with zero fill (out[t] = in[t - s], 0 outside; roll_zeropad,
+// test_timesC.py:55-77), nothing for an all-zero centroid: one kernel forms
+// the pair's correlation, its lags (k_sbd's, bit for bit) and the shifted
+// rows, which it reads again from L2.  Bound by the two transforms.  With
+// the shifts through memory, the bounds of a search over one centroid and a
+// second kernel to shift the rows, n=12000 m=700 took 143 us, 95 now.
+template <int F>
+__global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWaves) void k_align(
+    float* x, long n, int m, const float2* __restrict__ cspec, const float* __restrict__ cnorm,
+    const int* __restrict__ czero, const float2* __restrict__ twg, int rev) {
+  using G = FftGeom<F>;
+  constexpr int L = G::L, P = G::P;
+  extern __shared__ float2 smem[];
+  if (*czero) return;
+  float2* tw = smem;
+  float* red = reinterpret_cast<float*>(smem + fft_tw_lds<F>() + G::kGroups * fft_buf_len<F>());
+  for (int i = threadIdx.x; i < fft_tw_lds<F>(); i += blockDim.x) tw[i] = twg[i];
+  __syncthreads();
+  const int g = threadIdx.x / L, lane = threadIdx.x % L;
+  float2* buf = smem + fft_tw_lds<F>() + g * fft_buf_len<F>();
+  const long npairs = (n + 1) / 2;
+  for (long pr = (long)blockIdx.x * G::kGroups + g; pr < npairs;
+       pr += (long)gridDim.x * G::kGroups) {
+    const bool hasb = 2 * pr + 1 < n;
+    float* xa = x + 2 * pr * (long)m;
+    float* xb = hasb ? xa + m : xa;
+    float2 z[P];
+    float sa = 0.f, sb = 0.f;
+    const int ml = opaque(m);
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+      int t = lane + L * s;
+      float a = t < ml ? xa[t] : 0.f;
+      float b = (hasb && t < ml) ? xb[t] : 0.f;
+      z[s] = make_float2(a, b);
+      sa += a * a;
+      sb += b * b;
     }
-    __syncthreads();
+    sa = group_sum<L>(sa, red);
+    sb = group_sum<L>(sb, red);
+    fft<F, L, false>(z, buf, tw, twg, lane);
+#pragma unroll
+    for (int s = 0; s < P; ++s) z[s] = cmulc(z[s], cspec[s * L + lane]);
+    fft<F, L, true>(z, buf, tw, twg, lane);
+    float va, vb;
+    int ka, kb;
+    lag_max<F, L, P>(z, rev, lane, m, red, va, ka, vb, kb);
+    // den == 0: every lag is 0, the argmax is index 0
+    const float cn = cnorm[0];
+    if (sqrtf(sa) * cn == 0.f) ka = 0;
+    if (sqrtf(sb) * cn == 0.f) kb = 0;
+    const int ha = ka + 1 - m, hb = kb + 1 - m;
+    const int mo = opaque(m);
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+      const int pa = lane + L * s - ha, pb = lane + L * s - hb;
+      z[s].x = (unsigned)pa < (unsigned)mo ? xa[pa] : 0.f;
+      z[s].y = (unsigned)pb < (unsigned)mo ? xb[pb] : 0.f;
+    }
+    group_sync<L>();  // both rows read before they are overwritten
+    const int mw = opaque(m);
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+      const int t = lane + L * s;
+      if (t < mw) {
+        xa[t] = z[s].x;
+        if (hasb) xb[t] = z[s].y;
+      }
+    }
   }
 }
 
@@ -961,11 +1047,11 @@ __global__ __launch_bounds__(256) void k_znorm_group(const ZnormJob* __restrict_
   znorm_body(bid, nblk, a.x, a.rows, a.m, a.ddof);
 }
 
-template <int NV>
+template <int G, bool kTail, int NV>
 __global__ __launch_bounds__(256) void k_znorm_v_group(const ZnormJob* __restrict__ jobs,
                                                        const int* __restrict__ first, int njobs) {
   TCX_GROUP_JOB(ZnormJob)
-  znorm_v_body<NV>(bid, nblk, a.x, a.rows, a.m, a.ddof);
+  znorm_v_body<G, kTail, NV>(bid, nblk, a.x, a.rows, a.m, a.ddof);
 }
 
 template <int F>
@@ -1255,6 +1341,9 @@ hipError_t configure_sbd_kernels() {
     e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeOwn>,                                 \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
   if (e == hipSuccess)                                                                        \
+    e = hipFuncSetAttribute((const void*)k_align<FF>,                                         \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
+  if (e == hipSuccess)                                                                        \
     e = hipFuncSetAttribute((const void*)k_spectra<FF>,                                       \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
   if (e == hipSuccess)                                                                        \
@@ -1283,56 +1372,59 @@ hipError_t configure_sbd_kernels() {
   return e;
 }
 
+// The form of a z-norm: 0, three passes over the row (longer than a wave
+// holds); else the vectors a lane holds (1: 16 lanes per row with up to two,
+// for rows of at most 128 values), negative with the tail.
+int znorm_form(const float* x, int m) {
+  if (m > 4096) return 0;
+  int nv = 1;
+  if (m > 128)
+    for (nv = 2; 4 * kWave * nv < m;) nv *= 2;
+  return (m & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 ? nv : -nv;
+}
+
+long znorm_blocks(int form, long rows) {
+  const long per = form == 1 || form == -1 ? 16 : 4;
+  return (rows + per - 1) / per;
+}
+
+#define TCX_FOR_EACH_ZNORM(X)                                                         \
+  X(1, 16, false, 2) X(2, 64, false, 2) X(4, 64, false, 4) X(8, 64, false, 8)         \
+  X(16, 64, false, 16) X(-1, 16, true, 2) X(-2, 64, true, 2) X(-4, 64, true, 4)       \
+  X(-8, 64, true, 8) X(-16, 64, true, 16)
+
 hipError_t launch_znorm(float* x, long rows, int m, int ddof, hipStream_t st) {
   if (rows <= 0) return hipSuccess;
-  long blocks = (rows + 3) / 4;
-  if ((m & 3) == 0 && m <= 256 * 16 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
-    if (m <= 256 * 2)
-      hipLaunchKernelGGL(k_znorm_v<2>, dim3((unsigned)blocks), dim3(256), 0, st, x, rows, m, ddof);
-    else if (m <= 256 * 4)
-      hipLaunchKernelGGL(k_znorm_v<4>, dim3((unsigned)blocks), dim3(256), 0, st, x, rows, m, ddof);
-    else if (m <= 256 * 8)
-      hipLaunchKernelGGL(k_znorm_v<8>, dim3((unsigned)blocks), dim3(256), 0, st, x, rows, m, ddof);
-    else
-      hipLaunchKernelGGL(k_znorm_v<16>, dim3((unsigned)blocks), dim3(256), 0, st, x, rows, m,
-                         ddof);
-    return hipGetLastError();
+  const int form = znorm_form(x, m);
+  const dim3 grid((unsigned)znorm_blocks(form, rows));
+  switch (form) {
+#define X(FORM, G, TAIL, NV)                                                                     \
+  case FORM:                                                                                     \
+    hipLaunchKernelGGL((k_znorm_v<G, TAIL, NV>), grid, dim3(256), 0, st, x, rows, m, ddof);      \
+    break;
+    TCX_FOR_EACH_ZNORM(X)
+#undef X
+    default:
+      hipLaunchKernelGGL(k_znorm, grid, dim3(256), 0, st, x, rows, m, ddof);
   }
-  hipLaunchKernelGGL(k_znorm, dim3((unsigned)blocks), dim3(256), 0, st, x, rows, m, ddof);
   return hipGetLastError();
 }
 
 // ------------------------------------------------ grouped-form launchers
-long znorm_blocks(long rows) { return (rows + 3) / 4; }
-
-int znorm_vectors(const float* x, int m) {
-  if ((m & 3) != 0 || m > 256 * 16 || (reinterpret_cast<uintptr_t>(x) & 15) != 0) return 0;
-  return m <= 256 * 2 ? 2 : (m <= 256 * 4 ? 4 : (m <= 256 * 8 ? 8 : 16));
-}
-
-hipError_t launch_znorm_group(const GroupTable& g, int nv, hipStream_t st) {
+hipError_t launch_znorm_group(const GroupTable& g, int form, hipStream_t st) {
   if (g.blocks <= 0) return hipSuccess;
   const ZnormJob* j = static_cast<const ZnormJob*>(g.jobs);
-  switch (nv) {
+  switch (form) {
     case 0:
       hipLaunchKernelGGL(k_znorm_group, dim3(g.blocks), dim3(256), 0, st, j, g.first, g.njobs);
       break;
-    case 2:
-      hipLaunchKernelGGL(k_znorm_v_group<2>, dim3(g.blocks), dim3(256), 0, st, j, g.first,
-                         g.njobs);
-      break;
-    case 4:
-      hipLaunchKernelGGL(k_znorm_v_group<4>, dim3(g.blocks), dim3(256), 0, st, j, g.first,
-                         g.njobs);
-      break;
-    case 8:
-      hipLaunchKernelGGL(k_znorm_v_group<8>, dim3(g.blocks), dim3(256), 0, st, j, g.first,
-                         g.njobs);
-      break;
-    case 16:
-      hipLaunchKernelGGL(k_znorm_v_group<16>, dim3(g.blocks), dim3(256), 0, st, j, g.first,
-                         g.njobs);
-      break;
+#define X(FORM, G, TAIL, NV)                                                                     \
+  case FORM:                                                                                     \
+    hipLaunchKernelGGL((k_znorm_v_group<G, TAIL, NV>), dim3(g.blocks), dim3(256), 0, st, j,       \
+                       g.first, g.njobs);                                                        \
+    break;
+    TCX_FOR_EACH_ZNORM(X)
+#undef X
     default:
       return hipErrorInvalidValue;
   }
@@ -1495,13 +1587,28 @@ hipError_t launch_assign_prune_group(int F, const GroupTable& g, const float2* t
   return hipGetLastError();
 }
 
-hipError_t launch_apply_shift(float* x, long rows, int m, const int* shift, const int* skip,
-                              hipStream_t st) {
-  if (rows <= 0) return hipSuccess;
-  long blocks = rows < 4096 ? rows : 4096;
-  hipLaunchKernelGGL(k_apply_shift, dim3((unsigned)blocks), dim3(256), sizeof(float) * m, st,
-                     x, rows, m, shift, skip);
+template <int F>
+static hipError_t launch_align_F(float* x, long n, int m, const float2* cspec, const float* cnorm,
+                                 const int* czero, const float2* tw, int rev, hipStream_t st) {
+  using G = FftGeom<F>;
+  const long blocks = std::min(groups_blocks<F>((n + 1) / 2), 8192L);
+  hipLaunchKernelGGL((k_align<F>), dim3((unsigned)blocks), dim3(G::kBlock), sbd_smem<F>(), st, x,
+                     n, m, cspec, cnorm, czero, tw, rev);
   return hipGetLastError();
+}
+
+hipError_t launch_align(int F, float* x, long n, int m, const float2* cspec, const float* cnorm,
+                        const int* czero, const float2* tw, int rev, hipStream_t st) {
+  if (n <= 0) return hipSuccess;
+  switch (F) {
+#define X(FF) \
+  case FF:    \
+    return launch_align_F<FF>(x, n, m, cspec, cnorm, czero, tw, rev, st);
+    TCX_FOR_EACH_F(X)
+#undef X
+    default:
+      return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace tcx

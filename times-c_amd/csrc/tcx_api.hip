@@ -51,7 +51,7 @@ enum Slot {
   kSlotCspec, kSlotCnorm, kSlotCzero, kSlotLabel, kSlotShift, kSlotDist, kSlotCent,
   kSlotCentNew, kSlotBlkCount, kSlotBlkBase, kSlotGroupInfo,
   kSlotPerm, kSlotYhi, kSlotYlo, kSlotA0, kSlotPlan, kSlotPart,
-  kSlotS, kSlotInfo, kSlotDummy, kSlotWbuf, kSlotRbuf, kSlotBar, kSlotVout, kSlotSteps,
+  kSlotS, kSlotInfo, kSlotWbuf, kSlotRbuf, kSlotBar, kSlotVout, kSlotSteps,
   kSlotConv, kSlotErr, kSlotCmag, kSlotEvals, kSlotSvout, kSlotLzW, kSlotLzState, kSlotMask,
   kSlotRowStats, kSlotFitRowStats, kSlotKeyCounts, kSlotKeyOff, kSlotMinRow, kSlotXs, kSlotXn,
   kSlotLzXch, kSlotXm, kSlotUb, kSlotCm, kSlotCheck, kSlotCheckInfo, kSlotSplit, kNumSlots
@@ -1077,12 +1077,10 @@ int tcx_sbd_align(tcx_ctx* c, float* d_members, const float* d_center, int rows,
   float* norm;
   int* zero;
   TCX_TRY(spectra(c, d_center, 1, cols, &spec, &norm, &zero));
-  int *lab, *sh;
-  TCX_TRY(ws(c, kSlotDummy, (size_t)rows, &lab));
-  TCX_TRY(ws(c, kSlotShift, (size_t)rows, &sh));
-  TCX_TRY(assign_core(c, d_members, rows, cols, 1, spec, norm, convention, lab, nullptr, sh,
-                      nullptr, nullptr));
-  TCX_HIP(tcx::launch_apply_shift(d_members, rows, cols, sh, zero, c->stream));
+  const int F = fft_size(cols);
+  const float2* tw;
+  TCX_TRY(twiddles(c, F, &tw));
+  TCX_HIP(tcx::launch_align(F, d_members, rows, cols, spec, norm, zero, tw, convention, c->stream));
   TCX_HIP(hipStreamSynchronize(c->stream));
   return TCX_OK;
 }

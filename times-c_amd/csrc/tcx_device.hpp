@@ -263,6 +263,15 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
   return (readlane_f64(v, 0) + readlane_f64(v, 16)) + (readlane_f64(v, 32) + readlane_f64(v, 48));
 }
 
+// Sum over each row of 16 lanes; every lane of the row gets it.
+__device__ __forceinline__ double row16_sum_f64(double v) {
+  v += dpp_f64<0xB1>(v);
+  v += dpp_f64<0x4E>(v);
+  v += dpp_f64<0x124>(v);
+  v += dpp_f64<0x128>(v);
+  return v;
+}
+
 // ---------------------------------------------------------- in-register DFT
 // exp(-2 pi i q / 32): table of cos / sin used for compile-time butterflies.
 constexpr float kCos32[32] = {

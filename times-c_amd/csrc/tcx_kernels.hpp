@@ -102,8 +102,10 @@ hipError_t launch_bounds(int F, const uint16_t* xm, long n, const uint16_t* cm, 
 hipError_t launch_sbd(int F, int mode, const SbdArgs& a, hipStream_t st);
 // Chunks the centroids of n series are worth splitting into (1: none).
 int sbd_chunks(int F, long n, int k, int cus);
-hipError_t launch_apply_shift(float* x, long rows, int m, const int* shift, const int* skip,
-                              hipStream_t st);
+// Shifts each row in place by the lag of its largest NCC with one centroid
+// (spectrum, norm and all-zero flag given; an all-zero one changes nothing).
+hipError_t launch_align(int F, float* x, long n, int m, const float2* cspec, const float* cnorm,
+                        const int* czero, const float2* tw, int rev, hipStream_t st);
 hipError_t configure_sbd_kernels();
 
 // ------------------------------------------------------------ extraction
@@ -300,9 +302,10 @@ struct ZnormJob {
 };
 // Rows of every job z-normalized (jobs with m % 4 == 0 and 16-byte aligned
 // rows in groups by vector count nv: 0 = the scalar form, else 2, 4, 8, 16).
-hipError_t launch_znorm_group(const GroupTable& g, int nv, hipStream_t st);
-int znorm_vectors(const float* x, int m);  // nv of launch_znorm for these rows
-long znorm_blocks(long rows);
+hipError_t launch_znorm_group(const GroupTable& g, int form, hipStream_t st);
+int znorm_form(const float* x, int m);  // form of launch_znorm for these rows
+long znorm_blocks(int form, long rows);
+long row_stats_blocks(long rows);
 
 struct SeriesSpecJob {
   const float* x;
