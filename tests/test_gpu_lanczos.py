@@ -64,3 +64,24 @@ def test_slow_convergence_uses_the_rows_past_lds(ctx, m):
     labels = np.zeros(4000, np.int32)
     got, ref = _extract(ctx, X, labels, 1)
     assert rel_l2(got[0], ref[0]) <= 10 * m * 2.0 ** -16 / np.sqrt(4000.0)
+
+
+@pytest.mark.parametrize("m,k", [(257, 1), (288, 3), (300, 24), (449, 5), (512, 16), (512, 17),
+                                 (512, 33), (513, 2), (640, 8), (1023, 8), (1024, 8), (1024, 9)])
+def test_blocks_of_one_cluster(ctx, m, k):
+    """Orders above 256: 32 and 64 rows per block, 512 and 1024 columns, a
+    last block with fewer rows, and the first sizes past what fits the device
+    at once."""
+    X, y = T.generate(7 * m + k, 40 * k + 3, m, k, 0.3)
+    y[y == k // 2] = 0  # an empty cluster (k > 1)
+    got, ref = _extract(ctx, X, y, k)
+    assert max(centroid_errors(got, ref)) <= CENT_RTOL
+
+
+@pytest.mark.parametrize("m", [400, 900])
+def test_blocks_slow_convergence(ctx, m):
+    """White noise over many blocks: more steps than basis rows in LDS.  The
+    tolerance is the one of the resident form above, at I = m."""
+    X = np.random.default_rng(m).standard_normal((4000, m)).astype(np.float32)
+    got, ref = _extract(ctx, X, np.zeros(4000, np.int32), 1)
+    assert rel_l2(got[0], ref[0]) <= 10 * m * 2.0 ** -16 / np.sqrt(4000.0)

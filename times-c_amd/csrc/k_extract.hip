@@ -3726,6 +3726,398 @@ __global__ __launch_bounds__(64 * NW) void k_lz_res(
   lz_res_body<NW, U, T>(a, lz_tol);
 }
 
+// --------------------------------- Lanczos of one cluster over many blocks
+// k_lz_coop's process for m <= 64 U with one exchange per step instead of two:
+// each of the cluster's G members keeps its R rows of S_j in registers (wave p
+// of four the rows [p RW, (p+1) RW), lane l their columns l + 64 u) and the
+// whole basis (QL rows in LDS), publishes its rows of M q and reads every
+// member's; the three-term recurrence and the Gram-Schmidt pass against the
+// basis then run alike in every member, on the same values in the same
+// order, so all agree on alpha, beta and the acceptance test bit for bit.
+// Published values and their tags are k_lz_coop's, in two buffers used in
+// turn: a member writes the slots of a step again two steps later, after it
+// has read every member's rows of the step between, which those published
+// after reading theirs of the first.  Basis rows past QL (rare) go to the
+// cluster's Q buffer: every member stores the same bits there and reads
+// back its own or an equal store (device-scope accesses).
+// Bound by latency: the exchange and the FP64 sums of a step.  n=100000 m=512
+// k=16 (16 members of 32 rows): 212 us per refinement with two exchanges, the
+// rows of S in LDS and a dozen barriers per step, 114 us now.
+constexpr int kLzMultiWaves = 4;
+template <int U>
+constexpr int lz_multi_rows() { return U <= 8 ? 28 : 13; }
+template <int U>
+constexpr size_t lz_multi_lds() {
+  return sizeof(double) * (64 * U * (size_t)(2 + lz_multi_rows<U>()) + 3 * (kLzMax + 1) + 1 +
+                           kLzMax + kLzResSqDoubles + 1);
+}
+// Exchange words per cluster: two buffers of m pairs, end marks.
+__host__ __device__ constexpr long lz_multi_xch_len(int m, int G) { return 4L * m + G; }
+
+// Wave sums of the N values t[0..N) (N = 8 or 16): every lane gets the sum of
+// t[wave_rows_index<N>(lane)].
+template <int N>
+__device__ __forceinline__ int wave_rows_index(int lane) {
+  return N == 8 ? lane >> 3 : lane >> 2;
+}
+template <int N>
+__device__ __forceinline__ double wave_rows_sum(const double (&t)[N], int lane) {
+  static_assert(N == 8 || N == 16, "rows");
+  double a[N / 2];
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) a[i] = swap_sum_f64<32>(t[i], t[i + N / 2]);
+  double b[N / 4];
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i) b[i] = swap_sum_f64<16>(a[i], a[i + N / 4]);
+  double c[N / 8];
+  const bool up8 = lane & 8;  // partner: the mirror in 16 lanes
+#pragma unroll
+  for (int i = 0; i < N / 8; ++i)
+    c[i] = (up8 ? b[i + N / 8] : b[i]) + dpp_f64<0x140>(up8 ? b[i] : b[i + N / 8]);
+  double v = c[0];
+  if constexpr (N == 16) {
+    const bool up4 = lane & 4;  // the mirror in 8 lanes
+    v = (up4 ? c[1] : c[0]) + dpp_f64<0x141>(up4 ? c[0] : c[1]);
+  } else {
+    v += dpp_f64<0x141>(v);
+  }
+  v += dpp_f64<0x4E>(v);
+  v += dpp_f64<0xB1>(v);
+  return v;
+}
+
+template <int U, int RW, typename T>
+__global__ __launch_bounds__(64 * kLzMultiWaves, 1) void k_lz_multi(
+    const float* __restrict__ S, int m, int k, int G, int R, const int* __restrict__ counts,
+    uint64_t seed, int iter, int I, double lz_tol, double* Qfar, uint64_t* __restrict__ xch,
+    uint32_t* __restrict__ fails, uint32_t gen, long long timeout, double* __restrict__ vout,
+    double* __restrict__ svout, double* __restrict__ rout, int* __restrict__ steps_out,
+    int* __restrict__ conv_out) {
+  constexpr int D = 64 * U, NW = kLzMultiWaves, QL = lz_multi_rows<U>(), E = U / NW;
+  static_assert(U % NW == 0, "elements per wave: E per lane");
+  extern __shared__ __align__(16) double msh[];
+  double* xw = msh;                      // D: the gathered vector
+  double* wb = xw + D;                   // D: the projected one
+  double* Qs = wb + D;                   // QL x D basis rows
+  double* alpha = Qs + QL * D;           // kLzMax + 1
+  double* beta = alpha + kLzMax + 1;     // kLzMax + 1
+  double* cf = beta + kLzMax + 1;        // kLzMax + 2
+  double* y = cf + kLzMax + 2;           // kLzMax
+  double* wk = y + kLzMax;               // kLzResSqDoubles
+  int* bad = reinterpret_cast<int*>(wk + kLzResSqDoubles);  // a wait of this member gave up
+  // member -> (cluster, index): consecutive blocks go to consecutive XCDs,
+  // so numbering XCD by XCD puts the members of a cluster on one XCD
+  const int per = gridDim.x / 8;
+  const int p = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  const int j = p / G, b = p % G;
+  if (j >= k || counts[j] == 0) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int e0 = b * R;
+  const int nr = m - e0 < R ? m - e0 : R;
+  const float* Sg = S + (long)j * m * m + (long)e0 * m;
+  double* Qg = Qfar + (long)j * (kLzMax + 1) * m;
+  uint64_t* X = xch + (long)j * lz_multi_xch_len(m, G);
+  uint64_t* Done = X + 4L * m;
+  uint32_t* fail = fails + j;
+  const uint32_t tag0 = gen << kLzCoopEpochBits;
+  int len = 0, conv = 0;
+  auto give_up = [&]() {
+    if (tid == 0) __hip_atomic_store(fail, gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (b == 0 && tid == 0) {
+      steps_out[j] = len;
+      conv_out[j] = 0;
+    }
+  };
+  if (tid == 0) *bad = 0;
+  // the wave's rows of S, zero outside
+  T sr[RW][U];
+#pragma unroll
+  for (int q = 0; q < RW; ++q) {
+    const int row = wv * RW + q;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int c = lane + 64 * u;
+      sr[q][u] = row < nr && c < m ? (T)Sg[(long)row * m + c] : (T)0;
+    }
+  }
+  const int row = wv * RW + wave_rows_index<RW>(lane);  // the row this lane ends a matvec with
+  const bool writer = (lane & (64 / RW - 1)) == 0 && row < nr;
+  // this lane's row of S x, x the same in every wave
+  auto matvec = [&](const double (&x)[U]) {
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int q = 0; q < RW; ++q)
+#pragma unroll
+        for (int u = 0; u < U; ++u) asm volatile("" : "+v"(sr[q][u]));
+    }
+    double t[RW];
+#pragma unroll
+    for (int q = 0; q < RW; ++q) t[q] = 0.0;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int q = 0; q < RW; ++q) t[q] += (double)sr[q][u] * x[u];
+    return wave_rows_sum<RW>(t, lane);
+  };
+  const int own_e = wv * (D / NW) + lane;  // this lane's elements own_e + 64 i
+  const int own_n = own_e < m ? ((m - 1 - own_e) / 64 + 1 < E ? (m - 1 - own_e) / 64 + 1 : E) : 0;
+  // every member's rows published in buffer `buf` with `tag`: own elements
+  // and, through LDS, the whole vector; false when a wait gave up
+  auto gather = [&](int buf, uint32_t tag, double (&own)[E], double (&w)[U]) {
+    double v[E];
+    const bool good = poll_tagged<E>(X + 2L * buf * m + 2L * own_e, 64, own_n, tag, v, fail, gen,
+                                     timeout);
+    if (!good) *bad = 1;
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      own[i] = good && i < own_n ? v[i] : 0.0;
+      xw[own_e + 64 * i] = own[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) w[u] = xw[lane + 64 * u];
+    return *bad == 0;
+  };
+  auto spread = [&](double* dst, const double (&own)[E], double (&w)[U]) {
+#pragma unroll
+    for (int i = 0; i < E; ++i) dst[own_e + 64 * i] = own[i];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) w[u] = dst[lane + 64 * u];
+  };
+  // far rows through device-scope accesses (see above)
+  auto far = [&](int l, int e) {
+    return e < m ? ld_dev_f64(reinterpret_cast<uint64_t*>(Qg + (long)l * m + e)) : 0.0;
+  };
+  auto put_row = [&](int l, const double (&own)[E]) {
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      const int e = own_e + 64 * i;
+      if (l < QL)
+        Qs[l * D + e] = own[i];
+      else if (e < m)
+        st_dev_f64(reinterpret_cast<uint64_t*>(Qg + (long)l * m + e), own[i]);
+    }
+    if (l >= QL) wait_vmem();  // before the barrier ahead of its readers
+  };
+  // cf[l] = q_l . w for l <= it, rows split over the waves; ends with a barrier
+  auto dots = [&](const double (&w)[U], int it) {
+    constexpr int kB = 4;
+    const int near = it < QL ? it : QL - 1;
+    for (int l0 = wv; l0 <= near; l0 += kB * NW) {
+      double t[kB];
+#pragma unroll
+      for (int q = 0; q < kB; ++q) {
+        const double* r = Qs + (l0 + q * NW <= near ? l0 + q * NW : l0) * D + lane;
+        t[q] = 0.0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) t[q] += r[64 * u] * w[u];
+      }
+      const double v = wave_sum4_f64(t[0], t[1], t[2], t[3]);
+      const int l = l0 + (lane >> 4) * NW;
+      if ((lane & 15) == 0 && l <= near) cf[l] = v;
+    }
+    for (int l = QL + wv; l <= it; l += NW) {
+      double t = 0.0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) t += far(l, lane + 64 * u) * w[u];
+      t = wave_sum_f64(t);
+      if (lane == 0) cf[l] = t;
+    }
+    __syncthreads();
+  };
+  // sum_{l < n} c[l] q_l on this lane's elements
+  auto combine = [&](const double* c, int n, double (&o)[E]) {
+    double o1[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) o[i] = o1[i] = 0.0;
+    const int near = n < QL ? n : QL;
+    const double* r = Qs + own_e;
+    int l = 0;
+#pragma unroll 4
+    for (; l + 1 < near; l += 2, r += 2 * D) {
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        o[i] += c[l] * r[64 * i];
+        o1[i] += c[l + 1] * r[D + 64 * i];
+      }
+    }
+    if (l < near)
+#pragma unroll
+      for (int i = 0; i < E; ++i) o[i] += c[l] * r[64 * i];
+    for (l = QL; l < n; ++l)
+#pragma unroll
+      for (int i = 0; i < E; ++i) o[i] += c[l] * far(l, own_e + 64 * i);
+#pragma unroll
+    for (int i = 0; i < E; ++i) o[i] += o1[i];
+  };
+  auto sums = [&](const double (&a)[U], const double (&c)[U], const double (&r)[U], double& aa,
+                  double& ca, double& sa, double& ra) {
+    double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      t0 += a[u] * a[u];
+      t1 += c[u] * a[u];
+      t2 += a[u];
+      t3 += r[u] * a[u];
+    }
+    const double v = wave_sum4_f64(t0, t1, t2, t3);
+    aa = readlane_f64(v, 0);
+    ca = readlane_f64(v, 16);
+    sa = readlane_f64(v, 32);
+    ra = readlane_f64(v, 48);
+  };
+  double q[U], w[U], r[U], own[E], own_q[E], own_qp[E], qp[U];
+  // r = S 1, exchanged; q_0 = power_v0 / |power_v0|
+#pragma unroll
+  for (int u = 0; u < U; ++u) q[u] = lane + 64 * u < m ? 1.0 : 0.0;
+  const double r_row = matvec(q);
+  if (writer) {
+    put_tagged(X + 2L * (e0 + row), r_row, tag0 | 1);
+    rout[(long)j * m + e0 + row] = r_row;
+  }
+  double n0 = 0.0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int e = lane + 64 * u;
+    q[u] = e < m ? power_v0(seed, iter, j, e) : 0.0;
+    n0 += q[u] * q[u];
+    qp[u] = 0.0;
+  }
+  n0 = sqrt(wave_sum_f64(n0));
+  __syncthreads();  // *bad is set
+  if (!gather(0, tag0 | 1, own, r)) return give_up();
+  double sigma = 0.0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    sigma += r[u];
+    q[u] /= n0;
+  }
+  sigma = wave_sum_f64(sigma);
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const int e = own_e + 64 * i;
+    own_q[i] = e < m ? power_v0(seed, iter, j, e) / n0 : 0.0;
+    own_qp[i] = 0.0;
+  }
+  put_row(0, own_q);
+  __syncthreads();  // xw is read before the next gather writes it
+  const int jmax = m < kLzMax ? m : kLzMax;
+  const double inv_m = 1.0 / (double)m;
+  int prev_len = 0;
+  double yp0 = 0.0, yp1 = 0.0, bprev = 0.0;
+  double qq, qs, sv, rv;  // 1.q and r.q
+  sums(q, q, r, qq, qs, sv, rv);
+  for (int it = 0; it < jmax; ++it) {
+    const int buf = (it + 1) & 1;
+    const uint32_t tag = tag0 | (uint32_t)(2 + it);
+    const double sw_row = matvec(q);
+    if (writer)
+      put_tagged(X + 2L * buf * m + 2L * (e0 + row),
+                 sw_row - (r_row * sv + rv) * inv_m + sigma * sv * inv_m * inv_m, tag);
+    if (!gather(buf, tag, own, w)) return give_up();
+    double nw2, al, s1, r1;
+    sums(w, q, r, nw2, al, s1, r1);
+    // three-term recurrence, then Gram-Schmidt against the whole basis,
+    // again when it removed more than half of |w|^2
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      w[u] = w[u] - al * q[u] - bprev * qp[u];
+      qp[u] = q[u];
+    }
+#pragma unroll
+    for (int i = 0; i < E; ++i) own[i] = own[i] - al * own_q[i] - bprev * own_qp[i];
+    double w1 = 0.0, bb;
+#pragma unroll
+    for (int u = 0; u < U; ++u) w1 += w[u] * w[u];
+    w1 = wave_sum_f64(w1);
+    for (int pass = 0; pass < 2; ++pass) {
+      dots(w, it);
+      double o[E];
+      combine(cf, it + 1, o);
+#pragma unroll
+      for (int i = 0; i < E; ++i) own[i] -= o[i];
+      spread(wb, own, w);
+      double t;
+      sums(w, q, r, bb, t, s1, r1);
+      if (!(bb < 0.5 * w1)) break;
+      w1 = bb;
+    }
+    const double bnorm = sqrt(bb);
+    if (tid == 0) alpha[it] = al;
+    len = it + 1;
+    const bool breakdown = !(bnorm > 1e-12 * sqrt(nw2));
+    if (breakdown || len == jmax || lz_power_check(len)) {
+      __syncthreads();  // alpha, beta visible
+      if (len <= kLzResSq) {
+        tridiag_power_mfma<NW>(alpha, beta, len, I, wk, y);
+      } else {
+        if (wv == 0) tridiag_power_wave(alpha, beta, len, I, y);
+        __syncthreads();
+      }
+      const double y0 = lane < len ? y[lane] : 0.0, y1 = lane + 64 < len ? y[lane + 64] : 0.0;
+      const double dd = wave_sum_f64((y0 - yp0) * (y0 - yp0) + (y1 - yp1) * (y1 - yp1));
+      conv = breakdown || (prev_len > 0 && sqrt(dd) <= lz_tol);
+      yp0 = y0;
+      yp1 = y1;
+      prev_len = len;
+      if (conv || breakdown) break;
+    }
+    if (len == jmax) break;
+    if (tid == 0) beta[it + 1] = bnorm;
+    const double inv_b = 1.0 / bnorm;
+#pragma unroll
+    for (int u = 0; u < U; ++u) q[u] = w[u] * inv_b;
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      own_qp[i] = own_q[i];
+      own_q[i] = own[i] * inv_b;
+    }
+    bprev = bnorm;
+    sv = s1 * inv_b;
+    rv = r1 * inv_b;
+    put_row(it + 1, own_q);  // visible after the next gather's barrier
+  }
+  // v = Q y (zero when the check never passed) and the member's rows of S v
+#pragma unroll
+  for (int i = 0; i < E; ++i) own[i] = 0.0;
+  if (conv) combine(y, len, own);
+  spread(xw, own, w);
+  const double sv_row = matvec(w);
+  if (writer) {
+    svout[(long)j * m + e0 + row] = sv_row;
+    vout[(long)j * m + e0 + row] = xw[e0 + row];
+  }
+  // member 0 reports the cluster once every member has written its rows
+  const uint32_t tag = tag0 | (uint32_t)(2 + kLzMax);
+  wait_vmem();
+  __syncthreads();
+  if (tid == 0) st_dev_u64(Done + b, (uint64_t)tag << 32);
+  if (b == 0) {
+    bool good = timeout >= 0;
+    if (tid < kWave && good) {
+      const long long t0 = wall_clock64();
+      for (;;) {
+        bool mine = true;
+        for (int g = tid; g < G; g += kWave)
+          mine = mine && (uint32_t)(ld_dev_u64(Done + g) >> 32) == tag;
+        if (__all(mine)) break;
+        if (__hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gen ||
+            wall_clock64() - t0 > timeout) {
+          good = false;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+    }
+    if (tid == 0) {
+      steps_out[j] = len;
+      conv_out[j] = good ? conv : 0;
+    }
+  }
+}
+
 #define TCX_GROUP_ARGS(T) static_cast<const T*>(g.jobs), g.first, g.njobs
 
 hipError_t launch_group_count_group(const GroupTable& g, hipStream_t st) {
@@ -3893,6 +4285,63 @@ hipError_t launch_lz_res(const float* S, int m, int k, const int* counts, uint64
   return hipGetLastError();
 }
 
+// Forms of k_lz_multi: {U, RW, LDS}; rows per member R = 4 RW at most.
+bool plan_lz_multi(int m, int k, int cus, LzCoopPlan* p) {
+  if (m <= kLzResMaxD || m > kLzMultiMaxM || k <= 0) return false;
+  for (int form = m <= 512 ? 0 : 2; form < 3; ++form) {
+    const int rmax = form == 1 ? 64 : 32;
+    const int G = (m + rmax - 1) / rmax, R = (m + G - 1) / G;
+    const long nb = ((long)k * G + 7) / 8 * 8;
+    if (nb > cus || (long)(G - 1) * R >= m) continue;  // every member owns rows
+    const void* fn = form == 0   ? (const void*)k_lz_multi<8, 8, double>
+                     : form == 1 ? (const void*)k_lz_multi<8, 16, float>
+                                 : (const void*)k_lz_multi<16, 8, float>;
+    const size_t lds = form == 2 ? lz_multi_lds<16>() : lz_multi_lds<8>();
+    int per_cu = 0;  // every member must be resident at once
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64 * kLzMultiWaves, lds) !=
+        hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    if ((long)per_cu * cus < nb) continue;
+    p->G = G;
+    p->R = R;
+    p->nb = (int)nb;
+    p->form = form;
+    p->lds = lds;
+    p->xch_len = lz_multi_xch_len(m, G);
+    return true;
+  }
+  return false;
+}
+
+hipError_t launch_lz_multi(const LzCoopPlan& p, const float* S, int m, int k, const int* counts,
+                           uint64_t seed, int iter, int I, double lz_tol, double* Q,
+                           uint64_t* xch, uint32_t* fails, uint32_t gen, long long timeout,
+                           double* vout, double* svout, double* rout, int* steps_out,
+                           int* conv_out, hipStream_t st) {
+  if (gen == 0 || gen >= (1u << (32 - kLzCoopEpochBits))) return hipErrorInvalidValue;
+#define TCX_LZ_MULTI(U, RW, T)                                                                    \
+  hipLaunchKernelGGL((k_lz_multi<U, RW, T>), dim3(p.nb), dim3(64 * kLzMultiWaves), p.lds, st, S,  \
+                     m, k, p.G, p.R, counts, seed, iter, I, lz_tol, Q, xch, fails, gen, timeout,  \
+                     vout, svout, rout, steps_out, conv_out)
+  switch (p.form) {
+    case 0:
+      TCX_LZ_MULTI(8, 8, double);
+      break;
+    case 1:
+      TCX_LZ_MULTI(8, 16, float);
+      break;
+    case 2:
+      TCX_LZ_MULTI(16, 8, float);
+      break;
+    default:
+      return hipErrorInvalidValue;
+  }
+#undef TCX_LZ_MULTI
+  return hipGetLastError();
+}
+
 size_t power_lanczos_lds(int m) { return lanczos_smem(m); }
 
 hipError_t launch_power_lanczos_group(const GroupTable& g, double lz_tol, hipStream_t st) {
@@ -3973,6 +4422,14 @@ hipError_t configure_extract_kernels() {
   if (e == hipSuccess)
     e = hipFuncSetAttribute((const void*)k_align_pack_lds<16>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, kPackLdsMaxBytes);
+#define TCX_LZ_MULTI(U, RW, T)                                                               \
+  if (e == hipSuccess)                                                                       \
+    e = hipFuncSetAttribute((const void*)k_lz_multi<U, RW, T>,                               \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lz_multi_lds<U>());
+  TCX_LZ_MULTI(8, 8, double)
+  TCX_LZ_MULTI(8, 16, float)
+  TCX_LZ_MULTI(16, 8, float)
+#undef TCX_LZ_MULTI
 #define TCX_LZ_RES(NW, U, T)                                                                 \
   if (e == hipSuccess)                                                                       \
     e = hipFuncSetAttribute((const void*)k_lz_res<NW, U, T>,                                 \

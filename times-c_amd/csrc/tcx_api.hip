@@ -455,7 +455,8 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
     return TCX_OK;
   }
   tcx::LzCoopPlan cp;
-  if (mode == 0 && !mask && tcx::plan_lz_coop(m, k, c->cus, &cp)) {
+  const bool multi = mode == 0 && !mask && tcx::plan_lz_multi(m, k, c->cus, &cp);
+  if (multi || (mode == 0 && !mask && tcx::plan_lz_coop(m, k, c->cus, &cp))) {
     // exchange words and per-cluster failure words; their contents only
     // ever match the current launch generation, so they are zeroed only
     // when (re)allocated or when the generation wraps
@@ -487,12 +488,16 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
         const long long us = std::atoll(e);
         timeout = us < 0 ? -1 : c->wall_khz * us / 1000;
       }
-      TCX_HIP(tcx::launch_lz_coop(cp, S, m, k, counts, seed, iter, steps, tcx::kLzPowerTol, xch,
-                                  fails, gen, timeout, v, r, st_out, cv_out, st));
+      if (multi)
+        TCX_HIP(tcx::launch_lz_multi(cp, S, m, k, counts, seed, iter, steps, tcx::kLzPowerTol, Q,
+                                     xch, fails, gen, timeout, v, sv, r, st_out, cv_out, st));
+      else
+        TCX_HIP(tcx::launch_lz_coop(cp, S, m, k, counts, seed, iter, steps, tcx::kLzPowerTol, xch,
+                                    fails, gen, timeout, v, r, st_out, cv_out, st));
       TCX_HIP(hipEventRecord(c->coop_ev, st));
       g_coop_last[c->device] = c->coop_ev;
     }
-    TCX_HIP(tcx::launch_cluster_matvec(S, m, k, v, m, sv, nullptr, st));  // S v
+    if (!multi) TCX_HIP(tcx::launch_cluster_matvec(S, m, k, v, m, sv, nullptr, st));  // S v
     *vout = v;
     *svout = sv;
     *rout = r;

@@ -244,6 +244,7 @@ struct LzCoopPlan {
   bool s_lds = false;
   size_t lds = 0;            // dynamic LDS bytes per block
   long xch_len = 0;          // exchange words per cluster
+  int form = 0;              // k_lz_multi's register split
 };
 // False when m, k or the device do not allow every member to be resident.
 bool plan_lz_coop(int m, int k, int cus, LzCoopPlan* p);
@@ -256,6 +257,17 @@ hipError_t launch_lz_coop(const LzCoopPlan& p, const float* S, int m, int k, con
                           uint64_t seed, int iter, int I, double lz_tol, uint64_t* xch,
                           uint32_t* fails, uint32_t gen, long long timeout, double* vout,
                           double* rout, int* steps_out, int* conv_out, hipStream_t st);
+// The same with one exchange per step and the rows of S in registers
+// (k_lz_multi; S v written too, Q: (kLanczosMax + 1) x m per cluster for basis
+// rows past those in LDS), for kLzResMaxD < m <= kLzMultiMaxM when all members
+// fit the device at once.
+constexpr int kLzMultiMaxM = 1024;
+bool plan_lz_multi(int m, int k, int cus, LzCoopPlan* p);
+hipError_t launch_lz_multi(const LzCoopPlan& p, const float* S, int m, int k, const int* counts,
+                           uint64_t seed, int iter, int I, double lz_tol, double* Q,
+                           uint64_t* xch, uint32_t* fails, uint32_t gen, long long timeout,
+                           double* vout, double* svout, double* rout, int* steps_out,
+                           int* conv_out, hipStream_t st);
 hipError_t launch_power_lanczos(const float* S, int m, int k, const int* counts, uint64_t seed,
                                 int iter, int I, double lz_tol, double* Q, double* vout,
                                 double* rout, int* steps_out, int* conv_out, hipStream_t st);
