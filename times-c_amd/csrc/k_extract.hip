@@ -34,6 +34,16 @@ __global__ void k_fill_int(int* p, long count, int value) {
     p[i] = value;
 }
 
+// Start of a refinement: the status words zeroed, the lowest rows INT_MAX,
+// the row order all holes.
+__global__ __launch_bounds__(256) void k_refine_init(int* status, int* __restrict__ minrow, int k,
+                                                     int* __restrict__ perm, long n_pad) {
+  const long i0 = (long)blockIdx.x * 256 + threadIdx.x, step = (long)gridDim.x * 256;
+  if (i0 < kRefineStatusInts) status[i0] = 0;
+  for (long i = i0; i < k; i += step) minrow[i] = 0x7fffffff;
+  for (long i = i0; i < n_pad; i += step) perm[i] = -1;
+}
+
 // -------------------------------------------------------------- grouping
 // Rows are grouped by the key label * B + bin, bin = the row's previous
 // SBD distance (in [0, 2]) in B equal bins (B = 1 without distances).
@@ -772,7 +782,8 @@ __device__ __forceinline__ void syrk_block_of(int u, const int T, int& ti, int& 
 // kSyrkSub block u of S_j over the group's columns into that block's
 // partial.  Slots past the last group are holes.
 template <bool kSplit>
-__global__ __launch_bounds__(256) void k_syrk(const SyrkGroup* __restrict__ groups, int ngroups,
+__global__ __launch_bounds__(256) void k_syrk(const SyrkGroup* __restrict__ groups,
+                                              const SyrkPlanHead* __restrict__ head,
                                               const uint16_t* __restrict__ yhi,
                                               const uint16_t* __restrict__ ylo, int m,
                                               float* __restrict__ part) {
@@ -782,7 +793,7 @@ __global__ __launch_bounds__(256) void k_syrk(const SyrkGroup* __restrict__ grou
   // is derived from it
   const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x >> 3) * 4 + (int)(threadIdx.x >> 6));
   const int g = (blockIdx.x & 7) + 8 * (w / U);
-  if (g >= ngroups) return;
+  if (g >= head->ngroups) return;
   const int u = w % U;
   int ti, tj;
   syrk_block_of(u, T, ti, tj);
@@ -847,17 +858,97 @@ __device__ __forceinline__ void syrk_reduce_body(const int sb, const SyrkTile tl
 // Single fit: (kSyrkSub / 64)^2 blocks per kSyrkSub block of each cluster
 // with partials, clusters[c] covering the blocks from c * T(T+1)/2 on.
 __global__ __launch_bounds__(256) void k_syrk_reduce(const SyrkCluster* __restrict__ clusters,
+                                                     const SyrkPlanHead* __restrict__ head,
                                                      const float* __restrict__ part, int m,
                                                      float* __restrict__ S) {
   constexpr int kSub = kSyrkSub / 64;
   const int T = (m + kSyrkSub - 1) / kSyrkSub, U = T * (T + 1) / 2;
   const int t = blockIdx.x / (kSub * kSub), u = t % U;
+  if (t / U >= head->nclusters) return;
   const SyrkCluster c = clusters[t / U];
   int ti, tj;
   syrk_block_of(u, T, ti, tj);
   syrk_reduce_body(blockIdx.x % (kSub * kSub),
                              SyrkTile{c.cluster, ti, tj, c.part0 + u * c.nparts, c.nparts}, part,
                              m, S);
+}
+
+// The plan of S = Y^T Y (plan_syrk's, group for group) from the cluster sizes
+// on the device, by one block: the shortest chunk bound in whole 16-column
+// steps, at least kSyrkMinSteps, whose groups are at most gmax, by bisection
+// (each trial one block sum over the clusters), then every cluster's first
+// group and partial by a scan 256 clusters at a time.  Bound by its block sums'
+// latency, a few us; the host's plan took a wait for the sizes and two copies,
+// during which the device idled.  With the wait after the power stage left out
+// too (refine's pending), a fit's iteration waits once, not three times: a fit
+// n=512 m=128 k=4 about 1120 -> 965 us, one of 10 iterations n=100000 m=512
+// k=16 9450 -> 9030.
+__global__ __launch_bounds__(256) void k_syrk_plan(const long* __restrict__ offsets,
+                                                   const int* __restrict__ counts, int k, int U,
+                                                   int gmax, SyrkPlanHead* __restrict__ head,
+                                                   SyrkGroup* __restrict__ groups,
+                                                   SyrkCluster* __restrict__ clusters) {
+  __shared__ int red[4];
+  __shared__ int scan[2][256];
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  auto steps_of = [&](int j) -> int {
+    return counts[j] > 0 ? (int)((offsets[j + 1] - offsets[j] + 15) / 16) : 0;
+  };
+  auto block_total = [&](int v, bool take_max) -> int {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const int u = __shfl_xor(v, o);
+      v = take_max ? max(v, u) : v + u;
+    }
+    __syncthreads();
+    if (lane == 0) red[wid] = v;
+    __syncthreads();
+    return take_max ? max(max(red[0], red[1]), max(red[2], red[3]))
+                    : (red[0] + red[1]) + (red[2] + red[3]);
+  };
+  int mx = 0;
+  for (int j = t; j < k; j += 256) mx = max(mx, steps_of(j));
+  const int max_steps = block_total(mx, true);
+  if (max_steps == 0) {
+    if (t == 0) *head = SyrkPlanHead{0, 0};
+    return;
+  }
+  int lo = min(kSyrkMinSteps, max_steps), hi = max_steps;
+  while (lo < hi) {
+    const int mid = (lo + hi) / 2;
+    int g = 0;
+    for (int j = t; j < k; j += 256) g += (steps_of(j) + mid - 1) / mid;
+    if (block_total(g, false) <= gmax) hi = mid; else lo = mid + 1;
+  }
+  int g0 = 0, c0 = 0;  // groups and clusters before this tile of clusters
+  for (int j0 = 0; j0 < k; j0 += 256) {
+    const int j = j0 + t;
+    const int st = j < k ? steps_of(j) : 0, nc = (st + lo - 1) / lo;
+    scan[0][t] = nc;
+    scan[1][t] = st > 0;
+    __syncthreads();
+    for (int o = 1; o < 256; o <<= 1) {
+      const int a = t >= o ? scan[0][t - o] : 0, b = t >= o ? scan[1][t - o] : 0;
+      __syncthreads();
+      scan[0][t] += a;
+      scan[1][t] += b;
+      __syncthreads();
+    }
+    const int g = g0 + scan[0][t] - nc, c = c0 + scan[1][t] - (st > 0);
+    if (st > 0) {
+      const int part = g * U;  // U partials per group before
+      clusters[c] = SyrkCluster{j, part, nc};
+      const long off = offsets[j], len = offsets[j + 1] - off;
+      for (int q = 0; q < nc; ++q) {
+        const long s0 = (long)st * q / nc, s1 = (long)st * (q + 1) / nc;
+        groups[g + q] = SyrkGroup{part + q, nc, off + 16 * s0, off + (len < 16 * s1 ? len : 16 * s1)};
+      }
+    }
+    g0 += scan[0][255];
+    c0 += scan[1][255];
+    __syncthreads();  // scan is rewritten by the next tile
+  }
+  if (t == 0) *head = SyrkPlanHead{g0, c0};
 }
 
 // ---------------------------------------------------------- power iteration
@@ -1077,7 +1168,8 @@ __device__ __forceinline__ void power_body(const int bid, const int nblk,
     const double* __restrict__ vin, const double* __restrict__ svin,
     const double* __restrict__ rsum, const int* __restrict__ steps_in,
     const int* __restrict__ conv_in, int eig_mode, const int* __restrict__ mask,
-    int defer_fallback, float* __restrict__ c_out, PowerInfo* __restrict__ info) {
+    int defer_fallback, float* __restrict__ c_out, PowerInfo* __restrict__ info,
+    int* __restrict__ redo) {
   extern __shared__ double sh[];
   double* v = sh;
   double* w = sh + m;
@@ -1231,6 +1323,7 @@ __device__ __forceinline__ void power_body(const int bid, const int nblk,
     inf.fallback = fallback;
     inf.flipped = flipped;
     info[j] = inf;
+    if (redo && fallback) *redo = 1;  // to be rerun (every writer stores 1)
   }
 }
 
@@ -1240,8 +1333,9 @@ __global__ __launch_bounds__(kPowerThreads) void k_power(
     const double* __restrict__ vin, const double* __restrict__ svin,
     const double* __restrict__ rsum, const int* __restrict__ steps_in,
     const int* __restrict__ conv_in, int eig_mode, const int* __restrict__ mask,
-    int defer_fallback, float* __restrict__ c_out, PowerInfo* __restrict__ info) {
-  power_body(blockIdx.x, gridDim.x, S, m, counts, a0all, seed, iter, max_steps, tol, vin, svin, rsum, steps_in, conv_in, eig_mode, mask, defer_fallback, c_out, info);
+    int defer_fallback, float* __restrict__ c_out, PowerInfo* __restrict__ info,
+    int* __restrict__ redo) {
+  power_body(blockIdx.x, gridDim.x, S, m, counts, a0all, seed, iter, max_steps, tol, vin, svin, rsum, steps_in, conv_in, eig_mode, mask, defer_fallback, c_out, info, redo);
 }
 
 // ----------------------------------------------------- Lanczos power result
@@ -2710,7 +2804,7 @@ __global__ __launch_bounds__(kPowerThreads) void k_power_group(const PowerJob* _
   TCX_GROUP_JOB(PowerJob)
   power_body(bid, nblk, a.S, a.m, a.counts, a.a0, a.seed, a.iter, a.max_steps, a.tol, a.vin,
              a.svin, a.rsum, a.steps_in, a.conv_in, a.eig_mode, a.mask, a.defer_fallback, a.c_out,
-             a.info);
+             a.info, nullptr);
 }
 
 hipError_t launch_fill_int(int* p, long count, int value, hipStream_t st) {
@@ -2810,24 +2904,53 @@ long syrk_blocks(int m, int ngroups) {
   return 8 * (((ngroups + 7) / 8 * U + 3) / 4);
 }
 
-hipError_t launch_syrk(const SyrkGroup* groups, int ngroups, const uint16_t* yhi,
-                       const uint16_t* ylo, int m, int split, float* part, hipStream_t st) {
-  if (ngroups <= 0) return hipSuccess;
-  const dim3 grid((unsigned)syrk_blocks(m, ngroups));
-  if (split)
-    hipLaunchKernelGGL(k_syrk<true>, grid, dim3(256), 0, st, groups, ngroups, yhi, ylo, m, part);
-  else
-    hipLaunchKernelGGL(k_syrk<false>, grid, dim3(256), 0, st, groups, ngroups, yhi, ylo, m, part);
+hipError_t launch_refine_init(int* status, int* minrow, int k, int* perm, long n_pad,
+                              hipStream_t st) {
+  long blocks = (std::max<long>(n_pad, k) + 255) / 256;
+  if (blocks > 1024) blocks = 1024;
+  if (blocks < 1) blocks = 1;
+  hipLaunchKernelGGL(k_refine_init, dim3((unsigned)blocks), dim3(256), 0, st, status, minrow, k,
+                     perm, n_pad);
   return hipGetLastError();
 }
 
-hipError_t launch_syrk_reduce(const SyrkCluster* clusters, int nclusters, const float* part, int m,
-                              float* S, hipStream_t st) {
-  if (nclusters <= 0) return hipSuccess;
+int syrk_max_groups(int m, int cus) {
+  constexpr long kXcds = 8;
+  const long T = (m + kSyrkSub - 1) / kSyrkSub, U = T * (T + 1) / 2;  // waves per group
+  const long slots = 4L * (cus > 1 ? cus : 1);  // one wave per SIMD
+  const long per_xcd = slots / kXcds > 1 ? slots / kXcds : 1;
+  return (int)(U <= per_xcd ? kXcds * (per_xcd / U) : (slots / U > 1 ? slots / U : 1));
+}
+
+hipError_t launch_syrk_plan(const long* offsets, const int* counts, int m, int k, int cus,
+                            SyrkPlanHead* head, SyrkGroup* groups, SyrkCluster* clusters,
+                            hipStream_t st) {
+  const int T = (m + kSyrkSub - 1) / kSyrkSub;
+  hipLaunchKernelGGL(k_syrk_plan, dim3(1), dim3(256), 0, st, offsets, counts, k, T * (T + 1) / 2,
+                     syrk_max_groups(m, cus), head, groups, clusters);
+  return hipGetLastError();
+}
+
+hipError_t launch_syrk(const SyrkGroup* groups, const SyrkPlanHead* head, int max_groups,
+                       const uint16_t* yhi, const uint16_t* ylo, int m, int split, float* part,
+                       hipStream_t st) {
+  if (max_groups <= 0) return hipSuccess;
+  const dim3 grid((unsigned)syrk_blocks(m, max_groups));
+  if (split)
+    hipLaunchKernelGGL(k_syrk<true>, grid, dim3(256), 0, st, groups, head, yhi, ylo, m, part);
+  else
+    hipLaunchKernelGGL(k_syrk<false>, grid, dim3(256), 0, st, groups, head, yhi, ylo, m, part);
+  return hipGetLastError();
+}
+
+hipError_t launch_syrk_reduce(const SyrkCluster* clusters, const SyrkPlanHead* head,
+                              int max_clusters, const float* part, int m, float* S,
+                              hipStream_t st) {
+  if (max_clusters <= 0) return hipSuccess;
   constexpr int kSub = kSyrkSub / 64;
   const long T = (m + kSyrkSub - 1) / kSyrkSub, U = T * (T + 1) / 2;
-  hipLaunchKernelGGL(k_syrk_reduce, dim3((unsigned)(nclusters * U * kSub * kSub)), dim3(256), 0,
-                     st, clusters, part, m, S);
+  hipLaunchKernelGGL(k_syrk_reduce, dim3((unsigned)(max_clusters * U * kSub * kSub)), dim3(256), 0,
+                     st, clusters, head, part, m, S);
   return hipGetLastError();
 }
 
@@ -2839,10 +2962,10 @@ hipError_t launch_power(const float* S, int m, int k, const int* counts, const f
                         uint64_t seed, int iter, int max_steps, double tol, const double* vin,
                         const double* svin, const double* rsum, const int* steps_in,
                         const int* conv_in, int eig_mode, const int* mask, int defer_fallback,
-                        float* c_out, PowerInfo* info, hipStream_t st) {
+                        float* c_out, PowerInfo* info, int* redo, hipStream_t st) {
   hipLaunchKernelGGL(k_power, dim3(k), dim3(kPowerThreads), power_smem(m), st, S, m, counts,
                      a0, seed, iter, max_steps, tol, vin, svin, rsum, steps_in, conv_in, eig_mode,
-                     mask, defer_fallback, c_out, info);
+                     mask, defer_fallback, c_out, info, redo);
   return hipGetLastError();
 }
 

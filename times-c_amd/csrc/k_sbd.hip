@@ -240,10 +240,11 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWaves) void k_s
     const float2* __restrict__ twg, int rev, int* __restrict__ label,
     float* __restrict__ dist, int* __restrict__ shift, float* __restrict__ dmat,
     int* __restrict__ changed, float* __restrict__ ncc_out,
-    const int* __restrict__ fixed_label) {
+    const int* __restrict__ fixed_label, const int* __restrict__ skip) {
   using G = FftGeom<F>;
   constexpr int L = G::L, P = G::P;
   extern __shared__ float2 smem[];
+  if (MODE == kModeAssign && skip && *skip) return;
   float2* tw = smem;
   float* red = reinterpret_cast<float*>(smem + fft_tw_lds<F>() + G::kGroups * fft_buf_len<F>());
   for (int i = threadIdx.x; i < fft_tw_lds<F>(); i += blockDim.x) tw[i] = twg[i];
@@ -955,7 +956,9 @@ __global__ __launch_bounds__(PruneGeom<F>::kBlock, PruneGeom<F>::kMinWaves) void
     const float2* __restrict__ cspec, const float* __restrict__ cmag,
     const float* __restrict__ cnorm, const float2* __restrict__ twg, int rev,
     const int* __restrict__ order, int* __restrict__ label, float* __restrict__ dist,
-    int* __restrict__ shift, int* __restrict__ changed, unsigned long long* __restrict__ evals) {
+    int* __restrict__ shift, int* __restrict__ changed, unsigned long long* __restrict__ evals,
+    const int* __restrict__ skip) {
+  if (skip && *skip) return;
   assign_prune_body<F, kPre>(blockIdx.x, gridDim.x, x, xs, xn, ubg, ub_ld, n, npairs, m, k, cspec, cmag, cnorm, twg, rev, order, label, dist, shift, changed, evals);
 }
 
@@ -1139,7 +1142,7 @@ static hipError_t launch_sbd_F(const SbdArgs& a, hipStream_t st) {
                      sbd_smem<F>(), st, a.x, a.n, a.m, a.k, kc, a.cspec, a.cnorm, a.tw, a.rev,
                      split ? a.part_label : a.label, split ? a.part_dist : a.dist,
                      split ? a.part_shift : a.shift, a.dmat, split ? nullptr : a.changed,
-                     a.ncc_out, a.fixed_label);
+                     a.ncc_out, a.fixed_label, a.skip);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !split) return e;
   hipLaunchKernelGGL(k_split_min, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, st,
@@ -1176,12 +1179,12 @@ static hipError_t launch_prune_F(const PruneArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((k_assign_prune<F, true>), dim3((unsigned)blocks), dim3(G::kBlock),
                        prune_smem<F>(a.k), st, a.x, a.xs, a.xn, a.ub, a.ub_ld, a.n, a.npairs, a.m,
                        a.k, a.cspec, a.cmag, a.cnorm, a.tw, a.rev, a.order, a.label, a.dist,
-                       a.shift, a.changed, a.evals);
+                       a.shift, a.changed, a.evals, a.skip);
   else
     hipLaunchKernelGGL((k_assign_prune<F, false>), dim3((unsigned)blocks), dim3(G::kBlock),
                        prune_smem<F>(a.k), st, a.x, nullptr, nullptr, nullptr, 0, a.n, a.npairs,
                        a.m, a.k, a.cspec, a.cmag, a.cnorm, a.tw, a.rev, a.order, a.label, a.dist,
-                       a.shift, a.changed, a.evals);
+                       a.shift, a.changed, a.evals, a.skip);
   return hipGetLastError();
 }
 

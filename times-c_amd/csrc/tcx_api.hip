@@ -49,15 +49,42 @@ using tcx::fail;
 // Workspace slots (grow-only device buffers held by the context).
 enum Slot {
   kSlotCspec, kSlotCnorm, kSlotCzero, kSlotLabel, kSlotShift, kSlotDist, kSlotCent,
-  kSlotCentNew, kSlotBlkCount, kSlotBlkBase, kSlotGroupInfo,
+  kSlotCentNew, kSlotBlkCount, kSlotBlkBase, kSlotStatus,
   kSlotPerm, kSlotYhi, kSlotYlo, kSlotA0, kSlotPlan, kSlotPart,
-  kSlotS, kSlotInfo, kSlotWbuf, kSlotRbuf, kSlotBar, kSlotVout, kSlotSteps,
-  kSlotConv, kSlotErr, kSlotCmag, kSlotEvals, kSlotSvout, kSlotLzW, kSlotLzState, kSlotMask,
+  kSlotS, kSlotWbuf, kSlotRbuf, kSlotBar, kSlotVout, kSlotSteps,
+  kSlotConv, kSlotErr, kSlotCmag, kSlotSvout, kSlotLzW, kSlotLzState, kSlotMask,
   kSlotRowStats, kSlotFitRowStats, kSlotKeyCounts, kSlotKeyOff, kSlotMinRow, kSlotXs, kSlotXn,
   kSlotLzXch, kSlotXm, kSlotUb, kSlotCm, kSlotCheck, kSlotCheckInfo, kSlotSplit, kNumSlots
 };
 
+// What a refinement leaves on the device for its caller to read back: one
+// buffer (kSlotStatus), copied at once.  The first 256 bytes are zeroed when it
+// starts.
+struct RefineStatus {
+  static constexpr size_t kEvals = 0;      // inverse transforms of the assignment
+  static constexpr size_t kChanged = 128;  // a label changed (another line: plain stores)
+  static constexpr size_t kRedo = 132;     // a cluster needs the eigenvector path
+  static constexpr size_t kBad = 136;      // a label was outside [0, k)
+  static constexpr size_t kPlan = 192;     // SyrkPlanHead
+  static constexpr size_t kInfo = sizeof(int) * tcx::kRefineStatusInts;
+  int k;
+  size_t offsets() const { return kInfo + sizeof(tcx::PowerInfo) * (size_t)k; }
+  size_t counts() const { return offsets() + sizeof(long) * ((size_t)k + 1); }
+  size_t bytes() const { return counts() + sizeof(int) * (size_t)k; }
+};
+
+// A refinement whose results the host has not looked at yet.
+struct PendingRefine {
+  bool on = false;
+  const float* S = nullptr;
+  const float* a0 = nullptr;
+  const int* counts = nullptr;
+  float* cout = nullptr;
+  int iter = 0, max_steps = 0;
+};
+
 struct FitState {
+  PendingRefine pending;
   bool active = false;
   const float* d_x = nullptr;
   int n = 0, m = 0, k = 0;
@@ -242,7 +269,7 @@ int assign_core_tw(tcx_ctx* c, const float2* tw, const float* d_x, long n, int m
                    const int* order = nullptr, long npairs = 0,
                    unsigned long long* evals = nullptr, const float2* xs = nullptr,
                    const float* xn = nullptr, const float* ub = nullptr, int ub_ld = 0,
-                   bool may_split = false) {
+                   bool may_split = false, const int* skip = nullptr) {
   const int F = fft_size(m);
   int chunks = 1;
   float* part = nullptr;
@@ -276,6 +303,7 @@ int assign_core_tw(tcx_ctx* c, const float2* tw, const float* d_x, long n, int m
     p.xn = xn;
     p.ub = ub;
     p.ub_ld = ub_ld;
+    p.skip = skip;
     TCX_HIP(tcx::launch_assign_prune(F, p, c->stream));
     return TCX_OK;
   }
@@ -284,6 +312,7 @@ int assign_core_tw(tcx_ctx* c, const float2* tw, const float* d_x, long n, int m
   a.rev = rev; a.label = label; a.dist = dist; a.shift = shift; a.dmat = dmat;
   a.changed = changed;
   a.chunks = chunks;
+  a.skip = skip;
   if (part) {
     a.part_dist = part;
     a.part_label = reinterpret_cast<int*>(part + (size_t)chunks * n);
@@ -300,12 +329,13 @@ int assign_core(tcx_ctx* c, const float* d_x, long n, int m, int k, const float2
                 int* changed, const int* order = nullptr, long npairs = 0,
                 unsigned long long* evals = nullptr, const float* cmag = nullptr,
                 const float2* xs = nullptr, const float* xn = nullptr,
-                const float* ub = nullptr, int ub_ld = 0, bool may_split = false) {
+                const float* ub = nullptr, int ub_ld = 0, bool may_split = false,
+                const int* skip = nullptr) {
   const float2* tw;
   TCX_TRY(twiddles(c, fft_size(m), &tw));
   if (!cmag) cmag = reinterpret_cast<const float*>(c->slot_ptr[kSlotCmag]);
   return assign_core_tw(c, tw, d_x, n, m, k, cspec, cnorm, cmag, rev, label, dist, shift, dmat,
-                        changed, order, npairs, evals, xs, xn, ub, ub_ld, may_split);
+                        changed, order, npairs, evals, xs, xn, ub, ub_ld, may_split, skip);
 }
 
 // ------------------------------------------------ allocation-free assignment
@@ -363,7 +393,6 @@ int noalloc_scratch(int dev, unsigned char** out) {
 // (summed in chunk order); returns their total count.
 long plan_syrk(int m, int k, const long* off, const long* seg_len, int cus,
                std::vector<tcx::SyrkGroup>& groups, std::vector<tcx::SyrkCluster>& clusters) {
-  constexpr long kXcds = 8, kMinSteps = 16;
   const long T = (m + tcx::kSyrkSub - 1) / tcx::kSyrkSub, U = T * (T + 1) / 2;  // waves per group
   groups.clear();
   clusters.clear();
@@ -374,15 +403,13 @@ long plan_syrk(int m, int k, const long* off, const long* seg_len, int cus,
     max_steps = std::max(max_steps, steps[j]);
   }
   if (max_steps == 0) return 0;
-  const long slots = 4L * std::max(cus, 1);  // one wave per SIMD
-  const long per_xcd = std::max(slots / kXcds, 1L);
-  const long gmax = U <= per_xcd ? kXcds * (per_xcd / U) : std::max(slots / U, 1L);
+  const long gmax = tcx::syrk_max_groups(m, cus);
   auto groups_for = [&](long L) {
     long g = 0;
     for (int j = 0; j < k; ++j) g += (steps[j] + L - 1) / L;
     return g;
   };
-  long lo = std::min(kMinSteps, max_steps), hi = max_steps;
+  long lo = std::min<long>(tcx::kSyrkMinSteps, max_steps), hi = max_steps;
   while (lo < hi) {  // shortest chunk bound whose groups fit (else one chunk per cluster)
     const long mid = (lo + hi) / 2;
     if (groups_for(mid) <= gmax) hi = mid; else lo = mid + 1;
@@ -548,12 +575,70 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
   return TCX_OK;
 }
 
+// The clusters whose power result failed its tests (h_info) through the
+// eigenvector path: their centroids and infos rewritten.  Waits.
+int refine_redo(tcx_ctx* c, const float* S, int m, int k, const int* counts, const float* a0,
+                uint64_t seed, int iter, int max_steps, double tol, float* d_cout,
+                tcx::PowerInfo* d_info, std::vector<tcx::PowerInfo>& h_info) {
+  hipStream_t st = c->stream;
+  std::vector<int> redo(k, 0);
+  bool any = false;
+  for (int j = 0; j < k; ++j)
+    if (h_info[j].fallback && !h_info[j].empty && !h_info[j].zero) {
+      redo[j] = 1;
+      any = true;
+    }
+  if (!any) return TCX_OK;
+  int* d_mask;
+  TCX_TRY(ws(c, kSlotMask, (size_t)k, &d_mask));
+  TCX_HIP(hipMemcpyAsync(d_mask, redo.data(), sizeof(int) * k, hipMemcpyHostToDevice, st));
+  const double *vin, *svin, *rsum;
+  const int *steps_in, *conv_in;
+  TCX_TRY(power_lanczos(c, S, m, k, counts, seed, iter, max_steps, 1, d_mask, &vin, &svin, &rsum,
+                        &steps_in, &conv_in));
+  TCX_HIP(tcx::launch_power(S, m, k, counts, a0, seed, iter, max_steps, tol, vin, svin, rsum,
+                            steps_in, conv_in, 1, d_mask, 0, d_cout, d_info, nullptr, st));
+  void* pin;
+  TCX_TRY(pinned_area(c, sizeof(tcx::PowerInfo) * k, &pin));
+  TCX_HIP(hipMemcpyAsync(pin, d_info, sizeof(tcx::PowerInfo) * k, hipMemcpyDeviceToHost, st));
+  TCX_HIP(hipStreamSynchronize(st));
+  const tcx::PowerInfo* p = static_cast<const tcx::PowerInfo*>(pin);
+  h_info.assign(p, p + k);
+  return TCX_OK;
+}
+
+// Reads a refinement's status from its copy at `h`: TCX_ERR_ARG for a bad
+// label, the non-empty clusters, the infos.
+int read_status(const unsigned char* h, int k, RefineResult* res,
+                std::vector<tcx::PowerInfo>& info) {
+  const RefineStatus rs{k};
+  if (*reinterpret_cast<const int*>(h + RefineStatus::kBad))
+    return fail(TCX_ERR_ARG, "label outside [0, k)");
+  const int* counts = reinterpret_cast<const int*>(h + rs.counts());
+  res->sum_class = 0;
+  for (int j = 0; j < k; ++j) res->sum_class += counts[j] > 0;
+  const tcx::PowerInfo* p = reinterpret_cast<const tcx::PowerInfo*>(h + RefineStatus::kInfo);
+  info.assign(p, p + k);
+  return TCX_OK;
+}
+
+void count_steps(const std::vector<tcx::PowerInfo>& info, RefineResult* res) {
+  for (const tcx::PowerInfo& i : info) {
+    res->steps_max = std::max(res->steps_max, i.steps);
+    res->fallbacks += i.fallback;
+  }
+}
+
 // One refinement: group, align + pack, S, power iteration.  Reads the
 // labels, shifts and old-centroid zero flags; writes k*m new centroids.
+// With `pending` nothing is waited for: the caller reads the status
+// (read_status) at its own next wait, and reruns the clusters that failed
+// their tests (refine_redo) before it uses the centroids.
 int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_label,
            const int* d_shift, const int* d_czero, float* d_cout, int iter, uint64_t seed,
            int split, double tol, int cal_select, const double2* row_stats, RefineResult* res,
-           const float* d_dist = nullptr, float* d_check = nullptr) {
+           const float* d_dist = nullptr, float* d_check = nullptr,
+           PendingRefine* pending = nullptr) {
   hipStream_t st = c->stream;
   if (!row_stats && tcx::align_pack_uses_row_stats(m)) {
     double2* rs;
@@ -569,34 +654,30 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
   const int B = tcx::group_bins(n, k, d_dist != nullptr);
   const long K = (long)k * B;
   long nblk = (n + tcx::kGroupChunk - 1) / tcx::kGroupChunk;
-  int *blk_count, *blk_base, *counts, *kcounts, *minrow, *perm, *bad;
-  long *offsets, *koff;
+  int *blk_count, *blk_base, *kcounts, *minrow, *perm;
+  long* koff;
   TCX_TRY(ws(c, kSlotBlkCount, (size_t)(nblk * K), &blk_count));
   TCX_TRY(ws(c, kSlotBlkBase, (size_t)(nblk * K), &blk_base));
-  // cluster offsets (k + 1), counts (k) and the bad-label flag in one
-  // buffer, in the layout of the pinned readback below (one copy)
-  const size_t ginfo_bytes = sizeof(long) * (k + 1) + sizeof(int) * (k + 2);
-  unsigned char* ginfo;
-  TCX_TRY(ws(c, kSlotGroupInfo, ginfo_bytes, &ginfo));
-  offsets = reinterpret_cast<long*>(ginfo);
-  counts = reinterpret_cast<int*>(offsets + k + 1);
-  bad = counts + k;
+  const RefineStatus rs{k};
+  unsigned char* status;
+  TCX_TRY(ws(c, kSlotStatus, rs.bytes(), &status));
+  long* offsets = reinterpret_cast<long*>(status + rs.offsets());
+  int* counts = reinterpret_cast<int*>(status + rs.counts());
+  int* bad = reinterpret_cast<int*>(status + RefineStatus::kBad);
+  tcx::PowerInfo* info = reinterpret_cast<tcx::PowerInfo*>(status + RefineStatus::kInfo);
   TCX_TRY(ws(c, kSlotKeyCounts, (size_t)K, &kcounts));
   TCX_TRY(ws(c, kSlotKeyOff, (size_t)K, &koff));
   TCX_TRY(ws(c, kSlotMinRow, (size_t)k, &minrow));
-  TCX_HIP(tcx::launch_fill_int(bad, 1, 0, st));
-  TCX_HIP(tcx::launch_fill_int(minrow, k, 0x7fffffff, st));
-  TCX_HIP(tcx::launch_group_count(d_label, n, k, d_dist, B, blk_count, minrow, bad, st));
-  TCX_HIP(tcx::launch_group_scan((int)nblk, k, B, blk_count, blk_base, kcounts, counts, offsets,
-                                 koff, st));
-  // Placement and align + pack are launched before the host reads the
-  // cluster sizes, on buffers sized for the largest padded count
-  // (n + k * (kPackPad - 1)); their blocks past the padded end offsets[k]
-  // exit at once.  The host then plans S = Y^T Y while they run.
+  // Everything is sized for the largest padded count (n + k * (kPackPad -
+  // 1)); blocks past the padded end offsets[k] exit at once, and S = Y^T Y is
+  // planned on the device, so the host waits for nothing here.
   const long n_pad_max = std::max<long>(
       (n + (long)k * (tcx::kPackPad - 1)) / tcx::kPackPad * tcx::kPackPad, tcx::kPackPad);
   TCX_TRY(ws(c, kSlotPerm, (size_t)n_pad_max, &perm));
-  TCX_HIP(tcx::launch_fill_int(perm, n_pad_max, -1, st));
+  TCX_HIP(tcx::launch_refine_init(reinterpret_cast<int*>(status), minrow, k, perm, n_pad_max, st));
+  TCX_HIP(tcx::launch_group_count(d_label, n, k, d_dist, B, blk_count, minrow, bad, st));
+  TCX_HIP(tcx::launch_group_scan((int)nblk, k, B, blk_count, blk_base, kcounts, counts, offsets,
+                                 koff, st));
   TCX_HIP(tcx::launch_group_place(d_label, n, k, d_dist, B, blk_base, koff, perm, st));
   uint16_t *yhi, *ylo;
   float* a0;
@@ -607,52 +688,61 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
   TCX_TRY(ws(c, kSlotA0, (size_t)k * m, &a0));
   TCX_HIP(tcx::launch_align_pack(d_x, m, perm, n_pad_max, offsets, minrow, k, d_shift, d_czero,
                                  row_stats, yhi, ylo, a0, st));
-  void* pin;
-  TCX_TRY(pinned_area(c, ginfo_bytes, &pin));
-  long* p_off = static_cast<long*>(pin);
-  int* p_counts = reinterpret_cast<int*>(p_off + k + 1);
-  int* p_bad = p_counts + k;
-  TCX_HIP(hipMemcpyAsync(pin, ginfo, ginfo_bytes, hipMemcpyDeviceToHost, st));
-  TCX_HIP(hipStreamSynchronize(st));
-  // out-of-range labels were left out of the grouping above
-  if (*p_bad) return fail(TCX_ERR_ARG, "label outside [0, k)");
-  const std::vector<int> h_counts(p_counts, p_counts + k);
-  const std::vector<long> h_off(p_off, p_off + k + 1);
-  const long n_pad = h_off[k];
-  int nonempty = 0;
-  for (int j = 0; j < k; ++j) nonempty += h_counts[j] > 0;
-  std::vector<long> seg_len(k);
-  for (int j = 0; j < k; ++j) seg_len[j] = h_counts[j] > 0 ? h_off[j + 1] - h_off[j] : 0;
-  const long nparts =
-      plan_syrk(m, k, h_off.data(), seg_len.data(), c->cus, c->sgroups, c->sclusters);
-  // groups and clusters in one buffer, uploaded by one copy
-  const size_t groups_bytes = (sizeof(tcx::SyrkGroup) * c->sgroups.size() + 255) & ~(size_t)255;
-  const size_t plan_bytes = groups_bytes + sizeof(tcx::SyrkCluster) * c->sclusters.size();
+  // the plan: header, groups, clusters.  A chunk is at least kSyrkMinSteps
+  // steps but for one per cluster, and the groups fit one round of the device
+  // or are one per cluster.
+  const long T = (m + tcx::kSyrkSub - 1) / tcx::kSyrkSub, U = T * (T + 1) / 2;
+  long max_groups = std::min<long>(std::max<long>(tcx::syrk_max_groups(m, c->cus), k),
+                                   n_pad_max / (16 * tcx::kSyrkMinSteps) + k);
+  // Where a budget might have no room for the largest plan beside the rest
+  // (counted as if nothing of it were there yet), the sizes are read back and
+  // the plan is made on the host, with what it needs.
+  const size_t sub = sizeof(float) * tcx::kSyrkSub * tcx::kSyrkSub;
+  const bool host_plan = c->budget && c->ws_bytes + c->user_bytes + sub * (size_t)(max_groups * U) +
+                                              tcx::fit_workspace_bound(n, m, k, c->cus) >
+                                          c->budget;
+  long nparts = max_groups * U;
+  if (host_plan) {
+    void* pin;
+    TCX_TRY(pinned_area(c, rs.bytes(), &pin));
+    TCX_HIP(hipMemcpyAsync(pin, status, rs.bytes(), hipMemcpyDeviceToHost, st));
+    TCX_HIP(hipStreamSynchronize(st));
+    const unsigned char* h = static_cast<unsigned char*>(pin);
+    if (*reinterpret_cast<const int*>(h + RefineStatus::kBad))
+      return fail(TCX_ERR_ARG, "label outside [0, k)");
+    const long* h_off = reinterpret_cast<const long*>(h + rs.offsets());
+    const int* h_counts = reinterpret_cast<const int*>(h + rs.counts());
+    std::vector<long> seg_len(k);
+    for (int j = 0; j < k; ++j) seg_len[j] = h_counts[j] > 0 ? h_off[j + 1] - h_off[j] : 0;
+    nparts = plan_syrk(m, k, h_off, seg_len.data(), c->cus, c->sgroups, c->sclusters);
+    max_groups = (long)c->sgroups.size();
+  }
+  auto* d_head = reinterpret_cast<tcx::SyrkPlanHead*>(status + RefineStatus::kPlan);
+  const size_t groups_bytes =
+      (sizeof(tcx::SyrkGroup) * (size_t)std::max(max_groups, 1L) + 255) & ~(size_t)255;
+  const size_t plan_bytes =
+      groups_bytes + sizeof(tcx::SyrkCluster) * (host_plan ? c->sclusters.size() : (size_t)k);
   unsigned char* d_plan;
   TCX_TRY(ws(c, kSlotPlan, plan_bytes, &d_plan));
-  tcx::SyrkGroup* d_groups = reinterpret_cast<tcx::SyrkGroup*>(d_plan);
-  tcx::SyrkCluster* d_clusters = reinterpret_cast<tcx::SyrkCluster*>(d_plan + groups_bytes);
+  auto* d_groups = reinterpret_cast<tcx::SyrkGroup*>(d_plan);
+  auto* d_clusters = reinterpret_cast<tcx::SyrkCluster*>(d_plan + groups_bytes);
   float *part, *S;
-  tcx::PowerInfo* info;
   TCX_TRY(ws(c, kSlotPart, (size_t)std::max(nparts, 1L) * tcx::kSyrkSub * tcx::kSyrkSub, &part));
   TCX_TRY(ws(c, kSlotS, (size_t)k * m * m, &S));
-  TCX_TRY(ws(c, kSlotInfo, (size_t)k, &info));
-  const int ngroups = (int)c->sgroups.size(), nclusters = (int)c->sclusters.size();
-  if (ngroups > 0) {
-    // staged in the pinned area (idle here: its readback above was waited
-    // for and consumed; its next use, the power stage's readback, is ordered
-    // after this copy on the same stream and is sized in now, so the area is
-    // not regrown while the copy reads it), so the copy does not block the
-    // host
-    void* stage;
-    TCX_TRY(pinned_area(c, std::max(plan_bytes, sizeof(tcx::PowerInfo) * k), &stage));
-    unsigned char* h_plan = static_cast<unsigned char*>(stage);
-    std::memcpy(h_plan, c->sgroups.data(), sizeof(tcx::SyrkGroup) * ngroups);
-    std::memcpy(h_plan + groups_bytes, c->sclusters.data(), sizeof(tcx::SyrkCluster) * nclusters);
-    TCX_HIP(hipMemcpyAsync(d_plan, h_plan, plan_bytes, hipMemcpyHostToDevice, st));
+  if (host_plan) {
+    const tcx::SyrkPlanHead head{(int)c->sgroups.size(), (int)c->sclusters.size()};
+    TCX_HIP(hipMemcpyAsync(d_head, &head, sizeof(head), hipMemcpyHostToDevice, st));
+    TCX_HIP(hipMemcpyAsync(d_groups, c->sgroups.data(),
+                           sizeof(tcx::SyrkGroup) * c->sgroups.size(), hipMemcpyHostToDevice, st));
+    TCX_HIP(hipMemcpyAsync(d_clusters, c->sclusters.data(),
+                           sizeof(tcx::SyrkCluster) * c->sclusters.size(), hipMemcpyHostToDevice,
+                           st));
+    TCX_HIP(hipStreamSynchronize(st));
+  } else {
+    TCX_HIP(tcx::launch_syrk_plan(offsets, counts, m, k, c->cus, d_head, d_groups, d_clusters, st));
   }
-  TCX_HIP(tcx::launch_syrk(d_groups, ngroups, yhi, ylo, m, split, part, st));
-  TCX_HIP(tcx::launch_syrk_reduce(d_clusters, nclusters, part, m, S, st));
+  TCX_HIP(tcx::launch_syrk(d_groups, d_head, (int)max_groups, yhi, ylo, m, split, part, st));
+  TCX_HIP(tcx::launch_syrk_reduce(d_clusters, d_head, k, part, m, S, st));
   const int max_steps = m > 1000 ? 1000 : m;  // test_timesC.py:152-156
   const double* vin = nullptr;
   const double* svin = nullptr;
@@ -663,50 +753,40 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
   // test_timesC.py:184-192); 0: the power iterate, with the clusters that fail the
   // power result's tests rerun through the eigenvector path.
   const int mode = cal_select == 1 ? 1 : 0;
-  if (nonempty > 0)
-    TCX_TRY(power_lanczos(c, S, m, k, counts, seed, iter, max_steps, mode, nullptr, &vin, &svin,
-                          &rsum, &steps_in, &conv_in));
+  TCX_TRY(power_lanczos(c, S, m, k, counts, seed, iter, max_steps, mode, nullptr, &vin, &svin,
+                        &rsum, &steps_in, &conv_in));
   TCX_HIP(tcx::launch_power(S, m, k, counts, a0, seed, iter, max_steps, tol, vin, svin, rsum,
-                            steps_in, conv_in, mode, nullptr, 1, d_cout, info, st));
-  TCX_TRY(pinned_area(c, sizeof(tcx::PowerInfo) * k, &pin));
-  tcx::PowerInfo* p_info = static_cast<tcx::PowerInfo*>(pin);
-  TCX_HIP(hipMemcpyAsync(p_info, info, sizeof(tcx::PowerInfo) * k, hipMemcpyDeviceToHost, st));
-  TCX_HIP(hipStreamSynchronize(st));
-  std::vector<tcx::PowerInfo> h_info(p_info, p_info + k);
-  if (mode == 0) {
-    std::vector<int> redo(k, 0);
-    bool any = false;
-    for (int j = 0; j < k; ++j)
-      if (h_info[j].fallback && !h_info[j].empty && !h_info[j].zero) {
-        redo[j] = 1;
-        any = true;
-      }
-    if (any) {
-      int* d_mask;
-      TCX_TRY(ws(c, kSlotMask, (size_t)k, &d_mask));
-      TCX_HIP(hipMemcpyAsync(d_mask, redo.data(), sizeof(int) * k, hipMemcpyHostToDevice, st));
-      TCX_TRY(power_lanczos(c, S, m, k, counts, seed, iter, max_steps, 1, d_mask, &vin, &svin,
-                            &rsum, &steps_in, &conv_in));
-      TCX_HIP(tcx::launch_power(S, m, k, counts, a0, seed, iter, max_steps, tol, vin, svin, rsum,
-                                steps_in, conv_in, 1, d_mask, 0, d_cout, info, st));
-      TCX_HIP(hipMemcpyAsync(p_info, info, sizeof(tcx::PowerInfo) * k, hipMemcpyDeviceToHost,
-                             st));
-      TCX_HIP(hipStreamSynchronize(st));
-      h_info.assign(p_info, p_info + k);
-    }
+                            steps_in, conv_in, mode, nullptr, 1, d_cout, info,
+                            mode == 0 ? reinterpret_cast<int*>(status + RefineStatus::kRedo)
+                                      : nullptr,
+                            st));
+  if (res) res->n_pad = n_pad_max;
+  if (pending) {
+    *pending = PendingRefine{true, S, a0, counts, d_cout, iter, max_steps};
+    return TCX_OK;
   }
+  void* pin;
+  TCX_TRY(pinned_area(c, rs.bytes(), &pin));
+  TCX_HIP(hipMemcpyAsync(pin, status, rs.bytes(), hipMemcpyDeviceToHost, st));
+  TCX_HIP(hipStreamSynchronize(st));
+  RefineResult seen;
+  std::vector<tcx::PowerInfo> h_info;
+  TCX_TRY(read_status(static_cast<unsigned char*>(pin), k, &seen, h_info));
+  const int nonempty = seen.sum_class;
+  if (mode == 0)
+    TCX_TRY(refine_redo(c, S, m, k, counts, a0, seed, iter, max_steps, tol, d_cout, info, h_info));
   if (d_check && nonempty > 0) {
     // the budget check of TCX_S_AUTO: the same S from one BF16 product (the
     // hi panel only) through the same power stage; the largest relative L2
     // difference between its centroids and the split ones above
-    TCX_HIP(tcx::launch_syrk(d_groups, ngroups, yhi, ylo, m, 0, part, st));
-    TCX_HIP(tcx::launch_syrk_reduce(d_clusters, nclusters, part, m, S, st));
+    TCX_HIP(tcx::launch_syrk(d_groups, d_head, (int)max_groups, yhi, ylo, m, 0, part, st));
+    TCX_HIP(tcx::launch_syrk_reduce(d_clusters, d_head, k, part, m, S, st));
     TCX_TRY(power_lanczos(c, S, m, k, counts, seed, iter, max_steps, 0, nullptr, &vin, &svin,
                           &rsum, &steps_in, &conv_in));
     tcx::PowerInfo* cinfo;
     TCX_TRY(ws(c, kSlotCheckInfo, (size_t)k, &cinfo));
     TCX_HIP(tcx::launch_power(S, m, k, counts, a0, seed, iter, max_steps, tol, vin, svin, rsum,
-                              steps_in, conv_in, 0, nullptr, 1, d_check, cinfo, st));
+                              steps_in, conv_in, 0, nullptr, 1, d_check, cinfo, nullptr, st));
     const size_t cb = sizeof(float) * (size_t)k * m;
     TCX_TRY(pinned_area(c, 2 * cb + sizeof(tcx::PowerInfo) * k, &pin));
     float* h_split = static_cast<float*>(pin);
@@ -734,12 +814,8 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
     if (res) res->check_err = err;
   }
   if (res) {
-    res->n_pad = n_pad;
     res->sum_class = nonempty;
-    for (int j = 0; j < k; ++j) {
-      res->steps_max = std::max(res->steps_max, h_info[j].steps);
-      res->fallbacks += h_info[j].fallback;
-    }
+    count_steps(h_info, res);
   }
   return TCX_OK;
 }
@@ -887,7 +963,7 @@ size_t fit_workspace_bound(long n, int m, int k, int cus) {
   // grouping (with distances: the most bins)
   const size_t B = (size_t)group_bins(n, k, true), keys = Kc * B;
   const size_t nblk = (N + kGroupChunk - 1) / kGroupChunk;
-  b += 2 * r(4 * nblk * keys) + r(8 * (Kc + 1) + 4 * (Kc + 2)) + r(4 * keys) + r(8 * keys) +
+  b += 2 * r(4 * nblk * keys) + r(4 * keys) + r(8 * keys) +
        r(4 * Kc);
   // row order, Y panels (hi, lo), sign-fix rows
   const size_t npad = std::max<size_t>((N + Kc * (kPackPad - 1)) / kPackPad * kPackPad, kPackPad);
@@ -901,13 +977,13 @@ size_t fit_workspace_bound(long n, int m, int k, int cus) {
       std::min(std::max((size_t)4 * std::max(cus, 1) / U + 8, Kc), npad / 256 + Kc);
   const size_t nparts = groups * U;
   b += r(sizeof(SyrkGroup) * groups + 256 + sizeof(SyrkCluster) * Kc);
-  b += r(4 * nparts * kSyrkSub * kSyrkSub) + r(4 * Kc * Mm * Mm) + r(sizeof(PowerInfo) * Kc);
+  b += r(4 * nparts * kSyrkSub * kSyrkSub) + r(4 * Kc * Mm * Mm);
   // power stage: basis, v, S v, r, w, counters, states, exchange words, mask
   const size_t xch = Kc * (2 * (2 * (size_t)kLzCoopMaxG * (kLanczosMax + 2) + Mm) + kLzCoopMaxG);
   b += r(8 * Kc * (kLanczosMax + 1) * Mm) + 4 * r(8 * Kc * Mm) + 2 * r(4 * Kc) +
        r(sizeof(LzState) * Kc) + r(8 * xch + 4 * (Kc + 1)) + r(4 * Kc);
-  // evaluation count and changed flag; twiddles
-  b += r(8 * 17) + 8 * F;
+  // status and sizes; twiddles
+  b += r(RefineStatus{k}.bytes()) + 8 * F;
   return b;
 }
 
@@ -1309,9 +1385,13 @@ int fit_refine(tcx_ctx* c, FitState& f) {
     TCX_TRY(ws(c, kSlotCheck, (size_t)f.k * f.m, &check));
   TCX_HIP(hipEventRecord(c->ev[0], st));
   RefineResult rr;
+  // With the random-label start the assignment follows at once and its wait
+  // serves the refinement too (fit_assign), unless the number of clusters
+  // left or the precision check is wanted first.
+  const bool defer = f.o.init_mode == 0 && !f.o.stop_on_collapse && !check && f.o.cal_select == 0;
   TCX_TRY(refine(c, f.d_x, f.n, f.m, f.k, f.label, f.shift, f.zero, cnew, f.it, f.o.seed,
                  f.split, f.tol, f.o.cal_select, f.row_stats, &rr,
-                 f.have_dist ? f.dist : nullptr, check));
+                 f.have_dist ? f.dist : nullptr, check, defer ? &f.pending : nullptr));
   if (check) {
     ++f.s_checks;
     f.s_check_err = rr.check_err;
@@ -1327,55 +1407,98 @@ int fit_refine(tcx_ctx* c, FitState& f) {
   TCX_TRY(spectra(c, f.cent, f.k, f.m, &f.spec, &f.norm, &f.zero, f.cm));
   TCX_HIP(hipEventRecord(c->ev[1], st));
   f.ref_timed = true;  // read at the next synchronization (fit_assign)
-  f.sum_class = rr.sum_class;
   f.n_pad = rr.n_pad;
   f.have_order = true;
-  f.steps_max = std::max(f.steps_max, rr.steps_max);
-  f.fallbacks += rr.fallbacks;
+  if (!f.pending.on) {
+    f.sum_class = rr.sum_class;
+    f.steps_max = std::max(f.steps_max, rr.steps_max);
+    f.fallbacks += rr.fallbacks;
+  }
   return TCX_OK;
+}
+
+// Bounds and assignment of every series, launched (nothing is done when
+// *skip).
+int launch_fit_assign(tcx_ctx* c, FitState& f, unsigned char* status, const int* skip) {
+  hipStream_t st = c->stream;
+  const int* order = f.have_order ? reinterpret_cast<const int*>(c->slot_ptr[kSlotPerm]) : nullptr;
+  if (f.xs) TCX_HIP(tcx::launch_bounds(fft_size(f.m), f.xm, f.n, f.cm, f.k, f.ub, f.ub_ld, st));
+  TCX_HIP(hipEventRecord(c->ev[4], st));
+  return assign_core(c, f.d_x, f.n, f.m, f.k, f.spec, f.norm, f.o.convention, f.label, f.dist,
+                     f.shift, nullptr, reinterpret_cast<int*>(status + RefineStatus::kChanged),
+                     order, f.n_pad / 2,
+                     reinterpret_cast<unsigned long long*>(status + RefineStatus::kEvals), nullptr,
+                     f.xs, f.xn, f.ub, f.ub_ld, false, skip);
 }
 
 int fit_assign(tcx_ctx* c, FitState& f, int* h_changed) {
   hipStream_t st = c->stream;
-  // the evaluation count and the labels-changed flag in one buffer (one
-  // fill, one readback), on different 128-byte lines: the count takes an
-  // atomic add per block, the flag plain stores
-  constexpr int kChangedAt = 128 / sizeof(unsigned long long);
-  unsigned long long* evals;
-  TCX_TRY(ws(c, kSlotEvals, kChangedAt + 1, &evals));
-  int* changed = reinterpret_cast<int*>(evals + kChangedAt);
-  TCX_HIP(tcx::launch_fill_int(reinterpret_cast<int*>(evals), 2 * (kChangedAt + 1), 0, st));
-  TCX_HIP(hipEventRecord(c->ev[2], st));
-  const int* order = f.have_order ? reinterpret_cast<const int*>(c->slot_ptr[kSlotPerm]) : nullptr;
-  if (f.xs) TCX_HIP(tcx::launch_bounds(fft_size(f.m), f.xm, f.n, f.cm, f.k, f.ub, f.ub_ld, st));
-  TCX_HIP(hipEventRecord(c->ev[4], st));
-  TCX_TRY(assign_core(c, f.d_x, f.n, f.m, f.k, f.spec, f.norm, f.o.convention, f.label, f.dist,
-                      f.shift, nullptr, changed, order, f.n_pad / 2, evals, nullptr, f.xs,
-                      f.xn, f.ub, f.ub_ld));
-  f.have_dist = true;
+  const RefineStatus rs{f.k};
+  unsigned char* status;
+  TCX_TRY(ws(c, kSlotStatus, rs.bytes(), &status));
+  const bool pending = f.pending.on;
+  f.pending.on = false;
+  // the evaluation count and the labels-changed flag are zero since the
+  // refinement before started, unless an assignment has used them since
+  if (!pending)
+    TCX_HIP(tcx::launch_fill_int(reinterpret_cast<int*>(status), tcx::kRefineStatusInts, 0, st));
+  const int* redo = pending ? reinterpret_cast<int*>(status + RefineStatus::kRedo) : nullptr;
+  if (!pending) TCX_HIP(hipEventRecord(c->ev[2], st));  // else ev[1] is the same moment
+  TCX_TRY(launch_fit_assign(c, f, status, redo));
   TCX_HIP(hipEventRecord(c->ev[3], st));
   void* pin;
-  TCX_TRY(pinned_area(c, sizeof(unsigned long long) * (kChangedAt + 1), &pin));
-  unsigned long long* p_evals = static_cast<unsigned long long*>(pin);
-  int* p_changed = reinterpret_cast<int*>(p_evals + kChangedAt);
-  TCX_HIP(hipMemcpyAsync(p_evals, evals, sizeof(*p_evals) * kChangedAt + sizeof(int),
-                         hipMemcpyDeviceToHost, st));
-  if (f.o.labels_per_iter && f.it < f.o.max_iter)
-    TCX_HIP(hipMemcpyAsync(f.o.labels_per_iter + (size_t)f.it * f.n, f.label,
-                           sizeof(int) * f.n, hipMemcpyDeviceToHost, st));
+  TCX_TRY(pinned_area(c, rs.bytes(), &pin));
+  unsigned char* h = static_cast<unsigned char*>(pin);
+  const size_t bytes = pending ? rs.bytes() : RefineStatus::kInfo;
+  auto copy_labels = [&]() -> int {
+    if (f.o.labels_per_iter && f.it < f.o.max_iter)
+      TCX_HIP(hipMemcpyAsync(f.o.labels_per_iter + (size_t)f.it * f.n, f.label,
+                             sizeof(int) * f.n, hipMemcpyDeviceToHost, st));
+    return TCX_OK;
+  };
+  TCX_HIP(hipMemcpyAsync(h, status, bytes, hipMemcpyDeviceToHost, st));
+  TCX_TRY(copy_labels());
   TCX_HIP(hipStreamSynchronize(st));
-  *h_changed = *p_changed;
-  const unsigned long long h_evals = *p_evals;
+  hipEvent_t begin = pending ? c->ev[1] : c->ev[2];
+  if (pending) {
+    RefineResult rr;
+    std::vector<tcx::PowerInfo> info;
+    TCX_TRY(read_status(h, f.k, &rr, info));
+    if (*reinterpret_cast<const int*>(h + RefineStatus::kRedo)) {
+      // clusters for the eigenvector path: the assignment did nothing; rerun
+      // them, then the spectra and the assignment
+      const PendingRefine& p = f.pending;
+      TCX_TRY(refine_redo(c, p.S, f.m, f.k, p.counts, p.a0, f.o.seed, p.iter, p.max_steps, f.tol,
+                          p.cout, reinterpret_cast<tcx::PowerInfo*>(status + RefineStatus::kInfo),
+                          info));
+      TCX_TRY(spectra(c, f.cent, f.k, f.m, &f.spec, &f.norm, &f.zero, f.cm));
+      TCX_HIP(hipEventRecord(c->ev[1], st));
+      TCX_TRY(launch_fit_assign(c, f, status, nullptr));
+      TCX_HIP(hipEventRecord(c->ev[3], st));
+      TCX_TRY(pinned_area(c, rs.bytes(), &pin));
+      h = static_cast<unsigned char*>(pin);
+      TCX_HIP(hipMemcpyAsync(h, status, RefineStatus::kInfo, hipMemcpyDeviceToHost, st));
+      TCX_TRY(copy_labels());
+      TCX_HIP(hipStreamSynchronize(st));
+    }
+    count_steps(info, &rr);
+    f.sum_class = rr.sum_class;
+    f.steps_max = std::max(f.steps_max, rr.steps_max);
+    f.fallbacks += rr.fallbacks;
+  }
+  f.have_dist = true;
+  *h_changed = *reinterpret_cast<const int*>(h + RefineStatus::kChanged);
+  const auto h_evals = *reinterpret_cast<const unsigned long long*>(h + RefineStatus::kEvals);
   float ms = 0.f;
   if (f.ref_timed) {
     TCX_HIP(hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
     f.ms_ref += ms;
     f.ref_timed = false;
   }
-  TCX_HIP(hipEventElapsedTime(&ms, c->ev[2], c->ev[3]));
+  TCX_HIP(hipEventElapsedTime(&ms, begin, c->ev[3]));
   f.ms_asg += ms;
   f.ms_asg_last = ms;
-  TCX_HIP(hipEventElapsedTime(&ms, c->ev[2], c->ev[4]));
+  TCX_HIP(hipEventElapsedTime(&ms, begin, c->ev[4]));
   f.ms_bnd += ms;
   f.evals += (long long)h_evals;
   f.pairs += (long long)f.n * f.k;

@@ -31,6 +31,7 @@ struct SbdArgs {
   float* part_dist = nullptr;
   int* part_label = nullptr;
   int* part_shift = nullptr;
+  const int* skip = nullptr;     // assign: nothing is done when *skip (may be NULL)
 };
 
 // largest supported FFT length (m <= 4096)
@@ -85,6 +86,7 @@ struct PruneArgs {
   int* shift = nullptr;
   int* changed = nullptr;
   unsigned long long* evals = nullptr;  // inverse transforms run (may be NULL)
+  const int* skip = nullptr;     // nothing is done when *skip (may be NULL)
 };
 hipError_t launch_assign_prune(int F, const PruneArgs& a, hipStream_t st);
 // Half spectra X_r[0 .. F/2] of every row and the row norms (k_series_spec);
@@ -152,6 +154,11 @@ struct SyrkGroup {
 struct SyrkCluster {
   int cluster, part0, nparts;
 };
+struct SyrkPlanHead {
+  int ngroups, nclusters;  // clusters: those with members
+};
+constexpr int kSyrkMinSteps = 16;  // 16-column steps of a K chunk, at least
+int syrk_max_groups(int m, int cus);  // groups of one round of the device
 
 struct PowerInfo {
   double lambda;
@@ -189,15 +196,29 @@ hipError_t launch_align_pack(const float* x, int m, const int* perm, long n_pad,
 // one XCD), the launch over the groups, and the reduction of the clusters'
 // kSyrkSub x kSyrkSub partials into S.
 long syrk_blocks(int m, int ngroups);
-hipError_t launch_syrk(const SyrkGroup* groups, int ngroups, const uint16_t* yhi,
-                       const uint16_t* ylo, int m, int split, float* part, hipStream_t st);
-hipError_t launch_syrk_reduce(const SyrkCluster* clusters, int nclusters, const float* part, int m,
-                              float* S, hipStream_t st);
+// The first kRefineStatusInts ints of a refinement's status zeroed, minrow
+// INT_MAX, perm -1.
+constexpr int kRefineStatusInts = 64;
+hipError_t launch_refine_init(int* status, int* minrow, int k, int* perm, long n_pad,
+                              hipStream_t st);
+// The plan of S from the clusters' sizes on the device.
+hipError_t launch_syrk_plan(const long* offsets, const int* counts, int m, int k, int cus,
+                            SyrkPlanHead* head, SyrkGroup* groups, SyrkCluster* clusters,
+                            hipStream_t st);
+// max_groups, max_clusters: at least the plan's counts (the grid's size).
+hipError_t launch_syrk(const SyrkGroup* groups, const SyrkPlanHead* head, int max_groups,
+                       const uint16_t* yhi, const uint16_t* ylo, int m, int split, float* part,
+                       hipStream_t st);
+hipError_t launch_syrk_reduce(const SyrkCluster* clusters, const SyrkPlanHead* head,
+                              int max_clusters, const float* part, int m, float* S,
+                              hipStream_t st);
+// redo (may be NULL): set to 1 when a cluster failed its tests and
+// defer_fallback left it to the caller.
 hipError_t launch_power(const float* S, int m, int k, const int* counts, const float* a0,
                         uint64_t seed, int iter, int max_steps, double tol, const double* vin,
                         const double* svin, const double* rsum, const int* steps_in,
                         const int* conv_in, int eig_mode, const int* mask, int defer_fallback,
-                        float* c_out, PowerInfo* info, hipStream_t st);
+                        float* c_out, PowerInfo* info, int* redo, hipStream_t st);
 
 // Lanczos evaluation of the power iterate M^I v0 (one block per cluster).
 // Lanczos evaluation of the power iterate (one step = two launches).
