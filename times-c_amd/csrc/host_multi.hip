@@ -75,7 +75,7 @@ double ms_between(Clock::time_point a, Clock::time_point b) {
 
 // Readback layout of a job's grouping (offsets, counts, bad-label flag).
 size_t ginfo_bytes(int k) { return align_up(sizeof(long) * (k + 1) + sizeof(int) * (k + 2)); }
-constexpr size_t kEvcBytes = 256;  // evaluation count (8 B), changed flag at +128
+constexpr size_t kEvcBytes = kEvalBytes + 128;  // evaluation counters, changed flag
 
 struct GJob {
   tcx_job* job = nullptr;
@@ -344,7 +344,7 @@ struct Batch {
   unsigned long long* evals(GJob& j) {
     return reinterpret_cast<unsigned long long*>(evc_d + j.evc_off);
   }
-  int* changed(GJob& j) { return reinterpret_cast<int*>(evc_d + j.evc_off + 128); }
+  int* changed(GJob& j) { return reinterpret_cast<int*>(evc_d + j.evc_off + kEvalBytes); }
 };
 
 // ----------------------------------------------------------------- setup
@@ -1106,9 +1106,8 @@ int grouped_fit(tcx_ctx* ctx, tcx_job* jobs, const int* idx, int count, size_t h
     for (GJob* j : act) {
       if (!j->collapsed) {
         j->ms_assign += ms_between(tb, tc);
-        const unsigned long long ev =
-            *reinterpret_cast<const unsigned long long*>(b.evc_h + j->evc_off);
-        const int ch = *reinterpret_cast<const int*>(b.evc_h + j->evc_off + 128);
+        const unsigned long long ev = eval_sum(b.evc_h + j->evc_off);
+        const int ch = *reinterpret_cast<const int*>(b.evc_h + j->evc_off + kEvalBytes);
         j->evals += (long long)ev;
         j->pairs += (long long)j->n * j->k;
         j->have_dist = true;

@@ -39,7 +39,7 @@ __global__ void k_fill_int(int* p, long count, int value) {
 __global__ __launch_bounds__(256) void k_refine_init(int* status, int* __restrict__ minrow, int k,
                                                      int* __restrict__ perm, long n_pad) {
   const long i0 = (long)blockIdx.x * 256 + threadIdx.x, step = (long)gridDim.x * 256;
-  if (i0 < kRefineStatusInts) status[i0] = 0;
+  for (long i = i0; i < kRefineStatusInts; i += step) status[i] = 0;
   for (long i = i0; i < k; i += step) minrow[i] = 0x7fffffff;
   for (long i = i0; i < n_pad; i += step) perm[i] = -1;
 }

@@ -776,7 +776,7 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
   const int g = threadIdx.x / L, lane = threadIdx.x % L;
   float2* buf = smem + fft_tw_lds<F>() + g * fft_buf_len<F>();
   float* ubs = ubs_all + (long)g * 2 * k;  // [0,k): series a, [k,2k): series b
-  unsigned long long my_evals = 0;
+  unsigned my_evals = 0;
   for (long pr = (long)bid * G::kGroups + g; pr < npairs;
        pr += (long)nblk * G::kGroups) {
     long ia = order ? order[2 * pr] : 2 * pr;
@@ -946,7 +946,13 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
       }
     }
   }
-  if (evals && lane == 0 && my_evals) atomicAdd(evals, my_evals);
+  if (evals) {  // one add per wave (a group of several waves: of its first)
+    unsigned v = lane == 0 ? my_evals : 0;
+#pragma unroll
+    for (int o = L; o < kWave; o *= 2) v += __shfl_xor(v, o);
+    if (threadIdx.x % (L < kWave ? kWave : L) == 0 && v)
+      atomicAdd(evals + (bid % kEvalSlots) * kEvalStride, (unsigned long long)v);
+  }
 }
 
 template <int F, bool kPre>

@@ -58,14 +58,14 @@ enum Slot {
 };
 
 // What a refinement leaves on the device for its caller to read back: one
-// buffer (kSlotStatus), copied at once.  The first 256 bytes are zeroed when it
-// starts.
+// buffer (kSlotStatus), copied at once.  The bytes before kInfo are zeroed when
+// it starts.
 struct RefineStatus {
-  static constexpr size_t kEvals = 0;      // inverse transforms of the assignment
-  static constexpr size_t kChanged = 128;  // a label changed (another line: plain stores)
-  static constexpr size_t kRedo = 132;     // a cluster needs the eigenvector path
-  static constexpr size_t kBad = 136;      // a label was outside [0, k)
-  static constexpr size_t kPlan = 192;     // SyrkPlanHead
+  static constexpr size_t kEvals = 0;  // inverse transforms of the assignment
+  static constexpr size_t kChanged = tcx::kEvalBytes;  // a label changed (plain stores)
+  static constexpr size_t kRedo = kChanged + 4;   // a cluster needs the eigenvector path
+  static constexpr size_t kBad = kChanged + 8;    // a label was outside [0, k)
+  static constexpr size_t kPlan = kChanged + 64;  // SyrkPlanHead
   static constexpr size_t kInfo = sizeof(int) * tcx::kRefineStatusInts;
   int k;
   size_t offsets() const { return kInfo + sizeof(tcx::PowerInfo) * (size_t)k; }
@@ -1488,7 +1488,7 @@ int fit_assign(tcx_ctx* c, FitState& f, int* h_changed) {
   }
   f.have_dist = true;
   *h_changed = *reinterpret_cast<const int*>(h + RefineStatus::kChanged);
-  const auto h_evals = *reinterpret_cast<const unsigned long long*>(h + RefineStatus::kEvals);
+  const unsigned long long h_evals = tcx::eval_sum(h + RefineStatus::kEvals);
   float ms = 0.f;
   if (f.ref_timed) {
     TCX_HIP(hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));

@@ -66,6 +66,20 @@ __host__ __device__ constexpr long bound_frag(long row, int f, int kpad) {
          (f & 3);
 }
 __host__ __device__ constexpr long bound_rows(long rows) { return (rows + 15) & ~15L; }
+// The count of inverse transforms is spread over kEvalSlots counters of a
+// 128-byte line each (the sum counts).  One counter took 10 ns per wave, one
+// wave after the other, which the kernel waited for: fit of ten iterations
+// n=100000 m=512 k=16 9030 us with one, 8420 now, 64 uneven jobs at once 66 and
+// 62 ms.
+constexpr int kEvalSlots = 16, kEvalStride = 128 / sizeof(unsigned long long);
+constexpr size_t kEvalBytes = 128 * kEvalSlots;
+inline unsigned long long eval_sum(const void* counters) {
+  unsigned long long s = 0;
+  for (int i = 0; i < kEvalSlots; ++i)
+    s += static_cast<const unsigned long long*>(counters)[i * kEvalStride];
+  return s;
+}
+
 struct PruneArgs {
   const float* x = nullptr;
   const float2* xs = nullptr;    // per-series half spectra [n][F/2+1] (may be NULL: from x)
@@ -85,7 +99,7 @@ struct PruneArgs {
   float* dist = nullptr;
   int* shift = nullptr;
   int* changed = nullptr;
-  unsigned long long* evals = nullptr;  // inverse transforms run (may be NULL)
+  unsigned long long* evals = nullptr;  // inverse transforms run, kEvalSlots counters (may be NULL)
   const int* skip = nullptr;     // nothing is done when *skip (may be NULL)
 };
 hipError_t launch_assign_prune(int F, const PruneArgs& a, hipStream_t st);
@@ -198,7 +212,7 @@ hipError_t launch_align_pack(const float* x, int m, const int* perm, long n_pad,
 long syrk_blocks(int m, int ngroups);
 // The first kRefineStatusInts ints of a refinement's status zeroed, minrow
 // INT_MAX, perm -1.
-constexpr int kRefineStatusInts = 64;
+constexpr int kRefineStatusInts = (kEvalBytes + 256) / sizeof(int);
 hipError_t launch_refine_init(int* status, int* minrow, int k, int* perm, long n_pad,
                               hipStream_t st);
 // The plan of S from the clusters' sizes on the device.
@@ -392,7 +406,7 @@ struct PruneJob {
   float* dist;
   int* shift;
   int* changed;
-  unsigned long long* evals;
+  unsigned long long* evals;  // kEvalSlots counters
   const long* npad;  // may be NULL; else npairs = *npad / 2, read on the device
 };
 long prune_blocks(int F, long npairs, int k, long n);  // grid cap tuned per (F, k, n)
