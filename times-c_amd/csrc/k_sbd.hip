@@ -234,7 +234,7 @@ __device__ __forceinline__ float div_by(float z, float d, float r) {
 }
 
 template <int F, int MODE>
-__global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWaves) void k_sbd(
+__global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWavesDense) void k_sbd(
     const float* __restrict__ x, long n, int m, int k, int kc,
     const float2* __restrict__ cspec, const float* __restrict__ cnorm,
     const float2* __restrict__ twg, int rev, int* __restrict__ label,
@@ -767,14 +767,15 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
     int* __restrict__ shift, int* __restrict__ changed, unsigned long long* __restrict__ evals) {
   using G = PruneGeom<F>;
   constexpr int L = G::L, P = FftGeom<F>::P;
+  constexpr bool kTG = kPre ? F > 1024 : F >= 1024;
   extern __shared__ float2 smem[];
   float2* tw = smem;
-  float* red = reinterpret_cast<float*>(smem + fft_tw_lds<F>() + G::kGroups * fft_buf_len<F>());
+  float* red = reinterpret_cast<float*>(smem + fft_tw_lds<F, kTG>() + G::kGroups * fft_buf_len<F>());
   float* ubs_all = red + 64;
-  for (int i = threadIdx.x; i < fft_tw_lds<F>(); i += blockDim.x) tw[i] = twg[i];
+  for (int i = threadIdx.x; i < fft_tw_lds<F, kTG>(); i += blockDim.x) tw[i] = twg[i];
   __syncthreads();
   const int g = threadIdx.x / L, lane = threadIdx.x % L;
-  float2* buf = smem + fft_tw_lds<F>() + g * fft_buf_len<F>();
+  float2* buf = smem + fft_tw_lds<F, kTG>() + g * fft_buf_len<F>();
   float* ubs = ubs_all + (long)g * 2 * k;  // [0,k): series a, [k,2k): series b
   unsigned my_evals = 0;
   for (long pr = (long)bid * G::kGroups + g; pr < npairs;
@@ -846,7 +847,7 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
       sb = group_sum<L>(sb, red);
       na = sqrtf(sa);
       nb = sqrtf(sb);
-      fft<F, L, false>(zx, buf, tw, twg, lane);
+      fft<F, L, false, kTG>(zx, buf, tw, twg, lane);
       // |X_a[f]| = |Z[f] + conj(Z[F-f])| / 2, |X_b[f]| = |Z[f] - conj(Z[F-f])| / 2
       float px[H + 1], py[H + 1];
       float ma[H + 1], mb[H + 1];
@@ -922,7 +923,7 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
         float2 z[P];
 #pragma unroll
         for (int s = 0; s < P; ++s) z[s] = cmulc(zx[s], cjs[s * L + lane]);
-        fft<F, L, true>(z, buf, tw, twg, lane);
+        fft<F, L, true, kTG>(z, buf, tw, twg, lane);
         float va, vb;
         lag_max<F, L, P>(z, rev, lane, m, red, va, ka, vb, kb);
         if (dena != 0.f) da = 1.f - (va / (float)F) / dena; else ka = 0;
@@ -956,7 +957,9 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
 }
 
 template <int F, bool kPre>
-__global__ __launch_bounds__(PruneGeom<F>::kBlock, PruneGeom<F>::kMinWaves) void k_assign_prune(
+__global__ __launch_bounds__(PruneGeom<F>::kBlock, kPre ? FftGeom<F>::kMinWaves
+                                                             : FftGeom<F>::kMinWavesPrune)
+void k_assign_prune(
     const float* __restrict__ x, const float2* __restrict__ xs, const float* __restrict__ xn,
     const float* __restrict__ ubg, int ub_ld, long n, long npairs, int m, int k,
     const float2* __restrict__ cspec, const float* __restrict__ cmag,
@@ -1157,11 +1160,11 @@ static hipError_t launch_sbd_F(const SbdArgs& a, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <int F>
+template <int F, bool TG = (F > 1024)>
 static size_t prune_smem(int k) {
   using G = PruneGeom<F>;
-  return sizeof(float2) * (fft_tw_lds<F>() + G::kGroups * fft_buf_len<F>()) + sizeof(float) * 64 +
-         sizeof(float) * 2 * (size_t)k * G::kGroups;
+  return sizeof(float2) * (fft_tw_lds<F, TG>() + G::kGroups * fft_buf_len<F>()) +
+         sizeof(float) * 64 + sizeof(float) * 2 * (size_t)k * G::kGroups;
 }
 
 // Largest k whose per-group bound lists fit the LDS of one workgroup.
@@ -1181,16 +1184,18 @@ static hipError_t launch_prune_F(const PruneArgs& a, hipStream_t st) {
   long blocks = (a.npairs + G::kGroups - 1) / G::kGroups;
   if (blocks < 1) blocks = 1;
   if (blocks > cap) blocks = cap;
+  constexpr bool kTG = F >= 1024;  // as in the body
+  const size_t smem = prune_smem<F, kTG>(a.k);
   if (a.xs && a.ub)
     hipLaunchKernelGGL((k_assign_prune<F, true>), dim3((unsigned)blocks), dim3(G::kBlock),
                        prune_smem<F>(a.k), st, a.x, a.xs, a.xn, a.ub, a.ub_ld, a.n, a.npairs, a.m,
                        a.k, a.cspec, a.cmag, a.cnorm, a.tw, a.rev, a.order, a.label, a.dist,
                        a.shift, a.changed, a.evals, a.skip);
   else
-    hipLaunchKernelGGL((k_assign_prune<F, false>), dim3((unsigned)blocks), dim3(G::kBlock),
-                       prune_smem<F>(a.k), st, a.x, nullptr, nullptr, nullptr, 0, a.n, a.npairs,
-                       a.m, a.k, a.cspec, a.cmag, a.cnorm, a.tw, a.rev, a.order, a.label, a.dist,
-                       a.shift, a.changed, a.evals, a.skip);
+    hipLaunchKernelGGL((k_assign_prune<F, false>), dim3((unsigned)blocks), dim3(G::kBlock), smem,
+                       st, a.x, nullptr, nullptr, nullptr, 0, a.n, a.npairs, a.m, a.k, a.cspec,
+                       a.cmag, a.cnorm, a.tw, a.rev, a.order, a.label, a.dist, a.shift, a.changed,
+                       a.evals, a.skip);
   return hipGetLastError();
 }
 

@@ -393,18 +393,20 @@ __host__ __device__ constexpr int tw_offset(int F, int P, int Ns) {
 // blocks per CU.  The entries are loaded ahead of the exchange before their
 // pass; read in the pass, their latency cost as much as the occupancy gave
 // (assign n=1024 m=1000 k=24: 138 us from LDS, 184 read in the pass, 128
-// loaded ahead; n=8192 m=3000 k=64: 5.69 ms from LDS, 3.2 ms now).
+// loaded ahead; n=8192 m=3000 k=64: 5.69 ms from LDS, 3.2 ms now).  TG: the late
+// passes read the global table; at F = 1024 asked for where four waves per SIMD
+// are wanted, whose LDS would not hold four blocks' tables.
 constexpr int kTwLdsMaxNs = 16;
-template <int F>
+template <int F, bool TG = (F > 1024)>
 constexpr int fft_tw_lds() {
-  return F <= 1024 ? F : tw_offset(F, F / fft_lanes(F), kTwLdsMaxNs * 16);
+  return !TG ? F : tw_offset(F, F / fft_lanes(F), kTwLdsMaxNs * 16);
 }
 
 // Whether the pass with stride Ns reads its twiddles from LDS.
-template <int F, int L, int Ns>
+template <int F, int L, int Ns, bool TG>
 constexpr bool tw_in_lds() {
   constexpr int P = F / L, R = (F / Ns < P) ? F / Ns : P;
-  return tw_offset(F, P, Ns) + (R - 1) * Ns <= fft_tw_lds<F>();
+  return tw_offset(F, P, Ns) + (R - 1) * Ns <= fft_tw_lds<F, TG>();
 }
 
 // This lane's twiddles of the pass with stride Ns from the global table: its
@@ -427,7 +429,7 @@ __device__ __forceinline__ void load_twiddles(const float2* __restrict__ twg, in
 // wg: the pass's twiddles where they come from the global table, loaded by
 // the pass before ahead of its exchange, so that their latency runs beside
 // the exchange's.
-template <int F, int L, bool INV, int Ns>
+template <int F, int L, bool INV, int Ns, bool TG>
 __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
                                               const float2* tw,
                                               const float2* __restrict__ twg, int lane,
@@ -474,7 +476,7 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
 #pragma unroll
       for (int r = 1; r < R; ++r) {
         float2 w;
-        if constexpr (tw_in_lds<F, L, Ns>()) {
+        if constexpr (tw_in_lds<F, L, Ns, TG>()) {
           w = tw[kOff + (r - 1) * Ns + kk];
         } else {
           // the empty asms stand where a load would: the compiler orders the
@@ -490,7 +492,7 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
     }
     dft<R, INV>(b);
     if constexpr (!kLast) {
-      if constexpr (!tw_in_lds<F, L, Ns * R>())
+      if constexpr (!tw_in_lds<F, L, Ns * R, TG>())
         if (t == NB - 1) load_twiddles<F, L, Ns * R>(twg, lane, wn);
       // base + r*Ns: (j-kk)*R is a multiple of Ns*R and kk < Ns, so
       // (base & 31) + ((r*Ns) & 31) < 32 for every r < R (Ns, R powers of
@@ -507,17 +509,17 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[F / L], float2* buf,
   }
   if constexpr (!kLast) {
     group_sync<L>();
-    stockham_pass<F, L, INV, Ns * R>(v, buf, tw, twg, lane, wn);
+    stockham_pass<F, L, INV, Ns * R, TG>(v, buf, tw, twg, lane, wn);
   }
 }
 
 // Unnormalized transform: forward uses exp(-2 pi i f t / F), inverse
 // exp(+2 pi i f t / F) (no 1/F).
-template <int F, int L, bool INV>
+template <int F, int L, bool INV, bool TG = (F > 1024)>
 __device__ __forceinline__ void fft(float2 (&v)[F / L], float2* buf, const float2* tw,
                                     const float2* __restrict__ twg, int lane) {
   float2 none[F / L];
-  stockham_pass<F, L, INV, 1>(v, buf, tw, twg, lane, none);
+  stockham_pass<F, L, INV, 1, TG>(v, buf, tw, twg, lane, none);
 }
 
 // Lane-group geometry per FFT length: L lanes, P = F/L values per lane.
@@ -531,6 +533,18 @@ struct FftGeom {
   // a CU's blocks does: three at 168 VGPRs, at F = 8192 (blocks of 8 waves)
   // two blocks or four waves at 128
   static constexpr int kMinWaves = F <= 4096 ? 3 : 4;
+  // Four at 128 VGPRs, a few values spilled, where waiting and not the VALU
+  // bounds: the pruned assignment that reads the series (each pair's rows, then
+  // one candidate's spectrum after the other; at three waves the VALU was
+  // issuing 58% of the time at F = 1024, 100% at 256) and the dense one of long
+  // series.  Three and four waves: pruned n=66666 m=120 k=40 425, 466 us;
+  // n=32000 m=250 474, 435; n=16000 m=500 714, 490; n=8000 m=1000 503, 477;
+  // n=4000 m=2000 477, 452; n=30000 m=365 k=12 332, 225.  Dense n=32000 m=250
+  // k=40 865, 969; n=16000 m=500 738, 731; n=8000 m=1000 692, 670; n=4000
+  // m=2000 751, 714.  With the per-fit spectra loaded instead, four are slower
+  // (100000 series m=512 k=16, ten assignments: 4.5, 5.6 ms).
+  static constexpr int kMinWavesPrune = F >= 512 ? 4 : 3;
+  static constexpr int kMinWavesDense = F >= 2048 ? 4 : 3;
 };
 
 // Lag key of circular correlation position tau (0 <= tau < F): the index in
