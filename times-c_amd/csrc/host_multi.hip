@@ -291,20 +291,22 @@ struct Keyed {
 // Context buffers (ctx_buffer ids) of the executor.
 enum CtxBuf {
   kCbSlab, kCbGinfo, kCbInfo, kCbEvc, kCbGinfoH, kCbInfoH, kCbEvcH, kCbDoneD, kCbDoneH,
-  kCbOutH, kCbInitH, kCbUpDev, kCbUpPin, kCbAsgDev, kCbAsgPin, kCbCount
+  kCbOutH, kCbInitH, kCbUpDev, kCbUpPin, kCbAsgDev, kCbAsgPin,
+  kCbGramDev, kCbGramPin, kCbCount
 };
 static_assert(kCbCount <= kCtxBuffers, "context buffers");
 
 struct Batch {
   tcx_ctx* ctx = nullptr;
   hipStream_t st = nullptr;
-  // second stream: the block-form Gram Lanczos runs beside the resident
-  // form (default priority; joined back into st by an event)
+  // second stream: the block-form Gram Lanczos and the Gram form's way back
+  // run beside the resident and the two-launch forms (default priority;
+  // joined back into st by an event)
   hipStream_t st2 = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_res = nullptr, ev_join = nullptr;
   int cus = 0;
   std::vector<GJob> jobs;
-  Uploader up;
+  Uploader up, up_gram;  // up_gram: tables that st2 reads while up is rewritten
   // readback pools (device + pinned host), sized for every job of the run;
   // these, the done flags, the slab and the pinned staging are the
   // context's buffers (kept between calls)
@@ -331,6 +333,7 @@ struct Batch {
     if (st) (void)hipStreamSynchronize(st);
     if (st2) (void)hipStreamSynchronize(st2);
     if (ev_fork) (void)hipEventDestroy(ev_fork);
+    if (ev_res) (void)hipEventDestroy(ev_res);
     if (ev_join) (void)hipEventDestroy(ev_join);
     for (GJob& j : jobs)
       if (j.arena && !slab) (void)hipFree(j.arena);
@@ -720,9 +723,6 @@ int refine_power(Batch& b, const std::vector<GJob*>& act, double* ms_power) {
   GX_TRY(run_syrk(b, sj_off, by_off, tl_off, by));
   GX_HIP(launch_gram_tiles(reinterpret_cast<const GramItem*>(b.up.dev(gi_off)), (int)gitems.size(),
                            b.st));
-  // the two-launch form first: its finishing pass writes v, steps and conv
-  // of every cluster of its jobs, the Gram form's included
-  GX_TRY(power_split(b, split_set, 0));  // uploads its own tables
   // largest clusters first: a launch lasts as long as its slowest block,
   // so those start in the first wave of blocks (each cluster's result is
   // independent of its position)
@@ -730,19 +730,22 @@ int refine_power(Batch& b, const std::vector<GJob*>& act, double* ms_power) {
                    [](const LzResJob& a, const LzResJob& c) { return a.d > c.d; });
   std::stable_sort(glz.begin(), glz.end(),
                    [](const GramLzJob& a, const GramLzJob& c) { return a.nd > c.nd; });
-  b.up.reset();
-  const size_t gl_off = b.up.put_vec(glz), gm_off = b.up.put_vec(gmap);
-  const size_t wl_off = b.up.put_vec(wlz);
-  pw.stage(b.up);
-  GX_TRY(b.up.flush(b.st));
-  if (!glz.empty()) {  // the block form on the second stream, after the upload
-    GX_HIP(hipEventRecord(b.ev_fork, b.st));
-    GX_HIP(hipStreamWaitEvent(b.st2, b.ev_fork, 0));
-    GX_HIP(launch_gram_lanczos(reinterpret_cast<const GramLzJob*>(b.up.dev(gl_off)),
-                               (int)glz.size(), lds_lz, kLzPowerTol, b.st2));
-    GX_HIP(hipEventRecord(b.ev_join, b.st2));
-  }
-  const LzResJob* dwl = reinterpret_cast<const LzResJob*>(b.up.dev(wl_off));
+  b.up_gram.reset();
+  const size_t gl_off = b.up_gram.put_vec(glz), gm_off = b.up_gram.put_vec(gmap);
+  const size_t wl_off = b.up_gram.put_vec(wlz);
+  pw.stage(b.up_gram);
+  GX_TRY(b.up_gram.flush(b.st));
+  // Three chains over different clusters' vectors (the two-launch form leaves
+  // the clusters without a count alone), none of which fills the device: on
+  // st the resident form and then the two-launch form, on st2 the block form
+  // of Gram matrices and, once the resident form is done too, the Gram form's
+  // way back.  One after the other they took 2.3 ms per iteration of 64 uneven
+  // jobs, 62 ms in all; now 59.
+  GX_HIP(hipEventRecord(b.ev_fork, b.st));
+  GX_HIP(hipStreamWaitEvent(b.st2, b.ev_fork, 0));
+  GX_HIP(launch_gram_lanczos(reinterpret_cast<const GramLzJob*>(b.up_gram.dev(gl_off)),
+                             (int)glz.size(), lds_lz, kLzPowerTol, b.st2));
+  const LzResJob* dwl = reinterpret_cast<const LzResJob*>(b.up_gram.dev(wl_off));
   for (size_t i = 0; i < wlz.size();) {  // one launch per register split
     const int form = lz_res_form(wlz[i].d);
     size_t e = i;
@@ -750,10 +753,14 @@ int refine_power(Batch& b, const std::vector<GJob*>& act, double* ms_power) {
     GX_HIP(launch_lz_res_group(dwl + i, (int)(e - i), form, kLzPowerTol, b.st));
     i = e;
   }
-  if (!glz.empty()) GX_HIP(hipStreamWaitEvent(b.st, b.ev_join, 0));
-  GX_HIP(launch_gram_map(reinterpret_cast<const GramVecJob*>(b.up.dev(gm_off)), (int)gmap.size(),
-                         lds_map, b.st));
-  GX_HIP(launch_power_group(pw.table(b.up), b.st));
+  GX_HIP(hipEventRecord(b.ev_res, b.st));
+  GX_HIP(hipStreamWaitEvent(b.st2, b.ev_res, 0));
+  GX_HIP(launch_gram_map(reinterpret_cast<const GramVecJob*>(b.up_gram.dev(gm_off)),
+                         (int)gmap.size(), lds_map, b.st2));
+  GX_HIP(hipEventRecord(b.ev_join, b.st2));
+  GX_TRY(power_split(b, split_set, 0));  // uploads its own tables
+  GX_HIP(hipStreamWaitEvent(b.st, b.ev_join, 0));
+  GX_HIP(launch_power_group(pw.table(b.up_gram), b.st));
   GX_HIP(hipMemcpyAsync(b.info_h, b.info_d, b.info_bytes, hipMemcpyDeviceToHost, b.st));
   GX_HIP(hipStreamSynchronize(b.st));
   // clusters whose power result fails the tests: the eigenvector path
@@ -964,7 +971,9 @@ int grouped_fit(tcx_ctx* ctx, tcx_job* jobs, const int* idx, int count, size_t h
   }
   b.up.bind(ctx, kCbUpDev, kCbUpPin);
   b.up_asg.bind(ctx, kCbAsgDev, kCbAsgPin);
+  b.up_gram.bind(ctx, kCbGramDev, kCbGramPin);
   GX_HIP(hipEventCreateWithFlags(&b.ev_fork, hipEventDisableTiming));
+  GX_HIP(hipEventCreateWithFlags(&b.ev_res, hipEventDisableTiming));
   GX_HIP(hipEventCreateWithFlags(&b.ev_join, hipEventDisableTiming));
   b.jobs.resize(count);
   for (int q = 0; q < count; ++q) {

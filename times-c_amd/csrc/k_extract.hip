@@ -2778,6 +2778,13 @@ __global__ __launch_bounds__(kPowerThreads) void k_lz_setup_group(const LzJob* _
                                                                   const int* __restrict__ first,
                                                                   int njobs) {
   TCX_GROUP_JOB(LzJob)
+  if (a.counts[bid] == 0) {  // nothing of the cluster's vectors is touched
+    if (threadIdx.x == 0) {
+      a.state[bid].done = 1;
+      if (a.done_out) a.done_out[bid] = 1;
+    }
+    return;
+  }
   lz_setup_body(bid, nblk, a.m, a.counts, a.mask, a.seed, a.iter, a.rbuf, a.Q, a.state);
   if (threadIdx.x == 0 && a.done_out) a.done_out[bid] = a.state[bid].done;  // thread 0 wrote it
 }
@@ -2795,6 +2802,7 @@ __global__ __launch_bounds__(kPowerThreads) void k_lz_finish_group(const LzJob* 
                                                                    const int* __restrict__ first,
                                                                    int njobs) {
   TCX_GROUP_JOB(LzJob)
+  if (a.counts[bid] == 0) return;  // another form's, or empty
   lz_finish_body(bid, nblk, a.m, a.counts, a.Q, a.state, a.vout, a.steps_out, a.conv_out);
 }
 

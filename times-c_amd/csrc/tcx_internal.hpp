@@ -43,7 +43,7 @@ size_t device_free_bytes(tcx_ctx* c);
 // growing frees the old one: only while nothing in flight uses it.  Device
 // bytes count as workspace (held_bytes); trim_workspace and tcx_destroy
 // release them.
-constexpr int kCtxBuffers = 16;
+constexpr int kCtxBuffers = 18;
 int ctx_buffer(tcx_ctx* c, int id, size_t bytes, bool pinned, void** out);
 // Device bytes the context's kept buffers hold (reusable by the next call).
 size_t ctx_buffer_device_bytes(const tcx_ctx* c);
