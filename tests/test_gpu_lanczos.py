@@ -78,6 +78,18 @@ def test_blocks_of_one_cluster(ctx, m, k):
     assert max(centroid_errors(got, ref)) <= CENT_RTOL
 
 
+@pytest.mark.parametrize("m,k", [(512, 17), (512, 65), (511, 40), (738, 22), (769, 31),
+                                 (1024, 17)])
+def test_blocks_in_several_launches(ctx, m, k):
+    """More clusters than one launch holds (the first two take one, three; a
+    device of 256 CUs), among them empty ones at the ends of launches: every
+    cluster starts from its own vector."""
+    X, y = T.generate(5 * m + k, 30 * k, m, k, 0.3)
+    y[(y == 0) | (y == k - 1)] = k // 2
+    got, ref = _extract(ctx, X, y, k)
+    assert max(centroid_errors(got, ref)) <= CENT_RTOL
+
+
 @pytest.mark.parametrize("m", [400, 900])
 def test_blocks_slow_convergence(ctx, m):
     """White noise over many blocks: more steps than basis rows in LDS.  The

@@ -2760,14 +2760,6 @@ __global__ __launch_bounds__(256) void k_syrk_reduce_group(const SyrkJob* __rest
   syrk_reduce_body(blockIdx.x % (kSub * kSub), gt->t, jb.part, jb.m, jb.S);
 }
 
-__global__ __launch_bounds__(kPowerThreads) void k_power_lanczos_group(
-    const PowerLanczosJob* __restrict__ jobs, const int* __restrict__ first, int njobs,
-    double lz_tol) {
-  TCX_GROUP_JOB(PowerLanczosJob)
-  power_lanczos_body(bid, nblk, a.S, a.m, a.counts, a.seed, a.iter, a.I, lz_tol, a.Q, a.vout,
-                     a.rout, a.steps_out, a.conv_out);
-}
-
 __global__ __launch_bounds__(kMvThreads) void k_cluster_matvec_group(
     const ClusterMatvecJob* __restrict__ jobs, const int* __restrict__ first, int njobs) {
   TCX_GROUP_JOB(ClusterMatvecJob)
@@ -3915,8 +3907,8 @@ __device__ __forceinline__ double wave_rows_sum(const double (&t)[N], int lane) 
 
 template <int U, int RW, typename T>
 __global__ __launch_bounds__(64 * kLzMultiWaves, 1) void k_lz_multi(
-    const float* __restrict__ S, int m, int k, int G, int R, const int* __restrict__ counts,
-    uint64_t seed, int iter, int I, double lz_tol, double* Qfar, uint64_t* __restrict__ xch,
+    const float* __restrict__ S, int m, int j0, int k, int G, int R,
+    const int* __restrict__ counts, uint64_t seed, int iter, int I, double lz_tol, double* Qfar, uint64_t* __restrict__ xch,
     uint32_t* __restrict__ fails, uint32_t gen, long long timeout, double* __restrict__ vout,
     double* __restrict__ svout, double* __restrict__ rout, int* __restrict__ steps_out,
     int* __restrict__ conv_out) {
@@ -4108,7 +4100,7 @@ __global__ __launch_bounds__(64 * kLzMultiWaves, 1) void k_lz_multi(
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int e = lane + 64 * u;
-    q[u] = e < m ? power_v0(seed, iter, j, e) : 0.0;
+    q[u] = e < m ? power_v0(seed, iter, j0 + j, e) : 0.0;
     n0 += q[u] * q[u];
     qp[u] = 0.0;
   }
@@ -4125,7 +4117,7 @@ __global__ __launch_bounds__(64 * kLzMultiWaves, 1) void k_lz_multi(
 #pragma unroll
   for (int i = 0; i < E; ++i) {
     const int e = own_e + 64 * i;
-    own_q[i] = e < m ? power_v0(seed, iter, j, e) / n0 : 0.0;
+    own_q[i] = e < m ? power_v0(seed, iter, j0 + j, e) / n0 : 0.0;
     own_qp[i] = 0.0;
   }
   put_row(0, own_q);
@@ -4412,19 +4404,37 @@ hipError_t launch_lz_res(const float* S, int m, int k, const int* counts, uint64
   return hipGetLastError();
 }
 
-// Forms of k_lz_multi: {U, RW, LDS}; rows per member R = 4 RW at most.
+// Forms of k_lz_multi: {U, RW, LDS}; rows per member R = 4 RW at most.  The
+// members of a cluster must all be resident, so a launch takes as many clusters
+// as there are CUs for, and more clusters take several launches of equal size.
+// Of the two forms for m <= 512 the first has half the rows per member and is
+// taken when one launch of it holds every cluster, else the second with half the
+// members.  A launch takes about 115 us for m <= 512 and 170 above, the fused
+// form (m <= kFusedLanczosMaxM) per round of the CUs m^2 / 476 us, or m^2 / 137
+// when its rows of S are not 16-byte aligned; the plan is made where it is the
+// shorter.  One refinement, launches and the other form: m=512 k=48 0.33, 0.70
+// ms; m=738 k=22 0.65, 4.2; m=700 k=64 1.16, 1.25; m=300 k=200 0.54, 0.48; m=600
+// k=300 4.0, 1.5; against two launches per step m=1000 k=10 0.44, 0.72, k=200
+// 4.4, 5.9.
 bool plan_lz_multi(int m, int k, int cus, LzCoopPlan* p) {
   if (m <= kLzResMaxD || m > kLzMultiMaxM || k <= 0) return false;
   for (int form = m <= 512 ? 0 : 2; form < 3; ++form) {
     const int rmax = form == 1 ? 64 : 32;
     const int G = (m + rmax - 1) / rmax, R = (m + G - 1) / G;
-    const long nb = ((long)k * G + 7) / 8 * 8;
-    if (nb > cus || (long)(G - 1) * R >= m) continue;  // every member owns rows
+    const int most = cus / 8 * 8 / G;  // clusters of a launch
+    if (most < 1 || (form == 0 && most < k)) continue;
+    if ((long)(G - 1) * R >= m) continue;  // every member owns rows
+    const int launches = (k + most - 1) / most, per = (k + launches - 1) / launches;
+    const long rounds = (k + cus - 1) / cus;
+    if (launches > 1 && m <= kFusedLanczosMaxM &&
+        (long)launches * (m <= 512 ? 115 : 170) > rounds * m * m / (m % 4 ? 137 : 476))
+      return false;
+    const long nb = ((long)per * G + 7) / 8 * 8;
     const void* fn = form == 0   ? (const void*)k_lz_multi<8, 8, double>
                      : form == 1 ? (const void*)k_lz_multi<8, 16, float>
                                  : (const void*)k_lz_multi<16, 8, float>;
     const size_t lds = form == 2 ? lz_multi_lds<16>() : lz_multi_lds<8>();
-    int per_cu = 0;  // every member must be resident at once
+    int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64 * kLzMultiWaves, lds) !=
         hipSuccess) {
       (void)hipGetLastError();
@@ -4434,6 +4444,7 @@ bool plan_lz_multi(int m, int k, int cus, LzCoopPlan* p) {
     p->G = G;
     p->R = R;
     p->nb = (int)nb;
+    p->per = per;
     p->form = form;
     p->lds = lds;
     p->xch_len = lz_multi_xch_len(m, G);
@@ -4442,16 +4453,20 @@ bool plan_lz_multi(int m, int k, int cus, LzCoopPlan* p) {
   return false;
 }
 
-hipError_t launch_lz_multi(const LzCoopPlan& p, const float* S, int m, int k, const int* counts,
+hipError_t launch_lz_multi(const LzCoopPlan& p, const float* S, int m, int j0, int k,
+                           const int* counts,
                            uint64_t seed, int iter, int I, double lz_tol, double* Q,
                            uint64_t* xch, uint32_t* fails, uint32_t gen, long long timeout,
                            double* vout, double* svout, double* rout, int* steps_out,
                            int* conv_out, hipStream_t st) {
-  if (gen == 0 || gen >= (1u << (32 - kLzCoopEpochBits))) return hipErrorInvalidValue;
+  if (gen == 0 || gen >= (1u << (32 - kLzCoopEpochBits)) || k > p.per)
+    return hipErrorInvalidValue;
+  const long at = (long)j0 * m;
 #define TCX_LZ_MULTI(U, RW, T)                                                                    \
-  hipLaunchKernelGGL((k_lz_multi<U, RW, T>), dim3(p.nb), dim3(64 * kLzMultiWaves), p.lds, st, S,  \
-                     m, k, p.G, p.R, counts, seed, iter, I, lz_tol, Q, xch, fails, gen, timeout,  \
-                     vout, svout, rout, steps_out, conv_out)
+  hipLaunchKernelGGL((k_lz_multi<U, RW, T>), dim3(p.nb), dim3(64 * kLzMultiWaves), p.lds, st,     \
+                     S + at * m, m, j0, k, p.G, p.R, counts + j0, seed, iter, I, lz_tol,          \
+                     Q + at * (kLzMax + 1), xch, fails, gen, timeout, vout + at, svout + at,      \
+                     rout + at, steps_out + j0, conv_out + j0)
   switch (p.form) {
     case 0:
       TCX_LZ_MULTI(8, 8, double);
@@ -4466,16 +4481,6 @@ hipError_t launch_lz_multi(const LzCoopPlan& p, const float* S, int m, int k, co
       return hipErrorInvalidValue;
   }
 #undef TCX_LZ_MULTI
-  return hipGetLastError();
-}
-
-size_t power_lanczos_lds(int m) { return lanczos_smem(m); }
-
-hipError_t launch_power_lanczos_group(const GroupTable& g, double lz_tol, hipStream_t st) {
-  if (g.blocks <= 0) return hipSuccess;
-  if (g.lds > lanczos_smem(kFusedLanczosMaxM)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_power_lanczos_group, dim3(g.blocks), dim3(kPowerThreads), g.lds, st,
-                     TCX_GROUP_ARGS(PowerLanczosJob), lz_tol);
   return hipGetLastError();
 }
 
@@ -4574,10 +4579,6 @@ hipError_t configure_extract_kernels() {
   if (e == hipSuccess)
     e = hipFuncSetAttribute((const void*)k_power_group, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)power_smem(4096));
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_power_lanczos_group,
-                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lanczos_smem(kFusedLanczosMaxM));
   if (e == hipSuccess)
     e = hipFuncSetAttribute((const void*)k_gram_lanczos, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lanczos_smem(kGramMaxND));

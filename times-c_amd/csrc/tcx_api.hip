@@ -446,12 +446,15 @@ struct RefineResult {
 std::mutex g_coop_mu;
 std::map<int, hipEvent_t> g_coop_last;
 
-// M^I v0 of every non-empty cluster by Lanczos.  From m = kLzCoopMinM, when
-// all k*G blocks fit on the device at once, one launch with G blocks per
-// cluster; else for m <= 768 one fused launch (one block per cluster, S_j
-// read from L2 every step); else per step one grid-wide matvec launch and
-// one per-cluster update launch, and every 8 steps from 16 on the host
-// reads the clusters' done flags and stops once all are done.
+// M^I v0 of every non-empty cluster by Lanczos.  m <= kLzResMaxD: one launch,
+// one block per cluster with S_j in its registers.  m <= kLzMultiMaxM: G blocks
+// per cluster with S_j in their registers, as many clusters per launch as the
+// device holds (plan_lz_multi says when the next forms are faster).  Above, when
+// all k*G blocks fit on the device at once, one launch with S_j in their LDS;
+// else for m <= 768 one fused launch (one block per cluster, S_j read from L2
+// every step); else per step one grid-wide matvec launch and one per-cluster
+// update launch, and every 8 steps from 16 on the host reads the clusters' done
+// flags and stops once all are done.
 // Returns on device the vectors v, S v, the row sums r = S 1, the Lanczos
 // step counts and the per-cluster acceptance flags.
 int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, uint64_t seed,
@@ -482,24 +485,31 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
     return TCX_OK;
   }
   tcx::LzCoopPlan cp;
-  const bool multi = mode == 0 && !mask && tcx::plan_lz_multi(m, k, c->cus, &cp);
-  if (multi || (mode == 0 && !mask && tcx::plan_lz_coop(m, k, c->cus, &cp))) {
+  bool multi = mode == 0 && !mask && tcx::plan_lz_multi(m, k, c->cus, &cp);
+  if (multi && cp.per < k && m <= 640) {
+    // where one launch of the form with S in its blocks' LDS or the L2 holds
+    // every cluster, several of this one are faster only for the longer rows
+    // (two launches and one: a refinement m=520 k=16 0.40 and 0.35 ms, m=600
+    // k=16 0.42, 0.39, m=700 k=16 0.44, 0.45, m=1000 k=10 0.44, 0.72)
+    tcx::LzCoopPlan one;
+    if (tcx::plan_lz_coop(m, k, c->cus, &one)) {
+      cp = one;
+      multi = false;
+    }
+  }
+  bool coop = multi || (mode == 0 && !mask && tcx::plan_lz_coop(m, k, c->cus, &cp));
+  const int per = multi ? cp.per : k;  // clusters of one launch
+  const size_t words = (size_t)per * cp.xch_len + ((size_t)per + 1) / 2;
+  if (multi && c->slot_bytes[kSlotLzXch] < sizeof(uint64_t) * words && c->budget &&
+      c->ws_bytes + c->user_bytes + sizeof(uint64_t) * words + 256 > c->budget)
+    coop = false;  // no room for the exchange
+  if (coop) {
     // exchange words and per-cluster failure words; their contents only
     // ever match the current launch generation, so they are zeroed only
     // when (re)allocated or when the generation wraps
     uint64_t* xch;
-    const size_t words = (size_t)k * cp.xch_len + ((size_t)k + 1) / 2;
     TCX_TRY(ws(c, kSlotLzXch, words, &xch));
-    uint32_t* fails = reinterpret_cast<uint32_t*>(xch + (size_t)k * cp.xch_len);
-    if (xch != c->lz_xch || c->slot_bytes[kSlotLzXch] != c->lz_xch_bytes ||
-        c->lz_gen + 1 >= tcx::kLzCoopMaxGen) {
-      TCX_HIP(tcx::launch_fill_int(reinterpret_cast<int*>(xch),
-                                   (long)(c->slot_bytes[kSlotLzXch] / sizeof(int)), 0, st));
-      c->lz_xch = xch;
-      c->lz_xch_bytes = c->slot_bytes[kSlotLzXch];
-      c->lz_gen = 0;
-    }
-    const uint32_t gen = ++c->lz_gen;
+    uint32_t* fails = reinterpret_cast<uint32_t*>(xch + (size_t)per * cp.xch_len);
     if (!c->coop_ev) TCX_HIP(hipEventCreateWithFlags(&c->coop_ev, hipEventDisableTiming));
     {
       std::lock_guard<std::mutex> lk(g_coop_mu);
@@ -515,12 +525,24 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
         const long long us = std::atoll(e);
         timeout = us < 0 ? -1 : c->wall_khz * us / 1000;
       }
-      if (multi)
-        TCX_HIP(tcx::launch_lz_multi(cp, S, m, k, counts, seed, iter, steps, tcx::kLzPowerTol, Q,
-                                     xch, fails, gen, timeout, v, sv, r, st_out, cv_out, st));
-      else
-        TCX_HIP(tcx::launch_lz_coop(cp, S, m, k, counts, seed, iter, steps, tcx::kLzPowerTol, xch,
-                                    fails, gen, timeout, v, r, st_out, cv_out, st));
+      for (int j0 = 0; j0 < k; j0 += per) {  // one after the other on st
+        if (xch != c->lz_xch || c->slot_bytes[kSlotLzXch] != c->lz_xch_bytes ||
+            c->lz_gen + 1 >= tcx::kLzCoopMaxGen) {
+          TCX_HIP(tcx::launch_fill_int(reinterpret_cast<int*>(xch),
+                                       (long)(c->slot_bytes[kSlotLzXch] / sizeof(int)), 0, st));
+          c->lz_xch = xch;
+          c->lz_xch_bytes = c->slot_bytes[kSlotLzXch];
+          c->lz_gen = 0;
+        }
+        const uint32_t gen = ++c->lz_gen;
+        if (multi)
+          TCX_HIP(tcx::launch_lz_multi(cp, S, m, j0, std::min(per, k - j0), counts, seed, iter,
+                                       steps, tcx::kLzPowerTol, Q, xch, fails, gen, timeout, v,
+                                       sv, r, st_out, cv_out, st));
+        else
+          TCX_HIP(tcx::launch_lz_coop(cp, S, m, k, counts, seed, iter, steps, tcx::kLzPowerTol,
+                                      xch, fails, gen, timeout, v, r, st_out, cv_out, st));
+      }
       TCX_HIP(hipEventRecord(c->coop_ev, st));
       g_coop_last[c->device] = c->coop_ev;
     }

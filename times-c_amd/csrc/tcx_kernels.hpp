@@ -280,6 +280,7 @@ struct LzCoopPlan {
   size_t lds = 0;            // dynamic LDS bytes per block
   long xch_len = 0;          // exchange words per cluster
   int form = 0;              // k_lz_multi's register split
+  int per = 0;               // clusters of one of its launches
 };
 // False when m, k or the device do not allow every member to be resident.
 bool plan_lz_coop(int m, int k, int cus, LzCoopPlan* p);
@@ -294,11 +295,13 @@ hipError_t launch_lz_coop(const LzCoopPlan& p, const float* S, int m, int k, con
                           double* rout, int* steps_out, int* conv_out, hipStream_t st);
 // The same with one exchange per step and the rows of S in registers
 // (k_lz_multi; S v written too, Q: (kLanczosMax + 1) x m per cluster for basis
-// rows past those in LDS), for kLzResMaxD < m <= kLzMultiMaxM when all members
-// fit the device at once.
+// rows past those in LDS), for kLzResMaxD < m <= kLzMultiMaxM, p.per clusters
+// per launch: here the k <= p.per from j0 on (S to conv_out are those of cluster
+// 0, xch and fails of this launch).
 constexpr int kLzMultiMaxM = 1024;
 bool plan_lz_multi(int m, int k, int cus, LzCoopPlan* p);
-hipError_t launch_lz_multi(const LzCoopPlan& p, const float* S, int m, int k, const int* counts,
+hipError_t launch_lz_multi(const LzCoopPlan& p, const float* S, int m, int j0, int k,
+                           const int* counts,
                            uint64_t seed, int iter, int I, double lz_tol, double* Q,
                            uint64_t* xch, uint32_t* fails, uint32_t gen, long long timeout,
                            double* vout, double* svout, double* rout, int* steps_out,
@@ -508,21 +511,6 @@ hipError_t launch_syrk_group(const SyrkJob* jobs, const GroupSyrkItem* items, in
                              int split, hipStream_t st);
 hipError_t launch_syrk_reduce_group(const SyrkJob* jobs, const GroupSyrkTile* tiles,
                                     int ntiles, hipStream_t st);
-
-struct PowerLanczosJob {
-  const float* S;
-  int m;
-  const int* counts;
-  uint64_t seed;
-  int iter, I;
-  double* Q;
-  double* vout;
-  double* rout;
-  int* steps_out;
-  int* conv_out;
-};
-size_t power_lanczos_lds(int m);
-hipError_t launch_power_lanczos_group(const GroupTable& g, double lz_tol, hipStream_t st);
 
 // Gram form of thin clusters (segment nd < m, nd <= kGramMaxND, m <=
 // kGramMaxM): G = Yc Yc^T in 64 x 64 tiles (the diagonal ones also form
