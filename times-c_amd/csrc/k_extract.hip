@@ -875,8 +875,8 @@ __global__ __launch_bounds__(256) void k_syrk_reduce(const SyrkCluster* __restri
 
 // The plan of S = Y^T Y (plan_syrk's, group for group) from the cluster sizes
 // on the device, by one block: the shortest chunk bound in whole 16-column
-// steps, at least kSyrkMinSteps, whose groups are at most gmax, by bisection
-// (each trial one block sum over the clusters), then every cluster's first
+// steps, at least kSyrkMinSteps, whose groups are at most gmax, each of the four
+// waves trying another bound at a time, then every cluster's first
 // group and partial by a scan 256 clusters at a time.  Bound by its block sums'
 // latency, a few us; the host's plan took a wait for the sizes and two copies,
 // during which the device idled.  With the wait after the power stage left out
@@ -894,31 +894,36 @@ __global__ __launch_bounds__(256) void k_syrk_plan(const long* __restrict__ offs
   auto steps_of = [&](int j) -> int {
     return counts[j] > 0 ? (int)((offsets[j + 1] - offsets[j] + 15) / 16) : 0;
   };
-  auto block_total = [&](int v, bool take_max) -> int {
+  int mx = 0;  // every wave for itself
+  for (int j = lane; j < k; j += 64) mx = max(mx, steps_of(j));
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const int u = __shfl_xor(v, o);
-      v = take_max ? max(v, u) : v + u;
-    }
-    __syncthreads();
-    if (lane == 0) red[wid] = v;
-    __syncthreads();
-    return take_max ? max(max(red[0], red[1]), max(red[2], red[3]))
-                    : (red[0] + red[1]) + (red[2] + red[3]);
-  };
-  int mx = 0;
-  for (int j = t; j < k; j += 256) mx = max(mx, steps_of(j));
-  const int max_steps = block_total(mx, true);
+  for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o));
+  const int max_steps = mx;
   if (max_steps == 0) {
     if (t == 0) *head = SyrkPlanHead{0, 0};
     return;
   }
+  const int st0 = lane < k ? steps_of(lane) : 0;  // k <= 64: read once
   int lo = min(kSyrkMinSteps, max_steps), hi = max_steps;
   while (lo < hi) {
-    const int mid = (lo + hi) / 2;
-    int g = 0;
-    for (int j = t; j < k; j += 256) g += (steps_of(j) + mid - 1) / mid;
-    if (block_total(g, false) <= gmax) hi = mid; else lo = mid + 1;
+    // the trials cut [lo, hi) in five; more steps, fewer groups
+    const int len = hi - lo, mid = lo + len * (wid + 1) / 5;
+    int g = (st0 + mid - 1) / mid;
+    for (int j = lane + 64; j < k; j += 64) g += (steps_of(j) + mid - 1) / mid;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) g += __shfl_xor(g, o);
+    __syncthreads();  // the previous trials are read
+    if (lane == 0) red[wid] = g;
+    __syncthreads();
+    int nlo = lo, nhi = hi;
+#pragma unroll
+    for (int w = 3; w >= 0; --w)
+      if (red[w] <= gmax) nhi = lo + len * (w + 1) / 5;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      if (red[w] > gmax) nlo = lo + len * (w + 1) / 5 + 1;
+    lo = nlo;
+    hi = nhi;
   }
   int g0 = 0, c0 = 0;  // groups and clusters before this tile of clusters
   for (int j0 = 0; j0 < k; j0 += 256) {
