@@ -293,8 +293,9 @@ int tcx_batch_run(tcx_batch* b, tcx_job* jobs, int njobs, int order);
  * device memory fits the batch's hbm_budget (0: 80% of the free device
  * memory) and join as others finish.  A job's results do not depend on the
  * other jobs; they equal those of tcx_kshape_fit to rounding (the power
- * stage is the one-block-per-cluster Lanczos up to m = 768 and the
- * two-launch form above; S takes one K chunk per tile).  Jobs with
+ * stage takes each cluster's Gram matrix where that is smaller, one block
+ * per cluster up to order 256 and for Gram matrices, and two launches per
+ * Lanczos step for the rest; S takes one K chunk per tile).  Jobs with
  * init_mode 1, cal_select 1 or k beyond the pruned assignment's limit run on
  * the worker pool as in tcx_batch_run.  Returns as tcx_batch_run; ms_refine
  * and ms_assign of a grouped job are the wall times of the grouped phases
