@@ -975,7 +975,7 @@ void k_assign_prune(
 // Each series against one centroid, shifted in place by the lag of its
 // largest NCC with zero fill (out[t] = in[t - s], 0 outside; roll_zeropad,
 // test_timesC.py:55-77), nothing for an all-zero centroid: one kernel forms
-// the pair's correlation, its lags (k_sbd's, bit for bit) and the shifted
+// the pair's correlation, its lags (the search's, bit for bit) and the shifted
 // rows, which it reads again from L2.  Bound by the two transforms.  With
 // the shifts through memory, the bounds of a search over one centroid and a
 // second kernel to shift the rows, n=12000 m=700 took 143 us, 95 now.
@@ -1020,10 +1020,17 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWaves) void k_a
     float va, vb;
     int ka, kb;
     lag_max<F, L, P>(z, rev, lane, m, red, va, ka, vb, kb);
-    // den == 0: every lag is 0, the argmax is index 0
+    // index 0, the argmax of an all-zero or all-NaN row, where a norm is zero or
+    // past the range or the distance is no number (lag_max then has no lag), as
+    // the search over centroids leaves it
     const float cn = cnorm[0];
-    if (sqrtf(sa) * cn == 0.f) ka = 0;
-    if (sqrtf(sb) * cn == 0.f) kb = 0;
+    auto key = [&](float ss, float v, int k) {
+      const float den = sqrtf(ss) * cn;
+      return ss < INFINITY && cn < INFINITY && den != 0.f && 1.f - (v / (float)F) / den < INFINITY
+                 ? k : 0;
+    };
+    ka = key(sa, va, ka);
+    kb = key(sb, vb, kb);
     const int ha = ka + 1 - m, hb = kb + 1 - m;
     const int mo = opaque(m);
 #pragma unroll
