@@ -240,7 +240,7 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWavesDense) voi
     const float2* __restrict__ twg, int rev, int* __restrict__ label,
     float* __restrict__ dist, int* __restrict__ shift, float* __restrict__ dmat,
     int* __restrict__ changed, float* __restrict__ ncc_out,
-    const int* __restrict__ fixed_label, const int* __restrict__ skip) {
+    const int* __restrict__ fixed_label, int search, const int* __restrict__ skip) {
   using G = FftGeom<F>;
   constexpr int L = G::L, P = G::P;
   extern __shared__ float2 smem[];
@@ -274,7 +274,9 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWavesDense) voi
     }
     sa = group_sum<L>(sa, red);
     sb = group_sum<L>(sb, red);
-    const float na = sqrtf(sa), nb = sqrtf(sb);
+    float na = sqrtf(sa), nb = sqrtf(sb);
+    if (MODE == kModeAssign && search && !(sa < INFINITY || (hasb && sb < INFINITY)))
+      na = nb = NAN;  // no distance
     fft<F, L, false>(zx, buf, tw, twg, lane);
 
     float bestA = INFINITY, bestB = INFINITY;
@@ -312,6 +314,14 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWavesDense) voi
         float da = 1.f, db = 1.f;
         if (dena != 0.f) da = 1.f - (va / (float)F) / dena; else ka = 0;
         if (denb != 0.f) db = 1.f - (vb / (float)F) / denb; else kb = 0;
+        if (MODE == kModeAssign && search) {
+          if (cn == 0.f && (na == na || nb == nb)) {
+            da = db = 1.f;
+            ka = kb = 0;
+          } else if (!(cn < INFINITY)) {
+            da = db = INFINITY;
+          }
+        }
         if (MODE == kModeOwn ? (j == fixA) : (da < bestA)) { bestA = da; labA = j; keyA = ka; }
         if (MODE == kModeOwn ? (j == fixB) : (db < bestB)) { bestB = db; labB = j; keyB = kb; }
         if (MODE == kModeAssign && dmat && lane == 0) {
@@ -1165,7 +1175,7 @@ static hipError_t launch_sbd_F(const SbdArgs& a, hipStream_t st) {
                      sbd_smem<F>(), st, a.x, a.n, a.m, a.k, kc, a.cspec, a.cnorm, a.tw, a.rev,
                      split ? a.part_label : a.label, split ? a.part_dist : a.dist,
                      split ? a.part_shift : a.shift, a.dmat, split ? nullptr : a.changed,
-                     a.ncc_out, a.fixed_label, a.skip);
+                     a.ncc_out, a.fixed_label, (int)a.search, a.skip);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !split) return e;
   hipLaunchKernelGGL(k_split_min, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, st,

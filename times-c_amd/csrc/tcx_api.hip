@@ -312,6 +312,7 @@ int assign_core_tw(tcx_ctx* c, const float2* tw, const float* d_x, long n, int m
   a.rev = rev; a.label = label; a.dist = dist; a.shift = shift; a.dmat = dmat;
   a.changed = changed;
   a.chunks = chunks;
+  a.search = !dmat && k <= tcx::prune_max_k(F);
   a.skip = skip;
   if (part) {
     a.part_dist = part;

@@ -31,6 +31,11 @@ struct SbdArgs {
   float* part_dist = nullptr;
   int* part_label = nullptr;
   int* part_shift = nullptr;
+  // assign, in place of the pruned search: as there, pairs of series without a
+  // finite norm and such centroids have no distance (label 0, INFINITY, the
+  // first lag), and an all-zero centroid is at distance 1 of both series of
+  // any other pair
+  bool search = false;
   const int* skip = nullptr;     // assign: nothing is done when *skip (may be NULL)
 };
 
