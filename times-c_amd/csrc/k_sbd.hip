@@ -233,8 +233,8 @@ __device__ __forceinline__ float div_by(float z, float d, float r) {
   return __builtin_fmaf(__builtin_fmaf(-q, d, z), r, q);
 }
 
-template <int F, int MODE>
-__global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWavesDense) void k_sbd(
+template <int F, int MODE, bool kFew>
+__global__ __launch_bounds__(FftGeom<F>::kBlock, kFew ? 2 : FftGeom<F>::kMinWavesDense) void k_sbd(
     const float* __restrict__ x, long n, int m, int k, int kc,
     const float2* __restrict__ cspec, const float* __restrict__ cnorm,
     const float2* __restrict__ twg, int rev, int* __restrict__ label,
@@ -299,8 +299,8 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWavesDense) voi
       // all of the spectrum in flight at once: without the barrier the compiler
       // may load and multiply one value after the other, a latency each (NCC at
       // F = 512 and 1024: n=700 m=301 k=12 38.3 us, 34.8 with it).  With 128
-      // registers (F >= 2048) the values would spill
-      if constexpr (F <= 1024 && MODE != kModeOwn) __builtin_amdgcn_sched_barrier(0);
+      // registers the values would spill
+      if constexpr ((F <= 1024 || kFew) && MODE != kModeOwn) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int s = 0; s < P; ++s) z[s] = cmulc(zx[s], z[s]);
       fft<F, L, true>(z, buf, tw, twg, lane);
@@ -973,9 +973,10 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
   }
 }
 
-template <int F, bool kPre>
-__global__ __launch_bounds__(PruneGeom<F>::kBlock, kPre ? FftGeom<F>::kMinWaves
-                                                             : FftGeom<F>::kMinWavesPrune)
+template <int F, bool kPre, bool kFew>
+__global__ __launch_bounds__(PruneGeom<F>::kBlock, kFew    ? 2
+                                                   : kPre ? FftGeom<F>::kMinWaves
+                                                          : FftGeom<F>::kMinWavesPrune)
 void k_assign_prune(
     const float* __restrict__ x, const float2* __restrict__ xs, const float* __restrict__ xn,
     const float* __restrict__ ubg, int ub_ld, long n, long npairs, int m, int k,
@@ -1152,11 +1153,18 @@ static int sbd_chunks_F(long npairs, int k, int cus) {
   using G = FftGeom<F>;
   const long blocks = (npairs + G::kGroups - 1) / G::kGroups;
   const long waves = blocks * (G::kBlock / kWave);
-  long c = 12L * cus / (waves > 0 ? waves : 1);
+  // at F = 8192 two per SIMD: one block of the two-wave form per CU
+  long c = (F > 4096 ? 8L : 12L) * cus / (waves > 0 ? waves : 1);
   if (c > k) c = k;
   if (c < 2) return 1;
   const long kc = (k + c - 1) / c;
   return (int)((k + kc - 1) / kc);
+}
+
+// Whether a launch has at most two waves per SIMD in all.
+template <int F>
+static bool few_waves(long blocks, int cus) {
+  return blocks * (FftGeom<F>::kBlock / kWave) <= 8L * cus;
 }
 
 template <int F, int MODE>
@@ -1171,7 +1179,10 @@ static hipError_t launch_sbd_F(const SbdArgs& a, hipStream_t st) {
   const int chunks = MODE == kModeOwn || a.chunks < 1 ? 1 : a.chunks;
   if (split && (!a.part_dist || !a.part_label || !a.part_shift)) return hipErrorInvalidValue;
   const int kc = (a.k + chunks - 1) / chunks;
-  hipLaunchKernelGGL((k_sbd<F, MODE>), dim3((unsigned)blocks, (unsigned)chunks), dim3(G::kBlock),
+  constexpr bool kFew = FftGeom<F>::kFewDense && MODE != kModeOwn;
+  auto* kernel = kFew && few_waves<F>(blocks * chunks, a.cus) ? k_sbd<F, MODE, kFew>
+                                                              : k_sbd<F, MODE, false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks, (unsigned)chunks), dim3(G::kBlock),
                      sbd_smem<F>(), st, a.x, a.n, a.m, a.k, kc, a.cspec, a.cnorm, a.tw, a.rev,
                      split ? a.part_label : a.label, split ? a.part_dist : a.dist,
                      split ? a.part_shift : a.shift, a.dmat, split ? nullptr : a.changed,
@@ -1208,18 +1219,17 @@ static hipError_t launch_prune_F(const PruneArgs& a, hipStream_t st) {
   long blocks = (a.npairs + G::kGroups - 1) / G::kGroups;
   if (blocks < 1) blocks = 1;
   if (blocks > cap) blocks = cap;
+  const bool pre = a.xs && a.ub;
   constexpr bool kTG = F >= 1024;  // as in the body
-  const size_t smem = prune_smem<F, kTG>(a.k);
-  if (a.xs && a.ub)
-    hipLaunchKernelGGL((k_assign_prune<F, true>), dim3((unsigned)blocks), dim3(G::kBlock),
-                       prune_smem<F>(a.k), st, a.x, a.xs, a.xn, a.ub, a.ub_ld, a.n, a.npairs, a.m,
-                       a.k, a.cspec, a.cmag, a.cnorm, a.tw, a.rev, a.order, a.label, a.dist,
-                       a.shift, a.changed, a.evals, a.skip);
-  else
-    hipLaunchKernelGGL((k_assign_prune<F, false>), dim3((unsigned)blocks), dim3(G::kBlock), smem,
-                       st, a.x, nullptr, nullptr, nullptr, 0, a.n, a.npairs, a.m, a.k, a.cspec,
-                       a.cmag, a.cnorm, a.tw, a.rev, a.order, a.label, a.dist, a.shift, a.changed,
-                       a.evals, a.skip);
+  constexpr bool kFew = FftGeom<F>::kFewPrune;
+  auto* kernel = pre                                   ? k_assign_prune<F, true, false>
+                 : kFew && few_waves<F>(blocks, a.cus) ? k_assign_prune<F, false, kFew>
+                                                       : k_assign_prune<F, false, false>;
+  const size_t smem = pre ? prune_smem<F>(a.k) : prune_smem<F, kTG>(a.k);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(G::kBlock), smem, st, a.x,
+                     pre ? a.xs : nullptr, pre ? a.xn : nullptr, pre ? a.ub : nullptr,
+                     pre ? a.ub_ld : 0, a.n, a.npairs, a.m, a.k, a.cspec, a.cmag, a.cnorm, a.tw,
+                     a.rev, a.order, a.label, a.dist, a.shift, a.changed, a.evals, a.skip);
   return hipGetLastError();
 }
 
@@ -1370,13 +1380,19 @@ hipError_t configure_sbd_kernels() {
   hipError_t e = hipSuccess;
 #define X(FF)                                                                                 \
   if (e == hipSuccess)                                                                        \
-    e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeAssign>,                              \
+    e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeAssign, false>,                       \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
   if (e == hipSuccess)                                                                        \
-    e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeNcc>,                                 \
+    e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeNcc, false>,                          \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
   if (e == hipSuccess)                                                                        \
-    e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeOwn>,                                 \
+    e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeOwn, false>,                          \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
+  if (e == hipSuccess)                                                                        \
+    e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeAssign, FftGeom<FF>::kFewDense>,      \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
+  if (e == hipSuccess)                                                                        \
+    e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeNcc, FftGeom<FF>::kFewDense>,         \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
   if (e == hipSuccess)                                                                        \
     e = hipFuncSetAttribute((const void*)k_align<FF>,                                         \
@@ -1385,11 +1401,15 @@ hipError_t configure_sbd_kernels() {
     e = hipFuncSetAttribute((const void*)k_spectra<FF>,                                       \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
   if (e == hipSuccess)                                                                        \
-    e = hipFuncSetAttribute((const void*)k_assign_prune<FF, false>,                           \
+    e = hipFuncSetAttribute((const void*)k_assign_prune<FF, false, false>,                    \
                             hipFuncAttributeMaxDynamicSharedMemorySize,                       \
                             (int)prune_smem<FF>(prune_max_k_F<FF>()));                        \
   if (e == hipSuccess)                                                                        \
-    e = hipFuncSetAttribute((const void*)k_assign_prune<FF, true>,                            \
+    e = hipFuncSetAttribute((const void*)k_assign_prune<FF, true, false>,                     \
+                            hipFuncAttributeMaxDynamicSharedMemorySize,                       \
+                            (int)prune_smem<FF>(prune_max_k_F<FF>()));                        \
+  if (e == hipSuccess)                                                                        \
+    e = hipFuncSetAttribute((const void*)k_assign_prune<FF, false, FftGeom<FF>::kFewPrune>,   \
                             hipFuncAttributeMaxDynamicSharedMemorySize,                       \
                             (int)prune_smem<FF>(prune_max_k_F<FF>()));                        \
   if (e == hipSuccess)                                                                        \

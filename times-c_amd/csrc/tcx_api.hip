@@ -304,6 +304,7 @@ int assign_core_tw(tcx_ctx* c, const float2* tw, const float* d_x, long n, int m
     p.ub = ub;
     p.ub_ld = ub_ld;
     p.skip = skip;
+    p.cus = c->cus;
     TCX_HIP(tcx::launch_assign_prune(F, p, c->stream));
     return TCX_OK;
   }
@@ -312,6 +313,7 @@ int assign_core_tw(tcx_ctx* c, const float2* tw, const float* d_x, long n, int m
   a.rev = rev; a.label = label; a.dist = dist; a.shift = shift; a.dmat = dmat;
   a.changed = changed;
   a.chunks = chunks;
+  a.cus = c->cus;
   a.search = !dmat && k <= tcx::prune_max_k(F);
   a.skip = skip;
   if (part) {
@@ -1166,6 +1168,7 @@ int tcx_ncc(tcx_ctx* c, const float* d_x, const float* d_y, float* d_out, int x_
   a.x = d_x; a.n = x_rows; a.m = cols; a.k = y_rows; a.cspec = spec; a.cnorm = norm;
   a.tw = tw; a.ncc_out = d_out;
   a.chunks = tcx::sbd_chunks(F, x_rows, y_rows, c->cus);
+  a.cus = c->cus;
   TCX_HIP(tcx::launch_sbd(F, tcx::kModeNcc, a, c->stream));
   TCX_HIP(hipStreamSynchronize(c->stream));
   return TCX_OK;

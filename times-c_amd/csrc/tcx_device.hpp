@@ -545,6 +545,11 @@ struct FftGeom {
   // (100000 series m=512 k=16, ten assignments: 4.5, 5.6 ms).
   static constexpr int kMinWavesPrune = F >= 512 ? 4 : 3;
   static constexpr int kMinWavesDense = F >= 2048 ? 4 : 3;
+  // With at most two waves per SIMD in the whole launch (few_waves) more of them
+  // have no use, and the spilled values only cost: those kernels have a second
+  // form with two.  Four and two waves: NCC n=400 m=2049 k=9 98 and 83 us, all
+  // distances n=512 m=3000 k=20 185 and 150, pruned n=1000 m=1500 k=2 44.8 and 37.7.
+  static constexpr bool kFewDense = F >= 2048, kFewPrune = F >= 4096;
 };
 
 // Lag key of circular correlation position tau (0 <= tau < F): the index in

@@ -36,6 +36,7 @@ struct SbdArgs {
   // first lag), and an all-zero centroid is at distance 1 of both series of
   // any other pair
   bool search = false;
+  int cus = 0;                   // compute units of the device
   const int* skip = nullptr;     // assign: nothing is done when *skip (may be NULL)
 };
 
@@ -106,6 +107,7 @@ struct PruneArgs {
   int* changed = nullptr;
   unsigned long long* evals = nullptr;  // inverse transforms run, kEvalSlots counters (may be NULL)
   const int* skip = nullptr;     // nothing is done when *skip (may be NULL)
+  int cus = 0;                   // compute units of the device
 };
 hipError_t launch_assign_prune(int F, const PruneArgs& a, hipStream_t st);
 // Half spectra X_r[0 .. F/2] of every row and the row norms (k_series_spec);
