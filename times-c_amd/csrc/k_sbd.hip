@@ -309,7 +309,7 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, kFew ? 2 : FftGeom<F>::kMinWave
       if constexpr (MODE != kModeNcc) {
         float va, vb;
         int ka, kb;
-        lag_max<F, L, P>(z, rev, lane, m, red, va, ka, vb, kb);
+        lag_max<F, L, P>(z, hasb, rev, lane, m, red, va, ka, vb, kb);
         // den == 0: NumPy divides by inf, every lag is 0, argmax is index 0
         float da = 1.f, db = 1.f;
         if (dena != 0.f) da = 1.f - (va / (float)F) / dena; else ka = 0;
@@ -942,7 +942,7 @@ __device__ __forceinline__ void assign_prune_body(const int bid, const int nblk,
         for (int s = 0; s < P; ++s) z[s] = cmulc(zx[s], cjs[s * L + lane]);
         fft<F, L, true, kTG>(z, buf, tw, twg, lane);
         float va, vb;
-        lag_max<F, L, P>(z, rev, lane, m, red, va, ka, vb, kb);
+        lag_max<F, L, P>(z, hasb, rev, lane, m, red, va, ka, vb, kb);
         if (dena != 0.f) da = 1.f - (va / (float)F) / dena; else ka = 0;
         if (denb != 0.f) db = 1.f - (vb / (float)F) / denb; else kb = 0;
       }
@@ -1037,7 +1037,7 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, FftGeom<F>::kMinWaves) void k_a
     fft<F, L, true>(z, buf, tw, twg, lane);
     float va, vb;
     int ka, kb;
-    lag_max<F, L, P>(z, rev, lane, m, red, va, ka, vb, kb);
+    lag_max<F, L, P>(z, hasb, rev, lane, m, red, va, ka, vb, kb);
     // index 0, the argmax of an all-zero or all-NaN row, where a norm is zero or
     // past the range or the distance is no number (lag_max then has no lag), as
     // the search over centroids leaves it

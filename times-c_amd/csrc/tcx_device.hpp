@@ -699,7 +699,9 @@ __device__ __forceinline__ int wave_first_key(const float2 (&z)[P], bool isx, fl
 // lane keeps its first row in key order that holds g) and a group minimum,
 // where a search would run to the slowest of the groups in a wave or of the
 // waves in a group.  If no lag holds g (rare: every lag below some wrap
-// position), the group takes the masked scan.  Groups wider than a wave
+// position), the group takes the masked scan; a second series that is not
+// there (hasb false) holds rounding noise, whose maximum is often at a wrap
+// position, and is left as it is.  Groups wider than a wave
 // exchange maxima and keys through `red` (32 words; its two halves and the
 // transform's own barriers keep the accesses of consecutive calls apart).
 // Measured with the other form at each width: inside a fit at F = 1024 the
@@ -708,8 +710,8 @@ __device__ __forceinline__ int wave_first_key(const float2 (&z)[P], bool isx, fl
 // k=32), at F = 2048 all distances of n=8000 m=1000 k=20 take 282 us against
 // 290 with the search and 364 with the scan.
 template <int F, int L, int P>
-__device__ __forceinline__ void lag_max(const float2 (&z)[P], int rev, int lane, int m, float* red,
-                                        float& va, int& ka, float& vb, int& kb) {
+__device__ __forceinline__ void lag_max(const float2 (&z)[P], bool hasb, int rev, int lane, int m,
+                                        float* red, float& va, int& ka, float& vb, int& kb) {
   constexpr int W = L < kWave ? L : kWave, NW = L / W;
   static_assert(2 * NW <= 16, "exchange words");
   int* ir = reinterpret_cast<int*>(red);
@@ -778,7 +780,7 @@ __device__ __forceinline__ void lag_max(const float2 (&z)[P], int rev, int lane,
       }
     }
   }
-  if (__any(ka < 0 || kb < 0)) {  // the same in every wave of a wide group
+  if (__any(ka < 0 || (kb < 0 && hasb))) {  // the same in every wave of a wide group
     int s_lo, s_hi;
     lag_rows(lane, L, mo, F, s_lo, s_hi);
     lag_argmax2<L, P>(z, s_lo, s_hi, rev, lane, mo, F, va, ka, vb, kb);
