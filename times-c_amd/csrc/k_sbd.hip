@@ -1147,9 +1147,15 @@ static hipError_t launch_spectra_F(const float* y, int rows, int m, const float2
 }
 
 // Chunks of centroids (blockIdx.y) that fill the device when the pairs alone
-// do not: as many as keep at most three waves per SIMD busy.
+// do not: as many as keep at most three waves per SIMD busy.  merge: the chunk
+// results take k_split_min, a launch of about 2 us more, which fewer transforms
+// than `least` saved per pair do not pay (all distances whole and in chunks:
+// n=1 m=12 k=2 17.6, 18.9 us, k=4 20.3, 19.2; n=9000 m=24 k=4 21.8, 23.3; n=3000
+// m=50 k=2 20.6, 21.8).  With more than a wave per SIMD in the pairs alone, the
+// chunks' own forward transforms cost what they save unless there are some more
+// centroids (n=9000 m=60 k=4 24.8, 26.1, n=3000 m=400 k=2 29.5, 30.9).
 template <int F>
-static int sbd_chunks_F(long npairs, int k, int cus) {
+static int sbd_chunks_F(long npairs, int k, int cus, bool merge) {
   using G = FftGeom<F>;
   const long blocks = (npairs + G::kGroups - 1) / G::kGroups;
   const long waves = blocks * (G::kBlock / kWave);
@@ -1158,6 +1164,9 @@ static int sbd_chunks_F(long npairs, int k, int cus) {
   if (c > k) c = k;
   if (c < 2) return 1;
   const long kc = (k + c - 1) / c;
+  const int least = F <= 16 || (F <= 64 && npairs > 2048) ? 6 : (F <= 128 ? 3 : 1);
+  if (merge && k - kc < least) return 1;
+  if (waves > 4L * cus && k < (F <= 128 ? 6 : 3)) return 1;
   return (int)((k + kc - 1) / kc);
 }
 
@@ -1363,11 +1372,11 @@ hipError_t launch_sbd(int F, int mode, const SbdArgs& a, hipStream_t st) {
   }
 }
 
-int sbd_chunks(int F, long n, int k, int cus) {
+int sbd_chunks(int F, long n, int k, int cus, bool merge) {
   switch (F) {
 #define X(FF) \
   case FF:    \
-    return sbd_chunks_F<FF>((n + 1) / 2, k, cus);
+    return sbd_chunks_F<FF>((n + 1) / 2, k, cus, merge);
     TCX_FOR_EACH_F(X)
 #undef X
     default:

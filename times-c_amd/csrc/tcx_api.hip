@@ -281,10 +281,12 @@ int assign_core_tw(tcx_ctx* c, const float2* tw, const float* d_x, long n, int m
     // another (n=256 m=256 k=24: 35 us split, 127 pruned; n=4096 m=500 k=24,
     // where two chunks would fit: 154 pruned).  With well separated classes
     // (noise 0.05, most of the search pruned) the smallest gain measured at
-    // the line is 49 against 262 us (n=2048 m=128 k=64).  Not when the budget
+    // the line is 49 against 262 us (n=2048 m=128 k=64); one pair alone, where a
+    // transform takes less than half a microsecond, now and then ends after two
+    // or three (n=1 m=24 k=12 20.8 us pruned, 22.0 split).  Not when the budget
     // has no room for the chunk results.
-    chunks = tcx::sbd_chunks(F, n, k, c->cus);
-    if (!dmat && chunks < kSplitMinChunks) chunks = 1;
+    chunks = tcx::sbd_chunks(F, n, k, c->cus, true);
+    if (!dmat && (chunks < kSplitMinChunks || (n <= 2 && F <= 128 && k < 16))) chunks = 1;
     const size_t bytes = ((size_t)chunks * n * 3 * sizeof(float) + 255) & ~(size_t)255;
     if (chunks > 1 && c->slot_bytes[kSlotSplit] < bytes && c->budget &&
         c->ws_bytes + c->user_bytes + bytes > c->budget)
@@ -1167,7 +1169,7 @@ int tcx_ncc(tcx_ctx* c, const float* d_x, const float* d_y, float* d_out, int x_
   tcx::SbdArgs a;
   a.x = d_x; a.n = x_rows; a.m = cols; a.k = y_rows; a.cspec = spec; a.cnorm = norm;
   a.tw = tw; a.ncc_out = d_out;
-  a.chunks = tcx::sbd_chunks(F, x_rows, y_rows, c->cus);
+  a.chunks = tcx::sbd_chunks(F, x_rows, y_rows, c->cus, false);
   a.cus = c->cus;
   TCX_HIP(tcx::launch_sbd(F, tcx::kModeNcc, a, c->stream));
   TCX_HIP(hipStreamSynchronize(c->stream));

@@ -123,8 +123,9 @@ hipError_t launch_series_spec(int F, const float* x, long n, int m, const float2
 hipError_t launch_bounds(int F, const uint16_t* xm, long n, const uint16_t* cm, int k, float* ub,
                          int ld, hipStream_t st);
 hipError_t launch_sbd(int F, int mode, const SbdArgs& a, hipStream_t st);
-// Chunks the centroids of n series are worth splitting into (1: none).
-int sbd_chunks(int F, long n, int k, int cus);
+// Chunks the centroids of n series are worth splitting into (1: none); merge:
+// assign, whose chunk results are merged.
+int sbd_chunks(int F, long n, int k, int cus, bool merge);
 // Shifts each row in place by the lag of its largest NCC with one centroid
 // (spectrum, norm and all-zero flag given; an all-zero one changes nothing).
 hipError_t launch_align(int F, float* x, long n, int m, const float2* cspec, const float* cnorm,
