@@ -219,11 +219,13 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock) void k_spectra(
 // ASSIGN: per series keep the centroid with the smallest
 //   dist = 1 - (max_lag cc / F) / (|x| |c_j|)       (first argmin)
 // and the lag key of its maximum (first argmax), test_timesC.py:258-260.
+// SEARCH: ASSIGN with the pruned search's results where a norm is no number,
+// zero or past the range.
 // OWN: the same of one given centroid per series (fixed_label): at most two
 // inverse transforms per pair.
 // NCC: write cc / F / (|x| |y|) for all 2m-1 lags (ncc.cuh:467-517 layout
 // out[x][y][lag]).
-// blockIdx.y is a chunk of kc centroids; with several chunks ASSIGN writes
+// blockIdx.y is a chunk of kc centroids; with several chunks ASSIGN and SEARCH write
 // each chunk's result at y * n (k_split_min then takes the first smallest).
 
 // z / d where r = 1 / d: the residual step makes the quotient the division's
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, kFew ? 2 : FftGeom<F>::kMinWave
     const float2* __restrict__ twg, int rev, int* __restrict__ label,
     float* __restrict__ dist, int* __restrict__ shift, float* __restrict__ dmat,
     int* __restrict__ changed, float* __restrict__ ncc_out,
-    const int* __restrict__ fixed_label, int search, const int* __restrict__ skip) {
+    const int* __restrict__ fixed_label, const int* __restrict__ skip) {
   using G = FftGeom<F>;
   constexpr int L = G::L, P = G::P;
   extern __shared__ float2 smem[];
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, kFew ? 2 : FftGeom<F>::kMinWave
     sa = group_sum<L>(sa, red);
     sb = group_sum<L>(sb, red);
     float na = sqrtf(sa), nb = sqrtf(sb);
-    if (MODE == kModeAssign && search && !(sa < INFINITY || (hasb && sb < INFINITY)))
+    if (MODE == kModeSearch && !(sa < INFINITY || (hasb && sb < INFINITY)))
       na = nb = NAN;  // no distance
     fft<F, L, false>(zx, buf, tw, twg, lane);
 
@@ -314,7 +316,7 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, kFew ? 2 : FftGeom<F>::kMinWave
         float da = 1.f, db = 1.f;
         if (dena != 0.f) da = 1.f - (va / (float)F) / dena; else ka = 0;
         if (denb != 0.f) db = 1.f - (vb / (float)F) / denb; else kb = 0;
-        if (MODE == kModeAssign && search) {
+        if constexpr (MODE == kModeSearch) {
           if (cn == 0.f && (na == na || nb == nb)) {
             da = db = 1.f;
             ka = kb = 0;
@@ -1183,7 +1185,7 @@ static hipError_t launch_sbd_F(const SbdArgs& a, hipStream_t st) {
   long blocks = (npairs + G::kGroups - 1) / G::kGroups;
   if (blocks < 1) blocks = 1;
   if (blocks > 8192) blocks = 8192;
-  const bool split = MODE == kModeAssign && a.chunks > 1;
+  const bool split = (MODE == kModeAssign || MODE == kModeSearch) && a.chunks > 1;
   if (split && a.changed) return hipErrorInvalidValue;
   const int chunks = MODE == kModeOwn || a.chunks < 1 ? 1 : a.chunks;
   if (split && (!a.part_dist || !a.part_label || !a.part_shift)) return hipErrorInvalidValue;
@@ -1195,7 +1197,7 @@ static hipError_t launch_sbd_F(const SbdArgs& a, hipStream_t st) {
                      sbd_smem<F>(), st, a.x, a.n, a.m, a.k, kc, a.cspec, a.cnorm, a.tw, a.rev,
                      split ? a.part_label : a.label, split ? a.part_dist : a.dist,
                      split ? a.part_shift : a.shift, a.dmat, split ? nullptr : a.changed,
-                     a.ncc_out, a.fixed_label, (int)a.search, a.skip);
+                     a.ncc_out, a.fixed_label, a.skip);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !split) return e;
   hipLaunchKernelGGL(k_split_min, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, st,
@@ -1360,11 +1362,12 @@ hipError_t launch_assign_prune(int F, const PruneArgs& a, hipStream_t st) {
 
 hipError_t launch_sbd(int F, int mode, const SbdArgs& a, hipStream_t st) {
   switch (F) {
-#define X(FF)                                                          \
-  case FF:                                                             \
-    return mode == kModeAssign ? launch_sbd_F<FF, kModeAssign>(a, st)   \
-           : mode == kModeOwn  ? launch_sbd_F<FF, kModeOwn>(a, st)      \
-                               : launch_sbd_F<FF, kModeNcc>(a, st);
+#define X(FF)                                                           \
+  case FF:                                                              \
+    return mode == kModeAssign   ? launch_sbd_F<FF, kModeAssign>(a, st) \
+           : mode == kModeOwn    ? launch_sbd_F<FF, kModeOwn>(a, st)    \
+           : mode == kModeSearch ? launch_sbd_F<FF, kModeSearch>(a, st) \
+                                 : launch_sbd_F<FF, kModeNcc>(a, st);
     TCX_FOR_EACH_F(X)
 #undef X
     default:
@@ -1398,7 +1401,13 @@ hipError_t configure_sbd_kernels() {
     e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeOwn, false>,                          \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
   if (e == hipSuccess)                                                                        \
+    e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeSearch, false>,                       \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
+  if (e == hipSuccess)                                                                        \
     e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeAssign, FftGeom<FF>::kFewDense>,      \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
+  if (e == hipSuccess)                                                                        \
+    e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeSearch, FftGeom<FF>::kFewDense>,      \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbd_smem<FF>()); \
   if (e == hipSuccess)                                                                        \
     e = hipFuncSetAttribute((const void*)k_sbd<FF, kModeNcc, FftGeom<FF>::kFewDense>,         \

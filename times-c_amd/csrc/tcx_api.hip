@@ -281,12 +281,11 @@ int assign_core_tw(tcx_ctx* c, const float2* tw, const float* d_x, long n, int m
     // another (n=256 m=256 k=24: 35 us split, 127 pruned; n=4096 m=500 k=24,
     // where two chunks would fit: 154 pruned).  With well separated classes
     // (noise 0.05, most of the search pruned) the smallest gain measured at
-    // the line is 49 against 262 us (n=2048 m=128 k=64); one pair alone, where a
-    // transform takes less than half a microsecond, now and then ends after two
-    // or three (n=1 m=24 k=12 20.8 us pruned, 22.0 split).  Not when the budget
-    // has no room for the chunk results.
-    chunks = tcx::sbd_chunks(F, n, k, c->cus, true);
-    if (!dmat && (chunks < kSplitMinChunks || (n <= 2 && F <= 128 && k < 16))) chunks = 1;
+    // the line is 49 against 262 us (n=2048 m=128 k=64); only a single short
+    // series may now and then end sooner (n=1 m=24 k=12 19 to 31 us pruned, 20.5
+    // split).  Not when the budget has no room for the chunk results.
+    chunks = tcx::sbd_chunks(F, n, k, c->cus, dmat != nullptr);
+    if (!dmat && chunks < kSplitMinChunks) chunks = 1;
     const size_t bytes = ((size_t)chunks * n * 3 * sizeof(float) + 255) & ~(size_t)255;
     if (chunks > 1 && c->slot_bytes[kSlotSplit] < bytes && c->budget &&
         c->ws_bytes + c->user_bytes + bytes > c->budget)
@@ -316,14 +315,14 @@ int assign_core_tw(tcx_ctx* c, const float2* tw, const float* d_x, long n, int m
   a.changed = changed;
   a.chunks = chunks;
   a.cus = c->cus;
-  a.search = !dmat && k <= tcx::prune_max_k(F);
   a.skip = skip;
   if (part) {
     a.part_dist = part;
     a.part_label = reinterpret_cast<int*>(part + (size_t)chunks * n);
     a.part_shift = a.part_label + (size_t)chunks * n;
   }
-  TCX_HIP(tcx::launch_sbd(F, tcx::kModeAssign, a, c->stream));
+  const bool search = !dmat && k <= tcx::prune_max_k(F);
+  TCX_HIP(tcx::launch_sbd(F, search ? tcx::kModeSearch : tcx::kModeAssign, a, c->stream));
   return TCX_OK;
 }
 

@@ -8,6 +8,11 @@ namespace tcx {
 constexpr int kModeAssign = 0;
 constexpr int kModeNcc = 1;
 constexpr int kModeOwn = 2;
+// assign in place of the pruned search: as there, pairs of series without a
+// finite norm and such centroids have no distance (label 0, INFINITY, the first
+// lag), and an all-zero centroid is at distance 1 of both series of any other
+// pair
+constexpr int kModeSearch = 3;
 
 struct SbdArgs {
   const float* x = nullptr;      // [n][m] series
@@ -31,11 +36,6 @@ struct SbdArgs {
   float* part_dist = nullptr;
   int* part_label = nullptr;
   int* part_shift = nullptr;
-  // assign, in place of the pruned search: as there, pairs of series without a
-  // finite norm and such centroids have no distance (label 0, INFINITY, the
-  // first lag), and an all-zero centroid is at distance 1 of both series of
-  // any other pair
-  bool search = false;
   int cus = 0;                   // compute units of the device
   const int* skip = nullptr;     // assign: nothing is done when *skip (may be NULL)
 };
@@ -124,7 +124,8 @@ hipError_t launch_bounds(int F, const uint16_t* xm, long n, const uint16_t* cm, 
                          int ld, hipStream_t st);
 hipError_t launch_sbd(int F, int mode, const SbdArgs& a, hipStream_t st);
 // Chunks the centroids of n series are worth splitting into (1: none); merge:
-// assign, whose chunk results are merged.
+// the merge of the chunk results is to be paid for (by all distances, which the
+// unsplit kernel gives as well).
 int sbd_chunks(int F, long n, int k, int cus, bool merge);
 // Shifts each row in place by the lag of its largest NCC with one centroid
 // (spectrum, norm and all-zero flag given; an all-zero one changes nothing).
