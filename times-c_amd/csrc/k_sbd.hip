@@ -362,12 +362,14 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, kFew ? 2 : FftGeom<F>::kMinWave
         if (changed && label[ia] != labA) *changed = 1;
         if (label) label[o + ia] = labA;
         if (dist) dist[o + ia] = bestA;
-        if (shift) shift[o + ia] = keyA + 1 - m;
+        // (1 - m) first: OWN's key of a series without a distance is INT_MAX,
+        // a shift past the row
+        if (shift) shift[o + ia] = keyA + (1 - m);
         if (hasb) {
           if (changed && label[ib] != labB) *changed = 1;
           if (label) label[o + ib] = labB;
           if (dist) dist[o + ib] = bestB;
-          if (shift) shift[o + ib] = keyB + 1 - m;
+          if (shift) shift[o + ib] = keyB + (1 - m);
         }
       }
     }
