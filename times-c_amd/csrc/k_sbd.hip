@@ -229,7 +229,8 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock) void k_spectra(
 // each chunk's result at y * n (k_split_min then takes the first smallest).
 
 // z / d where r = 1 / d: the residual step makes the quotient the division's
-// (Markstein) as long as nothing over- or underflows on the way.
+// (Markstein) as long as nothing overflows and the residual is exact: the
+// exponents of quotient and denominator sum to -103 or more.
 __device__ __forceinline__ float div_by(float z, float d, float r) {
   const float q = z * r;
   return __builtin_fmaf(__builtin_fmaf(-q, d, z), r, q);
@@ -346,9 +347,11 @@ __global__ __launch_bounds__(FftGeom<F>::kBlock, kFew ? 2 : FftGeom<F>::kMinWave
             }
           }
         };
-        // z / F is at most about the denominator, so in this range of it
-        // nothing over- or underflows but quotients below 2^-76
-        if (fminf(dA, dB) > 0x1p-50f && fmaxf(dA, dB) < 0x1p50f) {
+        // In this range of the denominators nothing overflows (z / F is at most
+        // about the denominator), and the residual, a multiple of 2^-46 times the
+        // powers of two in quotient and denominator, is exact but for quotients
+        // below 2^-77, whose last bit may differ from the division's
+        if (fminf(dA, dB) > 0x1p-26f && fmaxf(dA, dB) < 0x1p50f) {
           const float rA = 1.f / dA, rB = 1.f / dB;
           write([&](float v, int b) { return b ? div_by(v, dB, rB) : div_by(v, dA, rA); });
         } else {
