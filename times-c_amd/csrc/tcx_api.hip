@@ -655,6 +655,35 @@ void count_steps(const std::vector<tcx::PowerInfo>& info, RefineResult* res) {
   }
 }
 
+// Bytes by which slot s grows when `bytes` are asked of it.
+size_t slot_growth(const tcx_ctx* c, Slot s, size_t bytes) {
+  bytes = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
+  return bytes > c->slot_bytes[s] ? bytes - c->slot_bytes[s] : 0;
+}
+
+// At most what a refinement still allocates after the panels, but for the plan
+// of S and its partials, and what the grouping of a later one with distances
+// does: no more than fit_workspace_bound counts for it.
+size_t refine_growth(const tcx_ctx* c, long n, int m, int k) {
+  const size_t Kc = (size_t)k, Mm = (size_t)m;
+  const size_t vec = sizeof(double) * Kc * Mm;
+  size_t b = slot_growth(c, kSlotS, sizeof(float) * Kc * Mm * Mm) +
+             slot_growth(c, kSlotWbuf, vec * (tcx::kLanczosMax + 1)) +
+             slot_growth(c, kSlotVout, vec) + slot_growth(c, kSlotSvout, vec) +
+             slot_growth(c, kSlotRbuf, vec) + slot_growth(c, kSlotLzW, vec) +
+             slot_growth(c, kSlotSteps, sizeof(int) * Kc) +
+             slot_growth(c, kSlotConv, sizeof(int) * Kc) +
+             slot_growth(c, kSlotMask, sizeof(int) * Kc) +
+             slot_growth(c, kSlotLzState, sizeof(tcx::LzState) * Kc);
+  if (m > tcx::kLzResMaxD) b += slot_growth(c, kSlotLzXch, tcx::lz_xch_bound(m, k));
+  const size_t keys = Kc * tcx::group_bins(n, k, true);
+  const size_t nblk = ((size_t)n + tcx::kGroupChunk - 1) / tcx::kGroupChunk;
+  return b + slot_growth(c, kSlotBlkCount, sizeof(int) * nblk * keys) +
+         slot_growth(c, kSlotBlkBase, sizeof(int) * nblk * keys) +
+         slot_growth(c, kSlotKeyCounts, sizeof(int) * keys) +
+         slot_growth(c, kSlotKeyOff, sizeof(long) * keys);
+}
+
 // One refinement: group, align + pack, S, power iteration.  Reads the
 // labels, shifts and old-centroid zero flags; writes k*m new centroids.
 // With `pending` nothing is waited for: the caller reads the status
@@ -664,7 +693,7 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
            const int* d_shift, const int* d_czero, float* d_cout, int iter, uint64_t seed,
            int split, double tol, int cal_select, const double2* row_stats, RefineResult* res,
            const float* d_dist = nullptr, float* d_check = nullptr,
-           PendingRefine* pending = nullptr) {
+           PendingRefine* pending = nullptr, size_t later_bytes = 0) {
   hipStream_t st = c->stream;
   if (!row_stats && tcx::align_pack_uses_row_stats(m)) {
     double2* rs;
@@ -720,13 +749,18 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
   const long T = (m + tcx::kSyrkSub - 1) / tcx::kSyrkSub, U = T * (T + 1) / 2;
   long max_groups = std::min<long>(std::max<long>(tcx::syrk_max_groups(m, c->cus), k),
                                    n_pad_max / (16 * tcx::kSyrkMinSteps) + k);
-  // Where a budget might have no room for the largest plan beside the rest
-  // (counted as if nothing of it were there yet), the sizes are read back and
-  // the plan is made on the host, with what it needs.
-  const size_t sub = sizeof(float) * tcx::kSyrkSub * tcx::kSyrkSub;
-  const bool host_plan = c->budget && c->ws_bytes + c->user_bytes + sub * (size_t)(max_groups * U) +
-                                              tcx::fit_workspace_bound(n, m, k, c->cus) >
-                                          c->budget;
+  const size_t max_plan =
+      ((sizeof(tcx::SyrkGroup) * (size_t)std::max(max_groups, 1L) + 255) & ~(size_t)255) +
+      sizeof(tcx::SyrkCluster) * (size_t)k;
+  const size_t max_part = sizeof(float) * tcx::kSyrkSub * tcx::kSyrkSub * (size_t)(max_groups * U);
+  // Where the budget has no room for the largest plan beside what this
+  // refinement and the next ones still allocate, the sizes are read back and
+  // the plan is made on the host, with what it needs (about 40 us a refinement).
+  const bool host_plan =
+      c->budget && c->ws_bytes + c->user_bytes + slot_growth(c, kSlotPlan, max_plan) +
+                           slot_growth(c, kSlotPart, max_part) + refine_growth(c, n, m, k) +
+                           later_bytes >
+                       c->budget;
   long nparts = max_groups * U;
   if (host_plan) {
     void* pin;
@@ -747,7 +781,7 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
   const size_t groups_bytes =
       (sizeof(tcx::SyrkGroup) * (size_t)std::max(max_groups, 1L) + 255) & ~(size_t)255;
   const size_t plan_bytes =
-      groups_bytes + sizeof(tcx::SyrkCluster) * (host_plan ? c->sclusters.size() : (size_t)k);
+      host_plan ? groups_bytes + sizeof(tcx::SyrkCluster) * c->sclusters.size() : max_plan;
   unsigned char* d_plan;
   TCX_TRY(ws(c, kSlotPlan, plan_bytes, &d_plan));
   auto* d_groups = reinterpret_cast<tcx::SyrkGroup*>(d_plan);
@@ -756,14 +790,21 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
   TCX_TRY(ws(c, kSlotPart, (size_t)std::max(nparts, 1L) * tcx::kSyrkSub * tcx::kSyrkSub, &part));
   TCX_TRY(ws(c, kSlotS, (size_t)k * m * m, &S));
   if (host_plan) {
+    // staged in the pinned area: its readback above is consumed, and it is sized
+    // for the status copy that uses it next, on the same stream
+    const size_t at = 256;
+    void* stage;
+    TCX_TRY(pinned_area(c, std::max(at + plan_bytes, rs.bytes()), &stage));
+    unsigned char* h = static_cast<unsigned char*>(stage);
     const tcx::SyrkPlanHead head{(int)c->sgroups.size(), (int)c->sclusters.size()};
-    TCX_HIP(hipMemcpyAsync(d_head, &head, sizeof(head), hipMemcpyHostToDevice, st));
-    TCX_HIP(hipMemcpyAsync(d_groups, c->sgroups.data(),
-                           sizeof(tcx::SyrkGroup) * c->sgroups.size(), hipMemcpyHostToDevice, st));
-    TCX_HIP(hipMemcpyAsync(d_clusters, c->sclusters.data(),
-                           sizeof(tcx::SyrkCluster) * c->sclusters.size(), hipMemcpyHostToDevice,
-                           st));
-    TCX_HIP(hipStreamSynchronize(st));
+    std::memcpy(h, &head, sizeof(head));
+    if (head.ngroups > 0) {
+      std::memcpy(h + at, c->sgroups.data(), sizeof(tcx::SyrkGroup) * c->sgroups.size());
+      std::memcpy(h + at + groups_bytes, c->sclusters.data(),
+                  sizeof(tcx::SyrkCluster) * c->sclusters.size());
+      TCX_HIP(hipMemcpyAsync(d_plan, h + at, plan_bytes, hipMemcpyHostToDevice, st));
+    }
+    TCX_HIP(hipMemcpyAsync(d_head, h, sizeof(head), hipMemcpyHostToDevice, st));
   } else {
     TCX_HIP(tcx::launch_syrk_plan(offsets, counts, m, k, c->cus, d_head, d_groups, d_clusters, st));
   }
@@ -1005,9 +1046,8 @@ size_t fit_workspace_bound(long n, int m, int k, int cus) {
   b += r(sizeof(SyrkGroup) * groups + 256 + sizeof(SyrkCluster) * Kc);
   b += r(4 * nparts * kSyrkSub * kSyrkSub) + r(4 * Kc * Mm * Mm);
   // power stage: basis, v, S v, r, w, counters, states, exchange words, mask
-  const size_t xch = Kc * (2 * (2 * (size_t)kLzCoopMaxG * (kLanczosMax + 2) + Mm) + kLzCoopMaxG);
   b += r(8 * Kc * (kLanczosMax + 1) * Mm) + 4 * r(8 * Kc * Mm) + 2 * r(4 * Kc) +
-       r(sizeof(LzState) * Kc) + r(8 * xch + 4 * (Kc + 1)) + r(4 * Kc);
+       r(sizeof(LzState) * Kc) + r(lz_xch_bound(m, k)) + r(4 * Kc);
   // status and sizes; twiddles
   b += r(RefineStatus{k}.bytes()) + 8 * F;
   return b;
@@ -1410,6 +1450,10 @@ int fit_refine(tcx_ctx* c, FitState& f) {
   if (f.o.s_precision == TCX_S_AUTO && f.s_bf16_from < 0 && f.it >= 1 && f.s_checks < 3 &&
       f.o.cal_select == 0)
     TCX_TRY(ws(c, kSlotCheck, (size_t)f.k * f.m, &check));
+  size_t later = 0;  // what the check of a later iteration allocates
+  if (f.o.s_precision == TCX_S_AUTO && f.s_bf16_from < 0 && f.s_checks < 3 && f.o.cal_select == 0)
+    later = slot_growth(c, kSlotCheck, sizeof(float) * (size_t)f.k * f.m) +
+            slot_growth(c, kSlotCheckInfo, sizeof(tcx::PowerInfo) * (size_t)f.k);
   TCX_HIP(hipEventRecord(c->ev[0], st));
   RefineResult rr;
   // With the random-label start the assignment follows at once and its wait
@@ -1418,7 +1462,7 @@ int fit_refine(tcx_ctx* c, FitState& f) {
   const bool defer = f.o.init_mode == 0 && !f.o.stop_on_collapse && !check && f.o.cal_select == 0;
   TCX_TRY(refine(c, f.d_x, f.n, f.m, f.k, f.label, f.shift, f.zero, cnew, f.it, f.o.seed,
                  f.split, f.tol, f.o.cal_select, f.row_stats, &rr,
-                 f.have_dist ? f.dist : nullptr, check, defer ? &f.pending : nullptr));
+                 f.have_dist ? f.dist : nullptr, check, defer ? &f.pending : nullptr, later));
   if (check) {
     ++f.s_checks;
     f.s_check_err = rr.check_err;

@@ -291,6 +291,11 @@ struct LzCoopPlan {
   int form = 0;              // k_lz_multi's register split
   int per = 0;               // clusters of one of its launches
 };
+// Bytes of the exchange and failure words of k clusters, at most.
+inline size_t lz_xch_bound(int m, int k) {
+  const size_t words = 2 * (2 * (size_t)kLzCoopMaxG * (kLanczosMax + 2) + (size_t)m) + kLzCoopMaxG;
+  return 8 * (size_t)k * words + 4 * ((size_t)k + 1);
+}
 // False when m, k or the device do not allow every member to be resident.
 bool plan_lz_coop(int m, int k, int cus, LzCoopPlan* p);
 // xch: k * p.xch_len words and fails: k words, zero when first used; gen:
