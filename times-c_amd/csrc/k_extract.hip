@@ -2880,7 +2880,7 @@ bool align_pack_uses_row_stats(int m) { return m > kPackLdsMaxM; }
 
 hipError_t launch_align_pack(const float* x, int m, const int* perm, long n_pad,
                              const long* offsets, const int* minrow, int k, const int* shift,
-                             const int* czero, const double2* stats, uint16_t* yhi,
+                             const int* czero, const double2* stats, int cus, uint16_t* yhi,
                              uint16_t* ylo, float* a0, hipStream_t st) {
   if (n_pad <= 0) return hipSuccess;
   if (m <= kPackLdsMaxM) {
@@ -2888,7 +2888,7 @@ hipError_t launch_align_pack(const float* x, int m, const int* perm, long n_pad,
     // is packed alike in any block); fit n=512 m=128 k=4, one launch: 19.8 us with
     // 64 rows per block, 8.3 with 16
     int R = align_pack_form(m);
-    while (R > 16 && n_pad / R < 512 && !tuned_pack_rows(m)) R /= 2;
+    while (R > 16 && n_pad / R < 2L * cus && !tuned_pack_rows(m)) R /= 2;
     const size_t lds = sizeof(float) * (size_t)R * (m + 4);
     const dim3 grid((unsigned)(n_pad / R));
     if (R == 64)
@@ -4424,7 +4424,8 @@ hipError_t launch_lz_res(const float* S, int m, int k, const int* counts, uint64
 // shorter.  One refinement, launches and the other form: m=512 k=48 0.33, 0.70
 // ms; m=738 k=22 0.65, 4.2; m=700 k=64 1.16, 1.25; m=300 k=200 0.54, 0.48; m=600
 // k=300 4.0, 1.5; against two launches per step m=1000 k=10 0.44, 0.72, k=200
-// 4.4, 5.9.
+// 4.4, 5.9; two launches and one of k_lz_coop: m=520 k=16 0.40, 0.35, m=600 k=16
+// 0.42, 0.39, m=700 k=16 0.44, 0.45.
 bool plan_lz_multi(int m, int k, int cus, LzCoopPlan* p) {
   if (m <= kLzResMaxD || m > kLzMultiMaxM || k <= 0) return false;
   for (int form = m <= 512 ? 0 : 2; form < 3; ++form) {
@@ -4438,6 +4439,10 @@ bool plan_lz_multi(int m, int k, int cus, LzCoopPlan* p) {
     if (launches > 1 && m <= kFusedLanczosMaxM &&
         (long)launches * (m <= 512 ? 115 : 170) > rounds * m * m / (m % 4 ? 137 : 476))
       return false;
+    // where one launch of the form with S in its blocks' LDS or the L2 holds every
+    // cluster, several of this one are faster only for the longer rows
+    LzCoopPlan one;
+    if (launches > 1 && m <= 640 && plan_lz_coop(m, k, cus, &one)) return false;
     const long nb = ((long)per * G + 7) / 8 * 8;
     const void* fn = form == 0   ? (const void*)k_lz_multi<8, 8, double>
                      : form == 1 ? (const void*)k_lz_multi<8, 16, float>

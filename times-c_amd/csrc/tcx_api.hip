@@ -489,18 +489,7 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
     return TCX_OK;
   }
   tcx::LzCoopPlan cp;
-  bool multi = mode == 0 && !mask && tcx::plan_lz_multi(m, k, c->cus, &cp);
-  if (multi && cp.per < k && m <= 640) {
-    // where one launch of the form with S in its blocks' LDS or the L2 holds
-    // every cluster, several of this one are faster only for the longer rows
-    // (two launches and one: a refinement m=520 k=16 0.40 and 0.35 ms, m=600
-    // k=16 0.42, 0.39, m=700 k=16 0.44, 0.45, m=1000 k=10 0.44, 0.72)
-    tcx::LzCoopPlan one;
-    if (tcx::plan_lz_coop(m, k, c->cus, &one)) {
-      cp = one;
-      multi = false;
-    }
-  }
+  const bool multi = mode == 0 && !mask && tcx::plan_lz_multi(m, k, c->cus, &cp);
   bool coop = multi || (mode == 0 && !mask && tcx::plan_lz_coop(m, k, c->cus, &cp));
   const int per = multi ? cp.per : k;  // clusters of one launch
   const size_t words = (size_t)per * cp.xch_len + ((size_t)per + 1) / 2;
@@ -742,7 +731,7 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
   if (split) TCX_TRY(ws(c, kSlotYlo, panel, &ylo));
   TCX_TRY(ws(c, kSlotA0, (size_t)k * m, &a0));
   TCX_HIP(tcx::launch_align_pack(d_x, m, perm, n_pad_max, offsets, minrow, k, d_shift, d_czero,
-                                 row_stats, yhi, ylo, a0, st));
+                                 row_stats, c->cus, yhi, ylo, a0, st));
   // the plan: header, groups, clusters.  A chunk is at least kSyrkMinSteps
   // steps but for one per cluster, and the groups fit one round of the device
   // or are one per cluster.

@@ -213,7 +213,7 @@ hipError_t launch_row_stats(const float* x, long rows, int m, double2* stats, hi
 bool align_pack_uses_row_stats(int m);
 hipError_t launch_align_pack(const float* x, int m, const int* perm, long n_pad,
                              const long* offsets, const int* minrow, int k, const int* shift,
-                             const int* czero, const double2* stats, uint16_t* yhi,
+                             const int* czero, const double2* stats, int cus, uint16_t* yhi,
                              uint16_t* ylo, float* a0, hipStream_t st);
 // Single fit: blocks of k_syrk for ngroups groups (each group's waves on
 // one XCD), the launch over the groups, and the reduction of the clusters'
