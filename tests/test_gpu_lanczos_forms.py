@@ -66,3 +66,20 @@ def test_forced_give_up_takes_the_power_iteration(ctx, monkeypatch, m, k):
         assert max(errs) <= CENT_RTOL, (what, max(errs))
         olab, _, _, odm = O.assign(Z, r["centroids"].astype(np.float64), dmat=True)
         assert_labels_match(r["labels"], olab, odm, what=what)
+
+
+def test_old_exchange_words_are_no_failure():
+    """A launch of another shape leaves a tag (generation 1, a step) where the
+    second cluster's failure word lies now; the generation reaches that value
+    after 1024 launches and more, which must not make the cluster give up."""
+    with T.Context(0) as c:
+        steps = []
+        # two exchange words per value and buffer; then two clusters of
+        # 4 x 260 + 9 words each before the failure words
+        for m, k, times in ((1000, 1, 1), (260, 2, 1400)):
+            X, _ = T.generate(m + k, 20 * k, m, k, 0.3)
+            d = c.to_device(O.zscore(X.astype(np.float64)).astype(np.float32))
+            for _ in range(times):
+                r = c.fit(d, k, max_iter=1, seed=5)
+                steps.append(r["stats"]["power_steps_max"])
+        assert set(steps[1:]) == {steps[1]}

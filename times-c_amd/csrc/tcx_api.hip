@@ -132,6 +132,8 @@ struct tcx_ctx {
   void* lz_xch = nullptr;        // exchange buffer (and its size) the generation below refers to
   size_t lz_xch_bytes = 0;
   uint32_t lz_gen = 0;           // generation of the last multi-block Lanczos launch
+  const void* lz_fails = nullptr;  // its failure words, the first of which
+  int lz_nfails = 0;               // so many are only ever zero or a generation
   // the last S plan (host copies; the upload is staged in `pinned`)
   std::vector<tcx::SyrkGroup> sgroups;
   std::vector<tcx::SyrkCluster> sclusters;
@@ -497,9 +499,12 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
       c->ws_bytes + c->user_bytes + sizeof(uint64_t) * words + 256 > c->budget)
     coop = false;  // no room for the exchange
   if (coop) {
-    // exchange words and per-cluster failure words; their contents only
-    // ever match the current launch generation, so they are zeroed only
-    // when (re)allocated or when the generation wraps
+    // exchange words and per-cluster failure words; an exchange word's tag only
+    // ever matches the current launch generation, so they are zeroed only when
+    // (re)allocated or when the generation wraps.  A failure word is compared
+    // with the generation itself, which an old tag of another launch's exchange
+    // in its place equals some thousand launches later: they are zeroed when
+    // they move.
     uint64_t* xch;
     TCX_TRY(ws(c, kSlotLzXch, words, &xch));
     uint32_t* fails = reinterpret_cast<uint32_t*>(xch + (size_t)per * cp.xch_len);
@@ -526,7 +531,11 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
           c->lz_xch = xch;
           c->lz_xch_bytes = c->slot_bytes[kSlotLzXch];
           c->lz_gen = 0;
+        } else if (fails != c->lz_fails || per > c->lz_nfails) {
+          TCX_HIP(tcx::launch_fill_int(reinterpret_cast<int*>(fails), per, 0, st));
         }
+        c->lz_fails = fails;
+        c->lz_nfails = per;
         const uint32_t gen = ++c->lz_gen;
         if (multi)
           TCX_HIP(tcx::launch_lz_multi(cp, S, m, j0, std::min(per, k - j0), counts, seed, iter,
