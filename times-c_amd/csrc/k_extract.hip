@@ -3329,9 +3329,9 @@ __global__ __launch_bounds__(kPowerThreads) void k_gram_map(const GramVecJob* __
 // length kLzResSq is squared on the FP64 matrix cores (tridiag_power_mfma).
 // A step is bound by the latency of its exchanges and of its FP64 sums (at
 // order 256 also by the 128 widenings and multiply-adds per lane), not by
-// the matrix.  Measured, k = 4, m = 128, n = 512: 175 us per refinement when
-// the block read S from L2 every step behind a dozen barriers, 62 us now; a
-// launch of 16 steps takes 39 us at order 64, 50 us at 128, 76 us at 256.
+// the matrix.  Measured, launch in a fit n = 512 m = 128 k = 4: 175 us when the
+// block read S from L2 every step behind a dozen barriers, 59 us now; a launch
+// of 16 steps takes 39 us at order 64, 50 us at 128, 76 us at 256.
 // In a batch of 64 uneven jobs the clusters of order <= 256 took 1.9 ms per
 // iteration with a wave (order <= 128) or four waves reading the matrix from
 // L2, 0.3 ms now.

@@ -276,7 +276,9 @@ __host__ __device__ constexpr bool lz_power_check(int len) {
 
 // Lanczos with G blocks per cluster in one launch (members exchange through
 // device-scope memory and wait for each other, so all k*G blocks must be
-// resident at once).  Used from m = kLzCoopMinM on, when the plan fits.
+// resident at once).  Used for m > kLzMultiMaxM when the plan fits, and for
+// 512 < m <= 640 where it holds every cluster and plan_lz_multi needs several
+// launches.
 constexpr int kLzCoopMinM = 256;
 constexpr int kLzCoopMaxR = 64;   // rows of S per member
 constexpr int kLzCoopMaxG = 64;   // members per cluster
@@ -364,8 +366,9 @@ struct ZnormJob {
   long rows;
   int m, ddof;
 };
-// Rows of every job z-normalized (jobs with m % 4 == 0 and 16-byte aligned
-// rows in groups by vector count nv: 0 = the scalar form, else 2, 4, 8, 16).
+// Rows of every job z-normalized, jobs in groups by znorm_form: 0 the three
+// passes (m > 4096), else the 16-byte vectors per lane (1: 16 lanes per row),
+// negative with a tail for rows that are no whole aligned vectors.
 hipError_t launch_znorm_group(const GroupTable& g, int form, hipStream_t st);
 int znorm_form(const float* x, int m);  // form of launch_znorm for these rows
 long znorm_blocks(int form, long rows);
