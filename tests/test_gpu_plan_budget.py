@@ -44,3 +44,28 @@ def test_host_plan_only_without_room(ctx, n, m, k):
     for got in (dev, host):
         for f in ("labels", "centroids", "labels_per_iter"):
             assert np.array_equal(ref[f], got[f]), f
+
+
+def test_exchange_words_leave_room_for_later_refinements():
+    """From the second iteration on the grouping takes more keys (distance
+    bins, about 40 KB here).  A budget with room for that runs the fit, also
+    where it has room for the exchange words of the many-block Lanczos (226 KB
+    a launch), but not for both: the next form runs then."""
+    n, m, k = 300, 700, 30
+    X, _ = T.generate(3, n, m, 8, 0.4)
+
+    def accepted(budget, iters):
+        with T.Context(0, budget) as c:
+            d = c.to_device(X)
+            try:
+                c.fit(d, k, max_iter=iters, seed=1)
+            except T.TimescError:
+                return False
+            return c.workspace_bytes() + X.nbytes <= budget
+
+    lo, hi = 0, 1 << 28
+    while hi - lo > 256:  # the least budget of one iteration
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if accepted(mid, 1) else (mid, hi)
+    for more in range(64 << 10, 400 << 10, 12 << 10):
+        assert accepted(hi + more, 3), more

@@ -461,12 +461,14 @@ std::map<int, hipEvent_t> g_coop_last;
 // every step); else per step one grid-wide matvec launch and one per-cluster
 // update launch, and every 8 steps from 16 on the host reads the clusters' done
 // flags and stops once all are done.
+// reserve: bytes of the budget that the exchange words of the second form leave
+// to what is allocated later; without room the next form runs.
 // Returns on device the vectors v, S v, the row sums r = S 1, the Lanczos
 // step counts and the per-cluster acceptance flags.
 int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, uint64_t seed,
                   int iter, int steps, int mode, const int* mask, const double** vout,
                   const double** svout, const double** rout, const int** steps_out,
-                  const int** conv_out) {
+                  const int** conv_out, size_t reserve = 0) {
   hipStream_t st = c->stream;
   double *Q, *v, *sv, *r, *w;
   int *st_out, *cv_out;
@@ -496,7 +498,7 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
   const int per = multi ? cp.per : k;  // clusters of one launch
   const size_t words = (size_t)per * cp.xch_len + ((size_t)per + 1) / 2;
   if (multi && c->slot_bytes[kSlotLzXch] < sizeof(uint64_t) * words && c->budget &&
-      c->ws_bytes + c->user_bytes + sizeof(uint64_t) * words + 256 > c->budget)
+      c->ws_bytes + c->user_bytes + sizeof(uint64_t) * words + 256 + reserve > c->budget)
     coop = false;  // no room for the exchange
   if (coop) {
     // exchange words and per-cluster failure words; an exchange word's tag only
@@ -659,10 +661,21 @@ size_t slot_growth(const tcx_ctx* c, Slot s, size_t bytes) {
   return bytes > c->slot_bytes[s] ? bytes - c->slot_bytes[s] : 0;
 }
 
+// What later refinements of n series may allocate besides: the mask of clusters
+// rerun and the grouping with distances.
+size_t later_growth(const tcx_ctx* c, long n, int k) {
+  const size_t keys = (size_t)k * tcx::group_bins(n, k, true);
+  const size_t nblk = ((size_t)n + tcx::kGroupChunk - 1) / tcx::kGroupChunk;
+  return slot_growth(c, kSlotMask, sizeof(int) * (size_t)k) +
+         slot_growth(c, kSlotBlkCount, sizeof(int) * nblk * keys) +
+         slot_growth(c, kSlotBlkBase, sizeof(int) * nblk * keys) +
+         slot_growth(c, kSlotKeyCounts, sizeof(int) * keys) +
+         slot_growth(c, kSlotKeyOff, sizeof(long) * keys);
+}
+
 // At most what a refinement still allocates after the panels, but for the plan
-// of S and its partials, and what the grouping of a later one with distances
-// does: no more than fit_workspace_bound counts for it.
-size_t refine_growth(const tcx_ctx* c, long n, int m, int k) {
+// of S and its partials: no more than fit_workspace_bound counts for it.
+size_t power_growth(const tcx_ctx* c, int m, int k) {
   const size_t Kc = (size_t)k, Mm = (size_t)m;
   const size_t vec = sizeof(double) * Kc * Mm;
   size_t b = slot_growth(c, kSlotS, sizeof(float) * Kc * Mm * Mm) +
@@ -671,15 +684,9 @@ size_t refine_growth(const tcx_ctx* c, long n, int m, int k) {
              slot_growth(c, kSlotRbuf, vec) + slot_growth(c, kSlotLzW, vec) +
              slot_growth(c, kSlotSteps, sizeof(int) * Kc) +
              slot_growth(c, kSlotConv, sizeof(int) * Kc) +
-             slot_growth(c, kSlotMask, sizeof(int) * Kc) +
              slot_growth(c, kSlotLzState, sizeof(tcx::LzState) * Kc);
   if (m > tcx::kLzResMaxD) b += slot_growth(c, kSlotLzXch, tcx::lz_xch_bound(m, k));
-  const size_t keys = Kc * tcx::group_bins(n, k, true);
-  const size_t nblk = ((size_t)n + tcx::kGroupChunk - 1) / tcx::kGroupChunk;
-  return b + slot_growth(c, kSlotBlkCount, sizeof(int) * nblk * keys) +
-         slot_growth(c, kSlotBlkBase, sizeof(int) * nblk * keys) +
-         slot_growth(c, kSlotKeyCounts, sizeof(int) * keys) +
-         slot_growth(c, kSlotKeyOff, sizeof(long) * keys);
+  return b;
 }
 
 // One refinement: group, align + pack, S, power iteration.  Reads the
@@ -756,8 +763,8 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
   // the plan is made on the host, with what it needs (about 40 us a refinement).
   const bool host_plan =
       c->budget && c->ws_bytes + c->user_bytes + slot_growth(c, kSlotPlan, max_plan) +
-                           slot_growth(c, kSlotPart, max_part) + refine_growth(c, n, m, k) +
-                           later_bytes >
+                           slot_growth(c, kSlotPart, max_part) + power_growth(c, m, k) +
+                           later_growth(c, n, k) + later_bytes >
                        c->budget;
   long nparts = max_groups * U;
   if (host_plan) {
@@ -818,8 +825,11 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
   // test_timesC.py:184-192); 0: the power iterate, with the clusters that fail the
   // power result's tests rerun through the eigenvector path.
   const int mode = cal_select == 1 ? 1 : 0;
+  // what a later refinement may allocate, a larger plan included
+  const size_t reserve = later_growth(c, n, k) + later_bytes + slot_growth(c, kSlotPlan, max_plan) +
+                         slot_growth(c, kSlotPart, max_part);
   TCX_TRY(power_lanczos(c, S, m, k, counts, seed, iter, max_steps, mode, nullptr, &vin, &svin,
-                        &rsum, &steps_in, &conv_in));
+                        &rsum, &steps_in, &conv_in, reserve));
   TCX_HIP(tcx::launch_power(S, m, k, counts, a0, seed, iter, max_steps, tol, vin, svin, rsum,
                             steps_in, conv_in, mode, nullptr, 1, d_cout, info,
                             mode == 0 ? reinterpret_cast<int*>(status + RefineStatus::kRedo)
@@ -847,7 +857,7 @@ int refine(tcx_ctx* c, const float* d_x, long n, int m, int k, const int* d_labe
     TCX_HIP(tcx::launch_syrk(d_groups, d_head, (int)max_groups, yhi, ylo, m, 0, part, st));
     TCX_HIP(tcx::launch_syrk_reduce(d_clusters, d_head, k, part, m, S, st));
     TCX_TRY(power_lanczos(c, S, m, k, counts, seed, iter, max_steps, 0, nullptr, &vin, &svin,
-                          &rsum, &steps_in, &conv_in));
+                          &rsum, &steps_in, &conv_in, reserve));
     tcx::PowerInfo* cinfo;
     TCX_TRY(ws(c, kSlotCheckInfo, (size_t)k, &cinfo));
     TCX_HIP(tcx::launch_power(S, m, k, counts, a0, seed, iter, max_steps, tol, vin, svin, rsum,
