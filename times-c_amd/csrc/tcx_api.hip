@@ -477,10 +477,8 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
   TCX_TRY(ws(c, kSlotVout, (size_t)k * m, &v));
   TCX_TRY(ws(c, kSlotSvout, (size_t)k * m, &sv));
   TCX_TRY(ws(c, kSlotRbuf, (size_t)k * m, &r));
-  TCX_TRY(ws(c, kSlotLzW, (size_t)k * m, &w));
   TCX_TRY(ws(c, kSlotSteps, (size_t)k, &st_out));
   TCX_TRY(ws(c, kSlotConv, (size_t)k, &cv_out));
-  TCX_TRY(ws(c, kSlotLzState, (size_t)k, &state));
   if (mode == 0 && !mask && m <= tcx::kLzResMaxD) {
     // S_j fits the registers of one block: every step in one launch, S v too
     TCX_HIP(tcx::launch_lz_res(S, m, k, counts, seed, iter, steps, tcx::kLzPowerTol, Q, v, sv, r,
@@ -570,6 +568,8 @@ int power_lanczos(tcx_ctx* c, const float* S, int m, int k, const int* counts, u
     *conv_out = cv_out;
     return TCX_OK;
   }
+  TCX_TRY(ws(c, kSlotLzW, (size_t)k * m, &w));
+  TCX_TRY(ws(c, kSlotLzState, (size_t)k, &state));
   TCX_HIP(tcx::launch_cluster_matvec(S, m, k, nullptr, 0, r, nullptr, st));  // r = S 1
   TCX_HIP(tcx::launch_lz_setup(m, k, counts, mask, seed, iter, r, Q, state, st));
   const int jmax = m < tcx::kLanczosMax ? m : tcx::kLanczosMax;
